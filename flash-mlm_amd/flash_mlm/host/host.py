@@ -185,9 +185,11 @@ def _memo_run(m: _Memo, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, entry
     out = torch.empty(m.out_shape, dtype=q.dtype, device=q.device)
     p = _lib.AttnParams.from_buffer_copy(m.params)
     p.o = out.data_ptr()
-    keep = [q, out, k, v, m.extra]
+    # the first six as _prepare keeps them: the backward reads them (q, out, k, v, context)
+    kc, vc = (entry.k_cache, entry.v_cache) if entry is not None and p.k_ctx else (None, None)
+    keep = [q, out, k, v, kc, vc, m.extra]
     if entry is not None:
-        keep.append((entry.k_cache, entry.v_cache, entry.cu_seqlens_kv, entry.block_table))
+        keep.append((entry.cu_seqlens_kv, entry.block_table))
     if m.repack is not None:
         packed = m.repack(k, v)
         if packed is None:

@@ -537,3 +537,26 @@ def test_backward_non_positive_scale(scale, causal, device):
             assert float(got.abs().max()) == 0.0, name
             continue
         _close(got, ref, name)
+
+
+@pytest.mark.parametrize("with_context", [False, True])
+def test_backward_dense_repeated_call(with_context, device):
+    """The second dense call on the same tensors (a memoised launch) has the first one's
+    gradients, those of the cached context among them."""
+    gen = torch.Generator().manual_seed(31)
+    B, H, N, D, C = 2, 3, 37, 64, 50
+    leaves = [_leaf((B, H, N, D), torch.float16, device, gen) for _ in range(3)]
+    cache, layer = None, None
+    if with_context:
+        leaves += [_leaf((H * C, D), torch.float16, device, gen) for _ in range(2)]
+        cache, layer = InferenceCache(), 0
+        cache.prefill_kv_cache(0, k_cache=leaves[3], v_cache=leaves[4], context_batch_size=1, is_mla=False,
+                               num_heads=H, head_dim=D)
+    dout = torch.randn((B, H, N, D), generator=gen).to(torch.float16).to(device)
+
+    def grads():
+        out = flash_attn_mlm(*leaves[:3], 0.125, inference_cache=cache, layer_id=layer)
+        return torch.autograd.grad(out, leaves, dout)
+
+    for first, again in zip(grads(), grads()):
+        assert torch.equal(first, again)
