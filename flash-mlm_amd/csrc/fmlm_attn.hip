@@ -68,7 +68,10 @@ constexpr int kSortMax = 2048;      // sequences ordered longest-first up to thi
 constexpr int kSplitBK = 64;        // key tile of the split-capable kernel
 constexpr int kMaxSplits = 16;
 constexpr int kMinSplitTiles = 8;   // key tiles per part at least
+constexpr int kMinDenseTiles = 4;   // the same for a dense call's parts
 constexpr float kSplitRounds = 1.5f;
+constexpr int kMinHpackTiles = 4;      // head-packed: key tiles per part at least
+constexpr float kHpackPartCost = 4.f;  // and a part's start, end and merge, in key tiles
 // schedule header fields (int32 index)
 constexpr int kHdrUnits = 0;      // units in all queues
 constexpr int kHdrGroups = 1;     // split groups
@@ -86,7 +89,7 @@ __global__ __launch_bounds__(kSchedThreads) void schedule_kernel(const fmlm_attn
                                                                  int32_t* __restrict__ header,
                                                                  int4* __restrict__ groups,
                                                                  int groups_off, int records_off,
-                                                                 int rec_bytes, int hpack) {
+                                                                 int rec_bytes, int hpack) {  // records_off 0: elsewhere
   __shared__ int s_tiles[kSortMax];
   __shared__ int s_kt[kSortMax];            // key tiles per query tile
   __shared__ long long s_pre[kSortMax + 1];  // head-packed: work before each rank
@@ -133,7 +136,29 @@ __global__ __launch_bounds__(kSchedThreads) void schedule_kernel(const fmlm_attn
     // split only when the units are too few to fill the slots for kSplitRounds rounds;
     // parts of about total / (kSplitRounds * slots) key tiles, at least kMinSplitTiles,
     // the part size doubling until the records fit
-    if (tid == 0 && rec_cap > 0 && s_sum[0] < kSplitRounds * slots) {
+    if (hpack) {
+      // Head-packed tiles fill a CU each (128 KiB of LDS), so parts run in whole rounds of
+      // `slots`: lane S - 1 prices S parts for the longest sequence (the others' parts as
+      // long) as rounds x (key tiles of a part + what a part costs besides), and the
+      // cheapest is taken.
+      if (tid < 64 && rec_cap > 0 && s_sum[0] < kSplitRounds * slots) {
+        float kmax = 0.f;
+        for (int b = 0; b < B; ++b) kmax = fmaxf(kmax, s_tiles[b] > 0 ? s_work[b] : 0.f);
+        const float chunk = fmaxf((float)kMinHpackTiles, ceilf(kmax / (tid + 1)));
+        float parts = 0.f, recs = 0.f;
+        for (int b = 0; b < B; ++b) {
+          const float S = fminf(kMaxSplits, fmaxf(1.f, ceilf(s_work[b] / chunk)));
+          parts += s_tiles[b] * S;
+          if (S > 1.f) recs += s_tiles[b] * S;
+        }
+        float cost = ceilf(parts / slots) * (chunk + kHpackPartCost);
+        if (recs > (float)rec_cap || tid >= kMaxSplits) cost = INFINITY;
+        float best = cost;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) best = fminf(best, __shfl_xor(best, off));
+        if (cost == best && chunk < kmax) atomicMax(&s_chunk, (int)chunk);
+      }
+    } else if (tid == 0 && rec_cap > 0 && s_sum[0] < kSplitRounds * slots) {
       int chunk = max(kMinSplitTiles, (int)ceilf(s_sum[1] / (kSplitRounds * slots)));
       for (int it = 0; it < 24; ++it, chunk *= 2) {
         float recs = 0.f;
@@ -304,6 +329,25 @@ struct WorkItem {
   KvSeg seg[2];          // context, main
 };
 
+// Split-KV arguments of an attention launch: where the parts' records are (NULL: at the
+// schedule's kHdrRecordsOff), their size, and the parts per query tile of a dense call.
+struct SplitArgs {
+  char* records;
+  int32_t rec_bytes;
+  int32_t dense_parts;  // 1: not split
+};
+
+// record i, or NULL when the launch has no room for records
+FMLM_DEV char* split_record(const int32_t* hdr, const SplitArgs& spa, int i) {
+  char* base = spa.records;
+  if (!base) {
+    const int off = ldc(hdr, kHdrRecordsOff);
+    if (off <= 0) return nullptr;
+    base = (char*)hdr + off;
+  }
+  return base + (int64_t)i * spa.rec_bytes;
+}
+
 FMLM_DEV int64_t seg_row(const KvSeg& s, int i, bool is_v, const int32_t* cu, int B) {
   const int64_t base = is_v ? s.vbase : s.kbase;
   const int64_t sn = is_v ? s.vsn : s.ksn;
@@ -326,10 +370,11 @@ FMLM_DEV int4 ldc4(const int4* a, int i) {
 }
 
 // Unit u of a call: packed calls read queue entry u, dense calls map slot u (XCD u % 8,
-// position u / 8; group g = (b, h) has its ceil(N/BQ) tiles at consecutive positions of
-// XCD g % 8).  Returns false for a unit with nothing to do (an idle dense slot, or an entry
+// position u / 8; group g = (b, h) has its ceil(N/BQ) tiles, each with its spa.dense_parts
+// key ranges, at consecutive positions of XCD g % 8).  Returns false for a unit with nothing to do (an idle dense slot, or an entry
 // of a schedule built for other shapes).
-FMLM_DEV bool resolve_work(const fmlm_attn_params& p, const int4* units, int u, int BQ, WorkItem& w, bool hpack = false) {
+FMLM_DEV bool resolve_work(const fmlm_attn_params& p, const int4* units, int u, int BQ, WorkItem& w,
+                           const SplitArgs& spa, bool hpack = false) {
   int b, h, tile;
   w.split_s = 0;
   w.split_n = 1;
@@ -345,15 +390,23 @@ FMLM_DEV bool resolve_work(const fmlm_attn_params& p, const int4* units, int u, 
     if (un.w >= 0) {
       w.split_group = un.w & 0xfffff;
       w.split_s = (un.w >> 20) & 31;
-      w.split_n = ((un.w >> 25) & 15) + 1;
+      w.split_n = ((un.w >> 25) & 31) + 1;
       w.rec0 = un.z;
     }
   } else {
     const int nt = (p.N + BQ - 1) / BQ;
-    const int x = u % kXcds, pos = u / kXcds;
+    const int x = u % kXcds;
+    int pos = u / kXcds;
+    const int S = spa.dense_parts;
+    if (S > 1) {
+      w.split_s = pos % S;
+      w.split_n = S;
+      pos /= S;
+    }
     const int g = (pos / nt) * kXcds + x;
     tile = pos % nt;
     if (g >= p.B * p.H) return false;
+    w.rec0 = (g * nt + tile) * S;
     b = g / p.H;
     h = g - b * p.H;
   }
@@ -514,7 +567,8 @@ constexpr float kRescaleSlack = 8.0f;
 template <typename T, int D, int QB, int NW, int BK>
 __global__ __launch_bounds__(NW * 64, NW >= 8 ? 1 : 2) void attn_mfma_kernel(const fmlm_attn_params p,
                                                                const int4* __restrict__ units,
-                                                               const int32_t* __restrict__ hdr) {
+                                                               const int32_t* __restrict__ hdr,
+                                                               const SplitArgs spa) {
   typedef MfmaCfg<T, D, QB, NW, BK> C;
   typedef typename Mfma<T>::v8 v8;
   extern __shared__ __align__(16) char smem_raw[];
@@ -522,7 +576,7 @@ __global__ __launch_bounds__(NW * 64, NW >= 8 ? 1 : 2) void attn_mfma_kernel(con
 
   const int u = p.cu_seqlens_q ? workgroup_unit(hdr) : (int)blockIdx.x;
   WorkItem w;
-  if (u < 0 || !resolve_work(p, units, u, C::BQ, w)) return;
+  if (u < 0 || !resolve_work(p, units, u, C::BQ, w, spa)) return;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -855,7 +909,7 @@ struct Mfma3Cfg {
 
 template <typename T, int D, int QB, int NW, int BK, bool PAGED, int PPB>
 __global__ __launch_bounds__(NW * 64, NW >= 8 ? 1 : 2) void attn_mfma3_kernel(
-    const fmlm_attn_params p, const int4* __restrict__ units, const int32_t* __restrict__ hdr) {
+    const fmlm_attn_params p, const int4* __restrict__ units, const int32_t* __restrict__ hdr, const SplitArgs spa) {
   typedef Mfma3Cfg<T, D, QB, NW, BK, PPB> C;
   typedef typename Mfma<T>::v8 v8;
   extern __shared__ __align__(16) char smem_raw[];
@@ -864,7 +918,7 @@ __global__ __launch_bounds__(NW * 64, NW >= 8 ? 1 : 2) void attn_mfma3_kernel(
 
   const int u = p.cu_seqlens_q ? workgroup_unit(hdr) : (int)blockIdx.x;
   WorkItem w;
-  if (u < 0 || !resolve_work(p, units, u, C::BQ, w)) return;
+  if (u < 0 || !resolve_work(p, units, u, C::BQ, w, spa)) return;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -1465,10 +1519,9 @@ __global__ __launch_bounds__(NW * 64, NW >= 8 ? 1 : 2) void attn_mfma3_kernel(
   // ---- split part: this part's record (O / l, then m and l per row, all fp32) for
   // merge_kernel
   if (w.split_n > 1) {
-    char* const records = (char*)hdr + ldc(hdr, kHdrRecordsOff);
-    const int64_t rec_bytes = ldc(hdr, kHdrRecBytes);
     const int64_t ml_off = (int64_t)C::BQ * D * 4;  // m [BQ] then l [BQ]
-    char* const mine = records + (int64_t)(w.rec0 + w.split_s) * rec_bytes;
+    char* const mine = split_record(hdr, spa, w.rec0 + w.split_s);
+    if (!mine) return;
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
       const int row = (wave * QB + qb) * 16 + l16;
@@ -1534,9 +1587,9 @@ struct MlaRowsCfg {
   static constexpr int LDS_BYTES = 2 * TILEB;
 };
 
-template <typename T, bool PAGED, bool LSE>
+template <typename T, bool PAGED, bool LSE, bool SPLIT>
 __global__ __launch_bounds__(MlaRowsCfg::NT, 1) void attn_mla_rows_kernel(
-    const fmlm_attn_params p, const int4* __restrict__ units, const int32_t* __restrict__ hdr) {
+    const fmlm_attn_params p, const int4* __restrict__ units, const int32_t* __restrict__ hdr, const SplitArgs spa) {
   typedef MlaRowsCfg C;
   typedef typename Mfma<T>::v8 v8;
   constexpr int D = C::D, BK = C::BK;
@@ -1547,9 +1600,11 @@ __global__ __launch_bounds__(MlaRowsCfg::NT, 1) void attn_mla_rows_kernel(
   const bool hpack = p.cu_seqlens_q != nullptr;
   // the grid covers the queue slots (8 * cap workgroups), workgroup w taking entry w / 8
   // of queue w % 8: a sequence's tiles stay on the XCDs the schedule put them on
-  const int u = hpack ? queue_first(hdr, blockIdx.x) : (int)blockIdx.x;
+  // (spread_by_queue).  SPLIT, launches that may split: the units are covered as by the
+  // other kernels
+  const int u = !hpack ? (int)blockIdx.x : SPLIT ? workgroup_unit(hdr) : queue_first(hdr, blockIdx.x);
   WorkItem w;
-  if (u < 0 || !resolve_work(p, units, u, C::BQ, w, hpack)) return;
+  if (u < 0 || !resolve_work(p, units, u, C::BQ, w, SPLIT ? spa : SplitArgs{nullptr, 0, 1}, hpack)) return;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -1606,12 +1661,16 @@ __global__ __launch_bounds__(MlaRowsCfg::NT, 1) void attn_mla_rows_kernel(
     vv = vr * C::ROWB + 32 * (vsw >> 1) + 16 * (x ^ (vsw & 1)) + 8 * (l16 & 1);
   }
   // LDS fragment reads in flight ahead of their MFMA (the paged variant keeps its page
-  // window in registers, which the longer lead would spill)
-  constexpr int LEAD = PAGED ? 2 : 3;
+  // window in registers, the split variant its tile range, which the longer lead would
+  // spill)
+  constexpr int LEAD = PAGED || SPLIT ? 2 : 3;
 
   const int nt0 = (w.seg[0].n + BK - 1) / BK;
   const int nt1 = (w.seg[1].n + BK - 1) / BK;
   const int ntiles = nt0 + nt1;
+  // this part's tiles (split-KV)
+  const int tb = SPLIT ? (int)((int64_t)w.split_s * ntiles / w.split_n) : 0;
+  const int te = SPLIT ? (int)((int64_t)(w.split_s + 1) * ntiles / w.split_n) : ntiles;
   PageWindow pwin;  // paged context: page ids of the tiles around the last one fetched
   page_window_reset(pwin);
 
@@ -1650,16 +1709,18 @@ __global__ __launch_bounds__(MlaRowsCfg::NT, 1) void attn_mla_rows_kernel(
   for (int db = 0; db < C::NDB; ++db) o[db] = f32x4{0.f, 0.f, 0.f, 0.f};
   float m_i = -INFINITY, l_i = 0.f;
 
-  if (ntiles > 0) fetch(0, 0);
+  if (te > tb) fetch(tb, tb & 1);
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
-  for (int t = 0; t < ntiles; ++t) {
+  for (int t = tb; t < te; ++t) {
     const char* tile = smem_raw + (t & 1) * C::TILEB;
     // a wave with query rows loads its share of tile t+1 once its S MFMAs have read tile
     // t's K fragments (the DMA writes into LDS then overlap the P V phase rather than the
     // b128 fragment reads of S; measured 2.6-3.3% faster at config 5 than loading at the
     // top of the tile, and faster than any later point, which leaves the loads less time)
-    if (!wave_active && t + 1 < ntiles) fetch(t + 1, (t + 1) & 1);
+    // (SPLIT: at the top, where the latents of a short call still come from HBM and the
+    // loads need the whole tile's time)
+    if ((SPLIT || !wave_active) && t + 1 < te) fetch(t + 1, (t + 1) & 1);
     if (wave_active) {
       // Four phases of 32 fenced slots: slot f issues the LDS read of fragment f + LEAD
       // and the MFMA of fragment f.  K fragments f < 64 build S^T: half h = f / 32 covers
@@ -1766,7 +1827,7 @@ __global__ __launch_bounds__(MlaRowsCfg::NT, 1) void attn_mla_rows_kernel(
 #pragma unroll
       for (int f = 32; f < 64; ++f) slot(f);
       __builtin_amdgcn_s_setprio(0);
-      if (t + 1 < ntiles) fetch(t + 1, (t + 1) & 1);
+      if (!SPLIT && t + 1 < te) fetch(t + 1, (t + 1) & 1);
       half_check(1);
       __builtin_amdgcn_s_setprio(2);
 #pragma unroll
@@ -1782,6 +1843,24 @@ __global__ __launch_bounds__(MlaRowsCfg::NT, 1) void attn_mla_rows_kernel(
   // ---- epilogue: l over the 4 lanes holding the row's keys, O /= l, store the row
   l_i += __shfl_xor(l_i, 16);
   l_i += __shfl_xor(l_i, 32);
+  if (SPLIT && w.split_n > 1) {  // this part's record (O / l, then m and l per row, fp32) for merge_kernel
+    char* const mine = split_record(hdr, spa, w.rec0 + w.split_s);
+    // the lane's row and group computed anew: kept across the tile loop they would spill
+    int ln = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+    asm volatile("" : "+v"(ln));
+    const int rr = wave * 16 + (ln & 15), rg = ln >> 4;
+    if (!mine || rr >= w.qcount) return;
+    const float inv = l_i > 0.f ? 1.f / l_i : 0.f;
+    float* const dst = (float*)mine + rr * D + rg * 4;
+#pragma unroll
+    for (int db = 0; db < C::NDB; ++db) *(f32x4*)(dst + db * 16) = o[db] * inv;
+    if (rg == 0) {
+      float* const ml = (float*)mine + C::BQ * D;
+      ml[rr] = m_i;
+      ml[C::BQ + rr] = l_i;
+    }
+    return;
+  }
   if (row < w.qcount) {
     const float inv = l_i > 0.f ? 1.f / l_i : 1.f;
     char* dst = (char*)p.o + o_off * 2;
@@ -1839,13 +1918,12 @@ FMLM_DEV float4 load4<float>(const float* p) {
   return *(const float4*)p;
 }
 
-// fp32 (and head dims without an MFMA instantiation): TPR threads per query row, each
-// holding DPT dims of q and o; a row's partial dot products meet through xor shuffles
-// inside its TPR lanes.  K/V tiles of BKS keys are staged as fp32 in LDS and read as
-// float4 (a row's lanes cover one contiguous key row).
+// TPR threads per query row, each holding DPT dims of q and o; a row's partial dot products
+// meet through xor shuffles inside its TPR lanes.  K/V tiles of BKS keys are staged as fp32
+// in LDS and read as float4 (a row's lanes cover one contiguous key row).
 template <typename T, int D>
 __global__ __launch_bounds__(SimtCfg<D>::NT) void attn_simt_kernel(
-    const fmlm_attn_params p, const int4* __restrict__ units, const int32_t* __restrict__ hdr) {
+    const fmlm_attn_params p, const int4* __restrict__ units, const int32_t* __restrict__ hdr, const SplitArgs spa) {
   typedef SimtCfg<D> C;
   extern __shared__ __align__(16) char smem_raw[];
   float* Kf = (float*)smem_raw;
@@ -1853,7 +1931,7 @@ __global__ __launch_bounds__(SimtCfg<D>::NT) void attn_simt_kernel(
 
   const int u = p.cu_seqlens_q ? workgroup_unit(hdr) : (int)blockIdx.x;
   WorkItem w;
-  if (u < 0 || !resolve_work(p, units, u, C::RPW, w)) return;
+  if (u < 0 || !resolve_work(p, units, u, C::RPW, w, spa)) return;
   const int tid = threadIdx.x;
   const int row = tid / C::TPR;
   const int part = tid % C::TPR;
@@ -1947,40 +2025,82 @@ __global__ __launch_bounds__(SimtCfg<D>::NT) void attn_simt_kernel(
 // cut into S parts), O = sum_s 2^(m_s - M) l_s O_s / sum_s 2^(m_s - M) l_s with
 // M = max_s m_s, over the parts' records (O_s = part output / l_s as fp32, m_s in log2
 // units, l_s its row sum), so the merged row is rounded to the output type once, as an
-// unsplit row is.  Grid-stride over groups; 8 columns of a row per thread.
+// unsplit row is.  Packed calls list their groups in the schedule; a split dense call has
+// one group per query tile.  hpack: a tile's rows are (head, position) rows of the
+// sequence (see schedule_kernel).  A workgroup takes a chunk of a group's rows, one pass of
+// its threads at 8 columns each, so that a few large groups still spread over the chip.
 // ---------------------------------------------------------------------------
 constexpr int kMergeRows = 128;  // largest split-capable query tile
+constexpr int kMergeThreads = 256;
+// rows per chunk (at most one per thread / 8)
+__host__ __device__ inline int merge_chunk(int D) { return D <= 64 ? 32 : 2048 / D; }
+
+// chunks of a group's rows: a sequence of at most N rows has no more of them in any tile
+__host__ __device__ inline int merge_chunks(const fmlm_attn_params& p, int BQ, int hpack) {
+  const int rows = !hpack && p.N > 0 && p.N < BQ ? p.N : BQ, chunk = merge_chunk(p.D);
+  return (rows + chunk - 1) / chunk;
+}
+
+// 8 floats rounded to 8 elements of T at dst (16-byte aligned)
+template <typename T>
+FMLM_DEV void store8(char* dst, const f32x4& a0, const f32x4& a1) {
+  if constexpr (sizeof(T) == 4) {
+    *(f32x4*)dst = a0;
+    *(f32x4*)(dst + 16) = a1;
+  } else {
+    typename Mfma<T>::v8 res;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      res[e] = (T)a0[e];
+      res[4 + e] = (T)a1[e];
+    }
+    *(typename Mfma<T>::v8*)dst = res;
+  }
+}
 
 template <typename T>
-__global__ __launch_bounds__(256) void merge_kernel(const fmlm_attn_params p, int BQ,
-                                                    const int32_t* __restrict__ header) {
-  typedef typename Mfma<T>::v8 v8;
-  __shared__ float s_w[kMergeRows][kMaxSplits];  // per row: part weights / their sum
-  const int n_groups = header[kHdrGroups];
-  const int4* groups = (const int4*)((const char*)header + header[kHdrGroupsOff]);
-  const char* records = (const char*)header + header[kHdrRecordsOff];
-  const int64_t rec_bytes = header[kHdrRecBytes];
+__global__ __launch_bounds__(kMergeThreads) void merge_kernel(const fmlm_attn_params p, int BQ,
+                                                    const int32_t* __restrict__ header, const SplitArgs spa,
+                                                    int hpack) {
+  __shared__ float s_w[32][kMaxSplits];  // per row: part weights / their sum
+  __shared__ int64_t s_o[32];            // per row: element offset of its output row
+  const int nt = (p.N + BQ - 1) / BQ;  // dense: tiles per (sequence, head)
+  const int n_groups = header ? ldc(header, kHdrGroups) : p.B * p.H * nt;
+  const int chunks = merge_chunks(p, BQ, hpack);
+  const int64_t rec_bytes = spa.rec_bytes;
   const int D = p.D;
   const int64_t ml_off = (int64_t)BQ * D * 4;
-  for (int gi = blockIdx.x; gi < n_groups; gi += gridDim.x) {
-    const int4 gr = groups[gi];
-    const int b = gr.x, h = gr.y & 0xffff, tile = (int)((uint32_t)gr.y >> 16), S = gr.w;
+  for (int wi = blockIdx.x; wi < n_groups * chunks; wi += gridDim.x) {
+    const int gi = wi / chunks, r0 = (wi % chunks) * merge_chunk(D);
+    int b, h, tile, S, first;
+    if (header) {
+      const int4 gr = ldc4((const int4*)((const char*)header + ldc(header, kHdrGroupsOff)), gi);
+      b = gr.x, h = gr.y & 0xffff, tile = (int)((uint32_t)gr.y >> 16), first = gr.z, S = gr.w;
+    } else {
+      tile = gi % nt, b = gi / nt / p.H, h = gi / nt % p.H, S = spa.dense_parts, first = gi * S;
+    }
     if (b < 0 || b >= p.B || h >= p.H) continue;
     const SeqInfo si = seq_info(p, b);
-    const int qcount = min(BQ, si.len - tile * BQ);
-    const int64_t ob = p.o_layout == FMLM_LAYOUT_PACKED
-                           ? (int64_t)h * p.o_sh + (int64_t)si.q0 * p.o_sn
-                           : (int64_t)b * p.o_sb + (int64_t)h * p.o_sh;
-    const int64_t o_row0 = ob + (int64_t)tile * BQ * p.o_sn;
-    const char* rec0 = records + (int64_t)gr.z * rec_bytes;
+    const int rows = min(min(BQ, (hpack ? p.H : 1) * si.len - tile * BQ) - r0, merge_chunk(D));
+    if (rows <= 0) continue;
+    const char* rec0 = split_record(header, spa, first);
+    if (!rec0) return;
     // weights of row r: 2^(m_s - M) l_s / sum, all parts' (m, l) loaded at once
-    for (int r = threadIdx.x; r < qcount; r += blockDim.x) {
+    if ((int)threadIdx.x < rows) {
+      const int r = threadIdx.x;
+      int hq = h, pos = tile * BQ + r0 + r;
+      if (hpack) {
+        hq = pos / si.len;
+        pos -= hq * si.len;
+      }
+      s_o[r] = p.o_layout == FMLM_LAYOUT_PACKED ? (int64_t)hq * p.o_sh + (int64_t)(si.q0 + pos) * p.o_sn
+                                                : (int64_t)b * p.o_sb + (int64_t)hq * p.o_sh + (int64_t)pos * p.o_sn;
       float m[kMaxSplits], l[kMaxSplits];
 #pragma unroll
       for (int sp = 0; sp < kMaxSplits; ++sp) {
         const float* ml = (const float*)(rec0 + (sp < S ? sp : 0) * rec_bytes + ml_off);
-        m[sp] = sp < S ? ml[r] : -INFINITY;
-        l[sp] = sp < S ? ml[BQ + r] : 0.f;
+        m[sp] = sp < S ? ml[r0 + r] : -INFINITY;
+        l[sp] = sp < S ? ml[BQ + r0 + r] : 0.f;
       }
       float M = -INFINITY;
 #pragma unroll
@@ -1994,12 +2114,12 @@ __global__ __launch_bounds__(256) void merge_kernel(const fmlm_attn_params p, in
       const float inv = L > 0.f ? 1.f / L : 0.f;
 #pragma unroll
       for (int sp = 0; sp < kMaxSplits; ++sp) s_w[r][sp] = l[sp] * inv;
-      if (p.lse) store_lse(p, h, si.q0, tile * BQ + r, M, L);
+      if (p.lse) store_lse(p, hq, si.q0, pos, M, L);
     }
     __syncthreads();
-    for (int idx = threadIdx.x; idx < qcount * (D / 8); idx += blockDim.x) {
+    for (int idx = threadIdx.x; idx < rows * (D / 8); idx += blockDim.x) {
       const int row = idx / (D / 8), c8 = idx - row * (D / 8);
-      const char* src = rec0 + ((int64_t)row * D + c8 * 8) * 4;
+      const char* src = rec0 + ((int64_t)(r0 + row) * D + c8 * 8) * 4;
       f32x4 a0 = f32x4{0.f, 0.f, 0.f, 0.f}, a1 = a0;
 #pragma unroll 4
       for (int sp = 0; sp < S; ++sp) {
@@ -2009,15 +2129,9 @@ __global__ __launch_bounds__(256) void merge_kernel(const fmlm_attn_params p, in
         a0 += ws * x0;
         a1 += ws * x1;
       }
-      v8 res;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        res[e] = (T)a0[e];
-        res[4 + e] = (T)a1[e];
-      }
-      *(v8*)((char*)p.o + (o_row0 + (int64_t)row * p.o_sn + c8 * 8) * 2) = res;
+      store8<T>((char*)p.o + (s_o[row] + c8 * 8) * (int64_t)sizeof(T), a0, a1);
     }
-    __syncthreads();  // s_w is rewritten for the next group
+    __syncthreads();  // s_w is rewritten for the next chunk
   }
 }
 
@@ -2026,9 +2140,10 @@ struct Launch {
   int threads;
   int lds;
   const void* fn;
-  bool split = false;  // kernel can run split-KV units
+  bool split = false;  // kernel can run split-KV units (split_fn when set, for calls that may split)
   bool hpack = false;  // packed tiles span (head, position) rows (MLA: one latent for all heads)
   bool paged = false;  // kernel reads a paged context (key tile = FMLM_PAGE_ROWS rows)
+  const void* split_fn = nullptr;
 };
 
 template <typename T, int D, int QB, int NW, int BK>
@@ -2060,14 +2175,19 @@ static Launch mfma3_launch(bool paged) {
 // the paged instantiation only for paged contexts: the page lookup costs registers the
 // contiguous kernel (at 256 VGPRs) does not have; the LSE one only for calls that store
 // the row statistics
+template <typename T, bool SPLIT>
+static const void* mla_rows_fn(bool paged, bool lse) {
+  return paged ? (lse ? (const void*)&attn_mla_rows_kernel<T, true, true, SPLIT>
+                      : (const void*)&attn_mla_rows_kernel<T, true, false, SPLIT>)
+               : (lse ? (const void*)&attn_mla_rows_kernel<T, false, true, SPLIT>
+                      : (const void*)&attn_mla_rows_kernel<T, false, false, SPLIT>);
+}
 template <typename T>
 static Launch mla_rows_launch(bool paged, bool lse) {
   static_assert(MlaRowsCfg::BK == FMLM_PAGE_ROWS, "a paged context tile is one page");
-  const void* fn = paged ? (lse ? (const void*)&attn_mla_rows_kernel<T, true, true>
-                                : (const void*)&attn_mla_rows_kernel<T, true, false>)
-                         : (lse ? (const void*)&attn_mla_rows_kernel<T, false, true>
-                                : (const void*)&attn_mla_rows_kernel<T, false, false>);
-  return Launch{MlaRowsCfg::BQ, MlaRowsCfg::NT, MlaRowsCfg::LDS_BYTES, fn, false, true, true};
+  Launch L{MlaRowsCfg::BQ, MlaRowsCfg::NT, MlaRowsCfg::LDS_BYTES, mla_rows_fn<T, false>(paged, lse), true, true, true};
+  L.split_fn = mla_rows_fn<T, true>(paged, lse);
+  return L;
 }
 
 // MFMA kernels by head dim.  The pipelined kernel and the 512-wide latent kernel need
@@ -2162,17 +2282,18 @@ static int pick_launch(const fmlm_attn_params& p, Launch& L) {
   return 0;
 }
 
+constexpr int kMaxKernels = 128;  // kernels whose attributes are remembered
 // Allow the kernel's dynamic LDS (> 64 KiB for some tiles), once per kernel.
-static int allow_lds(const Launch& L) {
+static int allow_lds(const void* fn, int lds) {
   static std::mutex mu;
-  static const void* raised[64];
+  static const void* raised[kMaxKernels];
   static int n_raised = 0;
   std::lock_guard<std::mutex> lock(mu);
   for (int i = 0; i < n_raised; ++i)
-    if (raised[i] == L.fn) return 0;
-  hipError_t e = hipFuncSetAttribute(L.fn, hipFuncAttributeMaxDynamicSharedMemorySize, L.lds);
+    if (raised[i] == fn) return 0;
+  hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (e != hipSuccess) return (int)e;
-  if (n_raised < 64) raised[n_raised++] = L.fn;
+  if (n_raised < kMaxKernels) raised[n_raised++] = fn;
   return 0;
 }
 
@@ -2180,19 +2301,19 @@ static int allow_lds(const Launch& L) {
 // a query error.
 static int resident_slots(const Launch& L) {
   static std::mutex mu;
-  static const void* fns[64];
-  static int slots_of[64];
+  static const void* fns[kMaxKernels];
+  static int slots_of[kMaxKernels];
   static int n_fns = 0;
   std::lock_guard<std::mutex> lock(mu);
   for (int i = 0; i < n_fns; ++i)
     if (fns[i] == L.fn) return slots_of[i];
   int dev = 0, cus = 0, per_cu = 0;
-  if (allow_lds(L) != 0 || hipGetDevice(&dev) != hipSuccess ||
+  if (allow_lds(L.fn, L.lds) != 0 || hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
       hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, L.fn, L.threads, L.lds) != hipSuccess)
     return 0;
   const int slots = cus * (per_cu > 0 ? per_cu : 1);
-  if (n_fns < 64) {
+  if (n_fns < kMaxKernels) {
     fns[n_fns] = L.fn;
     slots_of[n_fns++] = slots;
   }
@@ -2205,26 +2326,52 @@ struct SplitCfg {
   int slots = 0;
   int rec_cap = 0;        // 0: no split
   int64_t rec_bytes = 0;  // per record: rows x (D fp32 + m + l)
+  int dense_parts = 1;    // dense call: parts per query tile
 };
 
 static SplitCfg split_cfg(const fmlm_attn_params& p, const Launch& L) {
   SplitCfg sc;
-  if (!L.split || !p.cu_seqlens_q) return sc;
+  if (!L.split || L.bq > kMergeRows) return sc;
   sc.slots = resident_slots(L);
   if (sc.slots == 0) return sc;
+  const int64_t rec_bytes = ((int64_t)L.bq * (p.D * 4 + 8) + 15) / 16 * 16;
+  if (!p.cu_seqlens_q) {
+    // Every query tile has the same keys: S equal parts each, when the tiles fill at most
+    // half of the slots (from there on the parts' records and merge cost what the idle slots
+    // do: 512 tiles on 768 slots were slower split).  Bf16, 16 heads, 24 queries, D = 128,
+    // 6000 context rows: 16 tiles, one workgroup each, took 80 us unsplit; 11 parts each
+    // 19.7, 16 parts 19.0, 32 parts 22.8.
+    const int64_t tiles = (int64_t)p.B * p.H * ((p.N + L.bq - 1) / L.bq);
+    if (p.cu_seqlens_kv || tiles < 1 || 2 * tiles > sc.slots) return SplitCfg{};
+    const int64_t ctx = (p.flags & FMLM_FLAG_PREFILL) ? 0 : p.ctx_len;
+    const int64_t ktiles = (ctx + kSplitBK - 1) / kSplitBK + (p.N + kSplitBK - 1) / kSplitBK;
+    const int64_t S = std::min({(int64_t)kMaxSplits, sc.slots / tiles, ktiles / kMinDenseTiles});
+    if (S < 2) return SplitCfg{};
+    sc.dense_parts = (int)S;
+    sc.rec_cap = (int)(tiles * S);
+    sc.rec_bytes = rec_bytes;
+    return sc;
+  }
   // every sequence's tiles but its last are full, so there are at least
   // H * (total_q - B*bq) / bq units: when that already fills kSplitRounds rounds, the
   // schedule cannot split (and no records or merge launch are needed)
-  const int64_t min_units = (int64_t)p.H * (((int64_t)p.total_q - (int64_t)p.B * L.bq) / L.bq);
-  if (min_units >= (int64_t)(kSplitRounds * sc.slots) || L.bq > kMergeRows) return SplitCfg{};
+  const int64_t min_units = L.hpack ? ((int64_t)p.H * p.total_q - (int64_t)p.B * L.bq) / L.bq
+                                    : (int64_t)p.H * (((int64_t)p.total_q - (int64_t)p.B * L.bq) / L.bq);
+  if (min_units >= (int64_t)(kSplitRounds * sc.slots)) return SplitCfg{};
   sc.rec_cap = 3 * sc.slots;
-  sc.rec_bytes = ((int64_t)L.bq * (p.D * 4 + 8) + 15) / 16 * 16;
+  // The latent kernel: one or two whole rounds (see schedule_kernel), by the most units there
+  // can be.  16 sequences of 1-4 tokens, 64 heads, 1400-7800 latent rows each: 22 tiles took
+  // 261 us unsplit on as many CUs; split 47 us and the merge 10.  Up to 32 parts instead of
+  // 16: 15% slower (a part's fp32 record costs as much traffic as 8 tiles of keys).
+  if (L.hpack)
+    sc.rec_cap = (((int64_t)p.H * p.total_q + L.bq - 1) / L.bq + p.B <= sc.slots ? 1 : 2) * sc.slots;
+  sc.rec_bytes = rec_bytes;
   return sc;
 }
 
-// Units of a dense call: slots of 8 XCDs x ceil(B*H / 8) groups x ceil(N / bq) tiles.
-static int64_t dense_units(const fmlm_attn_params& p, int bq) {
-  return (int64_t)kXcds * (((int64_t)p.B * p.H + kXcds - 1) / kXcds) * ((p.N + bq - 1) / bq);
+// Units of a dense call: slots of 8 XCDs x ceil(B*H / 8) groups x ceil(N / bq) tiles x parts.
+static int64_t dense_units(const fmlm_attn_params& p, int bq, int parts) {
+  return (int64_t)kXcds * (((int64_t)p.B * p.H + kXcds - 1) / kXcds) * ((p.N + bq - 1) / bq) * parts;
 }
 
 // Entries per queue of a packed call: a bound on the launch's units, so that one queue
@@ -2235,18 +2382,25 @@ static int64_t queue_cap(const fmlm_attn_params& p, int bq, const SplitCfg& sc, 
   int64_t units = hpack ? ((int64_t)p.H * p.total_q + bq - 1) / bq + p.B
                         : (int64_t)p.H * (((int64_t)p.total_q + bq - 1) / bq + p.B);
   if (sc.rec_cap > 0) {
-    const int64_t split_units = (int64_t)(kSplitRounds * sc.slots) + 1 + sc.rec_cap;
+    const int64_t split_units = std::min(units, (int64_t)(kSplitRounds * sc.slots) + 1) + sc.rec_cap;
     units = split_units > units ? split_units : units;
   }
   return units;
 }
 
+// Head-packed launches that cannot split run every queue entry on its own XCD (8 * cap
+// workgroups): their queues are balanced by work and not by count, and overflow taken onto
+// other XCDs would break the one-latent-per-XCD placement.  One that may split has queues
+// of about equally long units, and 8 * cap workgroups of 128 KiB LDS, most of them idle,
+// would take longer to dispatch than a short call's work.
+static bool spread_by_queue(const Launch& L, const SplitCfg& sc) { return L.hpack && sc.rec_cap == 0; }
+
 // Grid (one unit per workgroup): a dense call's slots; cap workgroups for a packed call
-// (spares take what overflows a queue's static entries), 8 * cap head-packed.
+// (spares take what overflows a queue's static entries), 8 * cap when spread by queue.
 static int64_t grid_size(const fmlm_attn_params& p, const Launch& L, const SplitCfg& sc) {
-  if (!p.cu_seqlens_q) return dense_units(p, L.bq);
+  if (!p.cu_seqlens_q) return dense_units(p, L.bq, sc.dense_parts);
   const int64_t cap = queue_cap(p, L.bq, sc, L.hpack);
-  return L.hpack ? kXcds * cap : cap;
+  return spread_by_queue(L, sc) ? kXcds * cap : cap;
 }
 
 // Schedule buffer layout (see schedule_kernel): header, 8 queues, groups, records.
@@ -2266,9 +2420,12 @@ static SchedLayout sched_layout(const fmlm_attn_params& p, int bq, const SplitCf
   return l;
 }
 
-static int64_t workspace_for(const fmlm_attn_params& p, const Launch& L) {
-  if (!p.cu_seqlens_q) return 0;
-  return sched_layout(p, L.bq, split_cfg(p, L), L.hpack).bytes;
+// bytes of the split records of a call (0: it never splits)
+static int64_t records_for(const SplitCfg& sc) { return (int64_t)sc.rec_cap * sc.rec_bytes; }
+
+static int64_t workspace_for(const fmlm_attn_params& p, const Launch& L, const SplitCfg& sc) {
+  if (!p.cu_seqlens_q) return records_for(sc);
+  return sched_layout(p, L.bq, sc, L.hpack).bytes;
 }
 
 static int check_params(const fmlm_attn_params& p) {
@@ -2291,26 +2448,30 @@ static int check_params(const fmlm_attn_params& p) {
 }
 
 static int launch_schedule(const fmlm_attn_params& p, const Launch& L, const SplitCfg& sc, char* sched,
-                           hipStream_t s) {
+                           int64_t bytes, hipStream_t s) {
   const SchedLayout l = sched_layout(p, L.bq, sc, L.hpack);
   // the unit's 16-bit tile field: tiles of N rows, or of H*N (H*total_q) rows head-packed;
   // queue entries are addressed with 32-bit indices
   const int64_t rows = L.hpack ? (int64_t)p.H * (p.N > 0 ? p.N : p.total_q) : p.N;
   if (kXcds * l.cap > 0x7fffffff || p.H > 0xffff || (rows + L.bq - 1) / L.bq > 0xffff) return FMLM_E_ARG;
   int32_t* header = (int32_t*)sched;
+  // a buffer without room for the records: each launch brings its own (split_record)
+  const int64_t records_off = bytes >= l.bytes ? l.records_off : 0;
   hipLaunchKernelGGL(schedule_kernel, dim3(1), dim3(kSchedThreads), 0, s, p, L.bq, (int)l.cap,
                      sc.slots, sc.rec_cap, (int4*)(sched + l.units_off), header,
-                     (int4*)(sched + l.groups_off), (int)l.groups_off, (int)l.records_off,
+                     (int4*)(sched + l.groups_off), (int)l.groups_off, (int)records_off,
                      (int)sc.rec_bytes, (int)L.hpack);
   return launch_status();
 }
 
-// The attention launch (plus the split merge) over the schedule at `sched`, which is
-// built first when `build` is set.  sc must be the split sizing the schedule was (or is)
-// built with.
+// The attention launch (plus the split merge) over the schedule at `sched` (packed calls;
+// built first when `build` is set, in `bytes` bytes).  sc must be the split sizing the
+// schedule was (or is) built with; records: where split parts go, NULL for the schedule's
+// own record area.
 static int launch_attention(const fmlm_attn_params& p, const Launch& L, const SplitCfg& sc, char* sched,
-                            bool build, hipStream_t s) {
-  int rc = allow_lds(L);
+                            bool build, int64_t bytes, char* records, hipStream_t s) {
+  const void* const fn = sc.rec_cap > 0 && L.split_fn ? L.split_fn : L.fn;
+  int rc = allow_lds(fn, L.lds);
   if (rc) return rc;
   int4* units = nullptr;
   int32_t* header = nullptr;
@@ -2318,7 +2479,7 @@ static int launch_attention(const fmlm_attn_params& p, const Launch& L, const Sp
     header = (int32_t*)sched;
     units = (int4*)(sched + 256);
     if (build) {
-      rc = launch_schedule(p, L, sc, sched, s);
+      rc = launch_schedule(p, L, sc, sched, bytes, s);
       if (rc) return rc;
     }
   }
@@ -2326,15 +2487,18 @@ static int launch_attention(const fmlm_attn_params& p, const Launch& L, const Sp
   if (gx <= 0) return 0;
   if (gx > 0x7fffffff) return FMLM_E_ARG;
   fmlm_attn_params pc = p;
-  void* args[] = {(void*)&pc, (void*)&units, (void*)&header};
-  hipError_t e = hipLaunchKernel(L.fn, dim3((unsigned)gx), dim3(L.threads), args, (size_t)L.lds, s);
+  SplitArgs spa{records, (int32_t)sc.rec_bytes, sc.dense_parts};
+  void* args[] = {(void*)&pc, (void*)&units, (void*)&header, (void*)&spa};
+  hipError_t e = hipLaunchKernel(fn, dim3((unsigned)gx), dim3(L.threads), args, (size_t)L.lds, s);
   if (e != hipSuccess) return (int)e;
   if (sc.rec_cap > 0) {  // split groups (if the schedule made any) are merged here
-    const dim3 mg((unsigned)(sc.rec_cap < 1024 ? sc.rec_cap : 1024));
+    const int64_t groups = p.cu_seqlens_q ? sc.rec_cap / 2 : sc.rec_cap / sc.dense_parts;
+    const int hp = L.hpack && p.cu_seqlens_q;
+    const dim3 mg((unsigned)std::min<int64_t>(groups * merge_chunks(p, L.bq, hp), 4096));
     if (p.dtype == FMLM_DTYPE_BF16)
-      hipLaunchKernelGGL(merge_kernel<bf16>, mg, dim3(256), 0, s, p, L.bq, (const int32_t*)header);
+      hipLaunchKernelGGL(merge_kernel<bf16>, mg, dim3(kMergeThreads), 0, s, p, L.bq, (const int32_t*)header, spa, hp);
     else
-      hipLaunchKernelGGL(merge_kernel<f16>, mg, dim3(256), 0, s, p, L.bq, (const int32_t*)header);
+      hipLaunchKernelGGL(merge_kernel<f16>, mg, dim3(kMergeThreads), 0, s, p, L.bq, (const int32_t*)header, spa, hp);
   }
   return launch_status();
 }
@@ -2372,18 +2536,22 @@ static int scratch_on_current_device(char** out) {
 
 // The split sizing of the allocation-free path: as split_cfg, with the record count cut
 // so that the schedule and the records fit the scratch array (no split when fewer than
-// one record per workgroup slot would fit).  Returns false when even the unsplit
-// schedule does not fit.
+// one record per workgroup slot would fit; a dense call's parts are all or none).  Returns
+// false when even the unsplit schedule does not fit.
 static bool split_cfg_within(const fmlm_attn_params& p, const Launch& L, int64_t cap, SplitCfg& sc) {
   sc = split_cfg(p, L);
+  if (!p.cu_seqlens_q) {
+    if (records_for(sc) > cap) sc = SplitCfg{};
+    return true;
+  }
   auto fits = [&](int rec_cap) {
     SplitCfg t = sc;
     t.rec_cap = rec_cap;
     return sched_layout(p, L.bq, t, L.hpack).bytes <= cap;
   };
   if (fits(sc.rec_cap)) return true;
-  // the layout grows with the record count: the largest count in [slots, rec_cap) that fits
-  int lo = sc.slots, hi = sc.rec_cap - 1;
+  // the layout grows with the record count: the largest count in [lo, rec_cap) that fits
+  int lo = L.hpack ? 1 : sc.slots, hi = sc.rec_cap - 1;
   if (sc.rec_cap > 0 && lo <= hi && fits(lo)) {
     while (lo < hi) {
       const int mid = lo + (hi - lo + 1) / 2;
@@ -2409,8 +2577,9 @@ extern "C" int fmlm_attn_schedule(const fmlm_attn_params* pp, void* schedule,
   Launch L;
   const int rc = pick_launch(*pp, L);
   if (rc) return rc;
-  if (schedule_bytes < workspace_for(*pp, L)) return FMLM_E_WORKSPACE;
-  return launch_schedule(*pp, L, split_cfg(*pp, L), (char*)schedule, (hipStream_t)stream);
+  const SplitCfg sc = split_cfg(*pp, L);
+  if (schedule_bytes < workspace_for(*pp, L, sc) - records_for(sc)) return FMLM_E_WORKSPACE;
+  return launch_schedule(*pp, L, sc, (char*)schedule, schedule_bytes, (hipStream_t)stream);
 }
 
 extern "C" int fmlm_attn_params_size(void) { return (int)sizeof(fmlm_attn_params); }
@@ -2420,7 +2589,15 @@ extern "C" int64_t fmlm_attn_workspace_bytes(const fmlm_attn_params* p) {
   Launch L;
   const int rc = pick_launch(*p, L);
   if (rc) return rc;
-  return workspace_for(*p, L);
+  return workspace_for(*p, L, split_cfg(*p, L));
+}
+
+extern "C" int64_t fmlm_attn_records_bytes(const fmlm_attn_params* p) {
+  if (!p) return FMLM_E_ARG;
+  Launch L;
+  const int rc = pick_launch(*p, L);
+  if (rc) return rc;
+  return records_for(split_cfg(*p, L));
 }
 
 extern "C" int fmlm_attn_fwd(const fmlm_attn_params* pp, void* stream) {
@@ -2432,10 +2609,20 @@ extern "C" int fmlm_attn_fwd(const fmlm_attn_params* pp, void* stream) {
   rc = pick_launch(p, L);
   if (rc) return rc;
   if (p.B == 0 || p.H == 0) return 0;
-  const int64_t need = workspace_for(p, L);
-  if (need > 0 && !p.schedule && (!p.workspace || p.workspace_bytes < need)) return FMLM_E_WORKSPACE;
-  char* sched = (char*)(p.schedule ? p.schedule : p.workspace);
-  return launch_attention(p, L, split_cfg(p, L), sched, !p.schedule, (hipStream_t)stream);
+  SplitCfg sc = split_cfg(p, L);
+  const int64_t have = p.workspace ? p.workspace_bytes : 0;
+  char* const ws = (char*)p.workspace;
+  if (!p.cu_seqlens_q) {  // dense: the workspace holds split records only; without one, no split
+    if (have < records_for(sc)) sc = SplitCfg{};
+    return launch_attention(p, L, sc, nullptr, false, 0, ws, (hipStream_t)stream);
+  }
+  const int64_t need = workspace_for(p, L, sc);
+  if (p.schedule) {
+    char* const records = records_for(sc) > 0 && have >= records_for(sc) ? ws : nullptr;
+    return launch_attention(p, L, sc, (char*)p.schedule, false, 0, records, (hipStream_t)stream);
+  }
+  if (need > 0 && have < need) return FMLM_E_WORKSPACE;
+  return launch_attention(p, L, sc, ws, true, need, nullptr, (hipStream_t)stream);
 }
 
 extern "C" int fmlm_attn_fwd_noalloc(const fmlm_attn_params* pp, void* stream) {
@@ -2448,12 +2635,13 @@ extern "C" int fmlm_attn_fwd_noalloc(const fmlm_attn_params* pp, void* stream) {
   if (rc) return rc;
   if (p.B == 0 || p.H == 0) return 0;
   SplitCfg sc;
-  char* sched = nullptr;
-  if (p.cu_seqlens_q) {
-    if (!split_cfg_within(p, L, kNoAllocScratchBytes, sc)) return FMLM_E_WORKSPACE;
-    rc = scratch_on_current_device(&sched);
+  if (!split_cfg_within(p, L, kNoAllocScratchBytes, sc)) return FMLM_E_WORKSPACE;
+  char* scratch_mem = nullptr;
+  if (p.cu_seqlens_q || sc.rec_cap > 0) {
+    rc = scratch_on_current_device(&scratch_mem);
     if (rc) return rc;
   }
   // the schedule is always rebuilt: the array holds whatever the previous call left
-  return launch_attention(p, L, sc, sched, true, (hipStream_t)stream);
+  if (!p.cu_seqlens_q) return launch_attention(p, L, sc, nullptr, false, 0, scratch_mem, (hipStream_t)stream);
+  return launch_attention(p, L, sc, scratch_mem, true, kNoAllocScratchBytes, nullptr, (hipStream_t)stream);
 }

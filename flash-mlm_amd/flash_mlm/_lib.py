@@ -164,6 +164,7 @@ SIGNATURES = {
          _c_ptr, _c_ptr],
     ),
     "fmlm_attn_workspace_bytes": (ctypes.c_int64, [ctypes.POINTER(AttnParams)]),
+    "fmlm_attn_records_bytes": (ctypes.c_int64, [ctypes.POINTER(AttnParams)]),
     "fmlm_attn_schedule": (ctypes.c_int, [ctypes.POINTER(AttnParams), _c_ptr, _c_i64, _c_ptr]),
     "fmlm_attn_fwd": (ctypes.c_int, [ctypes.POINTER(AttnParams), _c_ptr]),
     "fmlm_attn_fwd_noalloc": (ctypes.c_int, [ctypes.POINTER(AttnParams), _c_ptr]),

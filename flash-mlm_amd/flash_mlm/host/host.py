@@ -100,7 +100,7 @@ _ROW_STATS = threading.local()
 class AttnLaunch:
     """A prepared fmlm_attn_fwd call: the parameter block plus the tensors it points to."""
 
-    __slots__ = ("lib", "params", "stream", "device", "keep", "unpack_kv", "lse")
+    __slots__ = ("lib", "params", "stream", "device", "keep", "unpack_kv", "lse", "records", "records_buf")
 
     def __init__(self, lib, params, stream, device, keep):
         self.lib, self.params, self.stream, self.device, self.keep = lib, params, stream, device, keep
@@ -108,6 +108,11 @@ class AttnLaunch:
         # K/V (causal_query_seq_attn): the backward unpacks their gradient
         self.unpack_kv = None
         self.lse = None  # the row statistics of the last run, when it stored them
+        # bytes of split partial results each run brings in a buffer of its own, so that runs
+        # of one schedule on several streams or threads never share them (0: none, or the
+        # parameter block's workspace holds them)
+        self.records = 0
+        self.records_buf = None  # kept only by a run on a stream other than the current one
 
     def __call__(self) -> None:
         p = self.params
@@ -118,6 +123,11 @@ class AttnLaunch:
         if getattr(_ROW_STATS, "on", False) and p.H > 0 and p.total_q > 0:
             self.lse = torch.empty(p.H * p.total_q, dtype=torch.float32, device=self.device)
             p.lse = self.lse.data_ptr()
+        if self.records:
+            buf = torch.empty(self.records, dtype=torch.uint8, device=self.device)
+            p.workspace, p.workspace_bytes = buf.data_ptr(), self.records
+            if _lib.stream_of(self.device) != self.stream:
+                self.records_buf = buf
         with _device_scope(self.device):
             rc = self.lib.fmlm_attn_fwd(p, self.stream)
         _lib.check(rc, "fmlm_attn_fwd")
@@ -151,12 +161,13 @@ def _tkey(t: torch.Tensor):
 
 
 class _Memo:
-    __slots__ = ("params", "entry_ref", "extra", "out_shape", "repack", "unpack_kv")
+    __slots__ = ("params", "entry_ref", "extra", "out_shape", "repack", "unpack_kv", "records")
 
     def __init__(self, plan: AttnLaunch, entry, extra, out_shape, repack=None):
         self.params = _lib.AttnParams.from_buffer_copy(plan.params)
         self.entry_ref = None if entry is None else weakref.ref(entry)
         self.extra, self.out_shape, self.repack, self.unpack_kv = extra, out_shape, repack, plan.unpack_kv
+        self.records = plan.records
 
 
 def _entry_of(inference_cache: InferenceCache | None, layer_id):
@@ -198,7 +209,7 @@ def _memo_run(m: _Memo, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, entry
         p.k, p.v = k_pk.data_ptr(), v_pk.data_ptr()
         keep.append(packed)
     plan = AttnLaunch(_lib.load(), p, _lib.stream_of(q.device), q.device, tuple(keep))
-    plan.unpack_kv = m.unpack_kv
+    plan.unpack_kv, plan.records = m.unpack_kv, m.records
     plan()
     return out, plan
 
@@ -426,27 +437,34 @@ def _prepare(
     ws_bytes = int(lib.fmlm_attn_workspace_bytes(p))
     _lib.check(ws_bytes if ws_bytes < 0 else 0, "fmlm_attn_workspace_bytes")
     stream = _lib.stream_of(q.device)
-    with _device_scope(q.device):
-        if ws_bytes > 0 and schedule_cache is not None:
-            # what the unit list depends on: the kernel (dtype, head dim, flags, K/V
-            # layout, paged context or not), whose tile size and occupancy fix the slots,
-            # the split records and the grid, and the shape (B, H, N, total_q); context
-            # lengths only steer where key ranges are split
-            key = (p.dtype, D, B, H, N, total_q, p.flags, p.kv_layout, block_table is not None, p.tile_config)
-            sched = schedule_cache.get(key)
-            if sched is None:
-                sched = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
-                _lib.check(lib.fmlm_attn_schedule(p, sched.data_ptr(), ws_bytes, stream), "fmlm_attn_schedule")
-                schedule_cache[key] = sched
-            p.schedule = sched.data_ptr()
-            ws = None
-        else:
-            sched = None
-            ws = _workspace(inference_cache, ws_bytes, q.device)
-            p.workspace = None if ws is None else ws.data_ptr()
-            p.workspace_bytes = ws_bytes
+    sched = ws = None
+    records = 0
+    if cu_seqlens_q is None:
+        records = ws_bytes  # a dense call needs a workspace for split partial results only
+    elif ws_bytes > 0 and schedule_cache is not None:
+        records = int(lib.fmlm_attn_records_bytes(p))
+        # what the unit list depends on: the kernel (dtype, head dim, flags, K/V
+        # layout, paged context or not), whose tile size and occupancy fix the slots,
+        # the split records and the grid, and the shape (B, H, N, total_q); context
+        # lengths only steer where key ranges are split
+        key = (p.dtype, D, B, H, N, total_q, p.flags, p.kv_layout, block_table is not None, p.tile_config)
+        sched = schedule_cache.get(key)
+        if sched is None:
+            nbytes = ws_bytes - records
+            sched = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
+            with _device_scope(q.device):
+                rc = lib.fmlm_attn_schedule(p, sched.data_ptr(), nbytes, stream)
+            _lib.check(rc, "fmlm_attn_schedule")
+            schedule_cache[key] = sched
+        p.schedule = sched.data_ptr()
+    elif ws_bytes > 0:
+        ws = _workspace(inference_cache, ws_bytes, q.device)
+        p.workspace = ws.data_ptr()
+        p.workspace_bytes = ws_bytes
     keep = (q, out, k, v, k_ctx, v_ctx, cu_seqlens_q, cu_seqlens_kv, ctx_index, block_table, ws, sched)
-    return AttnLaunch(lib, p, stream, q.device, keep)
+    plan = AttnLaunch(lib, p, stream, q.device, keep)
+    plan.records = records
+    return plan
 
 
 def _check_cache_dtype(k_cache: torch.Tensor, q: torch.Tensor) -> None:

@@ -215,9 +215,11 @@ typedef struct fmlm_attn_params {
                               cu_seqlens_q contents, B, H, total_q, dtype, D, flags and
                               kv_layout: then fmlm_attn_fwd launches the attention
                               kernel (plus the split merge) only.  Context lengths may
-                              differ; they only steer where key ranges are split.  The
-                              buffer also holds split partial results: launches that may
-                              overlap need separate schedule buffers                  */
+                              differ; they only steer where key ranges are split.  Split
+                              partial results go to `workspace` when it holds at least
+                              fmlm_attn_records_bytes (launches that overlap then only
+                              need workspaces of their own), else to the schedule buffer
+                              (launches that may overlap need separate ones)          */
   const int32_t* ctx_index;  /* [B] context batch of each sequence, or NULL (see above):
                                 index-mapped context batching.  No counterpart in the
                                 reference, whose roadmap lists it ("variable context
@@ -257,13 +259,19 @@ typedef struct fmlm_attn_params {
 } fmlm_attn_params;
 
 /* Bytes of device workspace (and of a schedule buffer) fmlm_attn_fwd needs for these
- * parameters (>= 0), or < 0 on unsupported dtype / head dim. */
+ * parameters (>= 0), or < 0 on unsupported dtype / head dim.  A dense call
+ * (cu_seqlens_q == NULL) also runs without: its key ranges are then not split. */
 FMLM_API int64_t fmlm_attn_workspace_bytes(const fmlm_attn_params* p);
 
+/* The part of fmlm_attn_workspace_bytes that holds split partial results (0 when the call
+ * never splits), or < 0 as above.  A schedule buffer without that part serves calls that
+ * bring a workspace of this many bytes. */
+FMLM_API int64_t fmlm_attn_records_bytes(const fmlm_attn_params* p);
+
 /* Build the work schedule (one entry per query tile of the kernel's own tile size over
- * the real rows of every sequence) into `schedule` (fmlm_attn_workspace_bytes bytes) so
- * later fmlm_attn_fwd calls with p->schedule = schedule skip rebuilding it.  No
- * counterpart in the reference (its tile map is PackMetadata.batch_ids_q /
+ * the real rows of every sequence) into `schedule` (fmlm_attn_workspace_bytes bytes, or
+ * that less fmlm_attn_records_bytes) so later fmlm_attn_fwd calls with p->schedule =
+ * schedule skip rebuilding it.  No counterpart in the reference (its tile map is PackMetadata.batch_ids_q /
  * q_tile_starts_q at block_n granularity, host_utils.py:74-107). */
 FMLM_API int fmlm_attn_schedule(const fmlm_attn_params* p, void* schedule, int64_t schedule_bytes,
                                 void* stream);

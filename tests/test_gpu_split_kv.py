@@ -1,0 +1,136 @@
+"""GPU tests of key ranges split over workgroups and merged (dense calls with few query
+tiles, the 512-wide latent with few query rows), against the float64 oracle and against
+the same call unsplit.
+
+Tolerance: 1e-2 as for every 16-bit forward test; the merged row differs from the unsplit
+one by the rounding of its fp32 weights only, so the two are within one rounding of the
+output type of each other (2^-8 relative at bf16, 2^-11 at fp16), plus 1e-5 for fp32."""
+
+from __future__ import annotations
+
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from flash_mlm import InferenceCache, _lib, build_pack_metadata, flash_attn_mlm, flash_attn_mlm_compressed, \
+    unpack_from_kernel
+from flash_mlm.host import host as hh
+from oracle import attention_ref as ar
+
+pytestmark = pytest.mark.gpu
+
+
+def _np(t):
+    return t.detach().float().cpu().numpy().astype(np.float64)
+
+
+def _randn(gen, shape, dtype, device, std=1.0):
+    return (torch.randn(shape, generator=gen) * std).to(dtype).to(device)
+
+
+DENSE = [
+    # B, H, N, D, context rows, context batches, dtype: part counts that divide the key
+    # tiles unevenly, one query row, a row past a tile, one row short of a key tile
+    (1, 4, 1, 64, 511, 1, torch.bfloat16),
+    (2, 3, 65, 64, 1000, 2, torch.float16),
+    (1, 2, 17, 128, 6001, 1, torch.bfloat16),
+    (1, 1, 128, 256, 640, 1, torch.float16),
+    (3, 2, 130, 32, 449, 3, torch.bfloat16),
+    (1, 3, 600, 16, 1, 1, torch.float16),
+]
+
+
+@pytest.mark.parametrize("B,H,N,D,C,cbs,dtype", DENSE)
+def test_dense_split_matches_oracle_and_unsplit(B, H, N, D, C, cbs, dtype, device):
+    gen = torch.Generator().manual_seed(D + N)
+    q, k, v = (_randn(gen, (B, H, N, D), dtype, device) for _ in range(3))
+    kc, vc = (_randn(gen, (cbs * H * C, D), dtype, device) for _ in range(2))
+    cache = InferenceCache()
+    cache.prefill_kv_cache(0, k_cache=kc, v_cache=vc, context_batch_size=cbs, is_mla=False, num_heads=H, head_dim=D)
+    scale = D ** -0.5
+    out, plan = hh._dense_impl(q, k, v, scale, cache, 0, False, None, False, run=False)
+    assert plan.records > 0, "the shape is meant to split"
+    plan()
+    tol = 1e-5 if dtype == torch.float32 else 1e-2
+    ref = ar.mlm_attention_dense(_np(q), _np(k), _np(v), scale, k_cache=_np(kc), v_cache=_np(vc), context_len=C,
+                                 context_batch_size=cbs)
+    np.testing.assert_allclose(_np(out), ref, atol=tol, rtol=tol)
+    again = flash_attn_mlm(q, k, v, scale, inference_cache=cache, layer_id=0)
+    assert torch.equal(again, out)
+    # without a workspace the C ABI runs the call unsplit
+    p = _lib.AttnParams.from_buffer_copy(plan.params)
+    whole = torch.full_like(out, float("nan"))
+    p.o, p.workspace, p.workspace_bytes = whole.data_ptr(), None, 0
+    _lib.check(plan.lib.fmlm_attn_fwd(ctypes.byref(p), plan.stream), "fmlm_attn_fwd")
+    ulp = {torch.bfloat16: 2.0**-8, torch.float16: 2.0**-11, torch.float32: 1e-5}[dtype]
+    torch.testing.assert_close(out.float(), whole.float(), atol=ulp * float(whole.float().abs().max()), rtol=ulp)
+
+
+@pytest.mark.parametrize("paged", [False, True])
+@pytest.mark.parametrize("H,lengths,ctx", [
+    (64, [1, 0, 4, 2], [2000, 900, 0, 5]),       # tiles of 64, 128 and 256 rows, short and empty contexts
+    (16, [3], [4097]),                           # one tile, the most parts
+    (5, [7, 1, 30], [333, 1024, 64 * 9]),        # odd heads: rows of a tile span heads
+])
+def test_latent_split_matches_oracle(H, lengths, ctx, paged, device):
+    gen = torch.Generator().manual_seed(H)
+    dtype, D, N, B = torch.bfloat16, 512, max(lengths), len(lengths)
+    q, k = (_randn(gen, (B, H, N, D), dtype, device, 0.5) for _ in range(2))
+    cu = [0, *np.cumsum(ctx).tolist()]
+    kc = _randn(gen, (cu[-1], D), dtype, device, 0.5)
+    cache = InferenceCache()
+    if paged:
+        need = [(c + 63) // 64 for c in ctx]
+        pool = torch.zeros((1, sum(need), 64, D), dtype=dtype, device=device)
+        table = torch.zeros((B, max(need)), dtype=torch.int32)
+        for b, c in enumerate(ctx):
+            first = sum(need[:b])
+            table[b, :need[b]] = torch.arange(first, first + need[b], dtype=torch.int32)
+            pool[0, first:first + need[b]].view(-1, D)[:c] = kc[cu[b]:cu[b + 1]]
+        cache.prefill_paged_kv_cache(0, k_pages=pool, block_table=table.to(device),
+                                     context_lens=torch.tensor(ctx, dtype=torch.int32), is_mla=True, num_heads=H,
+                                     head_dim=D)
+    else:
+        cache.prefill_kv_cache(0, k_cache=kc, total_context_len=cu[-1], context_batch_size=B, is_mla=True,
+                               cu_seqlens_kv=torch.tensor(cu, dtype=torch.int32, device=device), num_heads=H,
+                               head_dim=D)
+    meta = build_pack_metadata(torch.tensor(lengths, dtype=torch.int32, device=device), N, 64)
+    scale = D ** -0.5
+    out = flash_attn_mlm_compressed(q, k, k, H, meta, scale, cache, 0, is_mla=True, block_n=64)
+    ref = ar.mlm_attention_packed(_np(q), _np(k), _np(k), lengths, scale, is_mla=True, k_cache=_np(kc),
+                                  cu_seqlens_kv=cu, total_context_len=cu[-1], context_batch_size=B)
+    np.testing.assert_allclose(_np(unpack_from_kernel(out, meta, H)), ref, atol=1e-2, rtol=1e-2)
+
+
+def test_split_launches_of_one_schedule_do_not_share_partial_results(device):
+    """Calls on the same metadata from two streams may overlap: each brings its own records."""
+    gen = torch.Generator().manual_seed(9)
+    B, H, N, D = 4, 32, 4, 512
+    meta = build_pack_metadata(torch.tensor([4, 1, 3, 2], dtype=torch.int32, device=device), N, 64)
+    cases = []
+    for _ in range(2):
+        q, k = (_randn(gen, (B, H, N, D), torch.bfloat16, device, 0.5) for _ in range(2))
+        kc = _randn(gen, (B * 1500, D), torch.bfloat16, device, 0.5)
+        cache = InferenceCache()
+        cache.prefill_kv_cache(0, k_cache=kc, total_context_len=B * 1500, context_batch_size=B, is_mla=True,
+                               cu_seqlens_kv=torch.arange(B + 1, dtype=torch.int32, device=device) * 1500,
+                               num_heads=H, head_dim=D)
+        cases.append((q, k, cache))
+
+    def call(c):
+        return flash_attn_mlm_compressed(c[0], c[1], c[1], H, meta, D ** -0.5, c[2], 0, is_mla=True, block_n=64)
+
+    want = [call(c) for c in cases]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    got = [[], []]
+    for _ in range(20):
+        for i, s in enumerate(streams):
+            with torch.cuda.stream(s):
+                got[i].append(call(cases[i]))
+    torch.cuda.synchronize()
+    for i in range(2):
+        for g in got[i]:
+            assert torch.equal(g, want[i])
