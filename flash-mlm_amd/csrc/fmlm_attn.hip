@@ -18,8 +18,8 @@
 //   * O^T = V^T P^T with the same instruction; the accumulator again keeps one query
 //     per lane, so the online-softmax rescale is lane-local.
 //   * fp32 accumulation, exp2 with scale*log2(e) folded, P rounded to the input type.
-// The fp32 path (and head dims without an MFMA instantiation) uses a SIMT kernel with
-// the same addressing.
+// fp32 inputs have a kernel of their own on the fp32 MFMA (attn_f32_kernel); head dims
+// without an MFMA instantiation use a SIMT kernel with the same addressing.
 #include "fmlm_common.h"
 
 #include <algorithm>
@@ -1888,9 +1888,259 @@ __global__ __launch_bounds__(MlaRowsCfg::NT, 1) void attn_mla_rows_kernel(
 }
 
 // ---------------------------------------------------------------------------
+// fp32 kernel on the matrix cores (v_mfma_f32_16x16x4_f32: fp32 operands and accumulation,
+// 32 cycles each, so the products cost 16 times the 16-bit kernels' and bound the kernel:
+// nothing is staged in LDS, every fragment comes straight from L1 / L2).  One workgroup is
+// one (query tile of QB*16 rows, head); its 4 waves split every 64-key tile, 16 keys each,
+// and add up their partial results through LDS at the end, so that a call of a few query
+// rows still has 4 waves per tile at work.  Lane (j + 16g) of a fragment:
+//   K (A of S^T = K Q^T), Q (B)  row j, columns 16s + 4g .. +4 as one 16-byte load: MFMA e
+//                                of step s contracts columns 16s + 4g' + e, g' = 0..3
+//   S^T                          key 4g + r of query j in register r, which is the B
+//                                operand of the MFMA that contracts keys 4g' + r
+//   V^T (A of O^T = V^T P^T)     E consecutive columns of key row 4g + r in one load; MFMA
+//                                e builds the columns E*i + e (i < 16) of a 16E-wide group
+// so a lane ends up with 4E consecutive columns of O per group.
+// The next tile's K is loaded behind this tile's S, V behind the previous tile's P V: one
+// register copy of each.  Bound by the MFMAs: 8 x 12 heads x 512 x 512, D = 64, 73 us, 88
+// TFLOP/s (D = 128: 92; a library fp32 product reaches 154); the SIMT kernel below ran at
+// 13.  With loops in place of `skip` the compiler moved V's loads behind the S MFMAs: 85 us.
+// ---------------------------------------------------------------------------
+FMLM_DEV f32x4 mfma_f32(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+
+template <int D, int QB>
+struct F32Cfg {
+  static constexpr int NW = 4;
+  static constexpr int NT = NW * 64;
+  static constexpr int BQ = 16 * QB;
+  static constexpr int BK = kSplitBK;             // keys per tile, 16 per wave
+  static constexpr int DS = D / 16;               // 16-column steps of S^T
+  static constexpr int E = D >= 64 ? 4 : D / 16;  // columns per lane and V load
+  static constexpr int NG = D / (16 * E);         // column groups of O^T
+  static constexpr int OP = D + 4;                // LDS row pitch (floats): 16 rows on distinct banks
+  static constexpr int LDS_BYTES = NW * BQ * (OP + 2) * 4;
+  // waves per SIMD: the fragments of 256 columns take more than 256 registers
+  static constexpr int WPS = D >= 256 ? 1 : 2;
+  static_assert(BK == NW * 16, "16 keys of a tile per wave");
+};
+
+// E consecutive floats
+template <int E>
+struct FloatN {
+  typedef float type __attribute__((ext_vector_type(E)));
+};
+template <>
+struct FloatN<1> {
+  typedef float type;
+};
+template <int E>
+FMLM_DEV float elem_of(const typename FloatN<E>::type& x, int e) {
+  if constexpr (E == 1) return x;
+  else return x[e];
+}
+
+template <int D, int QB>
+__global__ __launch_bounds__(256, (F32Cfg<D, QB>::WPS)) void attn_f32_kernel(
+    const fmlm_attn_params p, const int4* __restrict__ units, const int32_t* __restrict__ hdr, const SplitArgs spa) {
+  typedef F32Cfg<D, QB> C;
+  typedef typename FloatN<C::E>::type vE;
+  extern __shared__ __align__(16) char smem_raw[];
+  float* const ob = (float*)smem_raw;             // [NW][BQ][OP]
+  float* const mb = ob + C::NW * C::BQ * C::OP;   // [NW][BQ]
+  float* const lb = mb + C::NW * C::BQ;           // [NW][BQ]
+
+  const int u = p.cu_seqlens_q ? workgroup_unit(hdr) : (int)blockIdx.x;
+  WorkItem w;
+  if (u < 0 || !resolve_work(p, units, u, C::BQ, w, spa)) return;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, g = lane >> 4;
+  const float c = p.scale * kLog2e;
+
+  f32x4 q[QB][C::DS];
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb) {
+    const int row = qb * 16 + l16;
+    const float* src = (const float*)p.q + w.q_row0 + (int64_t)row * w.q_sn + 4 * g;
+#pragma unroll
+    for (int ds = 0; ds < C::DS; ++ds)
+      q[qb][ds] = row < w.qcount ? *(const f32x4*)(src + 16 * ds) : f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+
+  const int n0 = w.seg[0].n, n1 = w.seg[1].n;
+  const int nt0 = (n0 + C::BK - 1) / C::BK;
+  const int ntiles = nt0 + (n1 + C::BK - 1) / C::BK;
+  const int tb = (int)((int64_t)w.split_s * ntiles / w.split_n);
+  const int te = (int)((int64_t)(w.split_s + 1) * ntiles / w.split_n);
+  const float* const kp0 = (const float*)w.seg[0].k + w.seg[0].kbase;
+  const float* const kp1 = (const float*)w.seg[1].k + w.seg[1].kbase;
+  const float* const vp0 = (const float*)w.seg[0].v + w.seg[0].vbase;
+  const float* const vp1 = (const float*)w.seg[1].v + w.seg[1].vbase;
+  // this wave's first key of tile t, and its segment's key count
+  auto key0 = [&](int t) { return (t < nt0 ? t : t - nt0) * C::BK + wave * 16; };
+  auto nkeys = [&](int t) { return t < nt0 ? n0 : n1; };
+  // a segment's last tile may have no keys of this wave: the context's is skipped, the
+  // main segment's ends the walk early
+  const int skip = wave * 16 >= n0 - (nt0 - 1) * C::BK ? nt0 - 1 : -1;
+  const int end = te == ntiles && te > nt0 && key0(te - 1) >= n1 ? te - 1 : te;
+  auto from = [&](int t) { return t == skip ? t + 1 : t; };
+  // row pitches lie below 2^22 elements (check_params): one 32 x 32 bit product
+  auto row_off = [](int key, int64_t sn) { return (uint64_t)(uint32_t)key * (uint32_t)sn; };
+  // rows past the segment's end repeat its last row (their scores are masked)
+  auto load_k = [&](int t, f32x4(&k)[C::DS]) {
+    const int key = min(key0(t) + l16, nkeys(t) - 1);
+    const float* src = (t < nt0 ? kp0 : kp1) + row_off(key, t < nt0 ? w.seg[0].ksn : w.seg[1].ksn) + 4 * g;
+#pragma unroll
+    for (int ds = 0; ds < C::DS; ++ds) k[ds] = *(const f32x4*)(src + 16 * ds);
+  };
+  auto load_v = [&](int t, vE(&v)[4][C::NG]) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int key = min(key0(t) + 4 * g + r, nkeys(t) - 1);
+      const float* src = (t < nt0 ? vp0 : vp1) + row_off(key, t < nt0 ? w.seg[0].vsn : w.seg[1].vsn) + C::E * l16;
+#pragma unroll
+      for (int dg = 0; dg < C::NG; ++dg) v[r][dg] = *(const vE*)(src + 16 * C::E * dg);
+    }
+  };
+
+  f32x4 o[QB][C::NG][C::E];
+  float m_i[QB], l_i[QB];
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb) {
+    m_i[qb] = -INFINITY;
+    l_i[qb] = 0.f;
+#pragma unroll
+    for (int dg = 0; dg < C::NG; ++dg)
+#pragma unroll
+      for (int e = 0; e < C::E; ++e) o[qb][dg][e] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+
+  int t = from(tb);
+  if (t < end) {
+    f32x4 k[C::DS];
+    vE v[4][C::NG];
+    load_k(t, k);
+    while (t < end) {
+      load_v(t, v);
+      __builtin_amdgcn_sched_barrier(0);  // the loads stay ahead of the MFMAs that cover them
+      f32x4 s[QB];
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) s[qb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ds = 0; ds < C::DS; ++ds)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int qb = 0; qb < QB; ++qb) s[qb] = mfma_f32(k[ds][e], q[qb][ds][e], s[qb]);
+      __builtin_amdgcn_sched_barrier(0);
+      const int lim = nkeys(t) - key0(t) - 4 * g;  // key 4g + r is valid iff r < lim
+      const int tn = from(t + 1);
+      load_k(tn < end ? tn : t, k);  // unconditional: a branch here would make the wait for V wait for K too
+      __builtin_amdgcn_sched_barrier(0);
+      bool grow = false;
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) s[qb][r] = r < lim ? s[qb][r] * c : -INFINITY;
+        grow |= fmaxf(fmaxf(s[qb][0], s[qb][1]), fmaxf(s[qb][2], s[qb][3])) > m_i[qb] + kRescaleSlack;
+      }
+      if (__builtin_amdgcn_ballot_w64(grow)) {  // lazy rescale (kRescaleSlack)
+#pragma unroll
+        for (int qb = 0; qb < QB; ++qb) {
+          const float mx = lane_max_xor16_32(fmaxf(fmaxf(s[qb][0], s[qb][1]), fmaxf(s[qb][2], s[qb][3])));
+          const float m_new = mx > m_i[qb] + kRescaleSlack ? mx : m_i[qb];
+          const float alpha = m_new == m_i[qb] ? 1.f : fast_exp2(m_i[qb] - m_new);
+          m_i[qb] = m_new;
+          l_i[qb] *= alpha;
+#pragma unroll
+          for (int dg = 0; dg < C::NG; ++dg)
+#pragma unroll
+            for (int e = 0; e < C::E; ++e) o[qb][dg][e] *= alpha;
+        }
+      }
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) s[qb][r] = fast_exp2(s[qb][r] - (m_i[qb] == -INFINITY ? 0.f : m_i[qb]));
+        l_i[qb] += (s[qb][0] + s[qb][1]) + (s[qb][2] + s[qb][3]);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int dg = 0; dg < C::NG; ++dg)
+#pragma unroll
+          for (int e = 0; e < C::E; ++e)
+#pragma unroll
+            for (int qb = 0; qb < QB; ++qb)
+              o[qb][dg][e] = mfma_f32(elem_of<C::E>(v[r][dg], e), s[qb][r], o[qb][dg][e]);
+      t = tn;
+    }
+  }
+
+  // ---- the waves' partial results to LDS, then the rows' sums over the waves
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb) {
+    const int row = qb * 16 + l16;
+    float l = l_i[qb];
+    l += __shfl_xor(l, 16);
+    l += __shfl_xor(l, 32);
+    if (g == 0) {
+      mb[wave * C::BQ + row] = m_i[qb];
+      lb[wave * C::BQ + row] = l;
+    }
+    float* dst = ob + (wave * C::BQ + row) * C::OP + 4 * C::E * g;
+#pragma unroll
+    for (int dg = 0; dg < C::NG; ++dg)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        vE x;
+        if constexpr (C::E == 1) x = o[qb][dg][0][r];
+        else
+#pragma unroll
+          for (int e = 0; e < C::E; ++e) x[e] = o[qb][dg][e][r];
+        *(vE*)(dst + 16 * C::E * dg + C::E * r) = x;
+      }
+  }
+  __syncthreads();
+  char* rec = nullptr;
+  if (w.split_n > 1) {
+    rec = split_record(hdr, spa, w.rec0 + w.split_s);
+    if (!rec) return;
+  }
+  for (int i = tid; i < C::BQ * (D / 4); i += C::NT) {
+    const int row = i / (D / 4), col = (i % (D / 4)) * 4;
+    if (row >= w.qcount) break;
+    float m[C::NW], M = -INFINITY, L = 0.f;
+#pragma unroll
+    for (int wv = 0; wv < C::NW; ++wv) {
+      m[wv] = mb[wv * C::BQ + row];
+      M = fmaxf(M, m[wv]);
+    }
+    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int wv = 0; wv < C::NW; ++wv) {
+      const float a = m[wv] == M ? 1.f : fast_exp2(m[wv] - M);
+      L += a * lb[wv * C::BQ + row];
+      acc += a * *(const f32x4*)(ob + (wv * C::BQ + row) * C::OP + col);
+    }
+    if (rec) {  // this part's record (O / l, then m and l per row) for merge_kernel
+      *(f32x4*)(rec + ((int64_t)row * D + col) * 4) = acc * (L > 0.f ? 1.f / L : 0.f);
+      if (col == 0) {
+        float* const ml = (float*)(rec + (int64_t)C::BQ * D * 4);
+        ml[row] = M;
+        ml[C::BQ + row] = L;
+      }
+    } else {
+      *(f32x4*)((float*)p.o + w.o_row0 + (int64_t)row * w.o_sn + col) = acc * (L > 0.f ? 1.f / L : 1.f);
+      if (p.lse && col == 0) store_lse(p, w.h, w.q0, w.qpos0 + row, M, L);
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
 // SIMT kernel: one query row per TPR threads (each holding D/TPR dims), K/V tiles
-// staged in LDS as fp32.  Used for fp32 inputs and head dims without an MFMA
-// instantiation.  Probabilities are rounded to T before P.V like the MFMA path.
+// staged in LDS as fp32.  Used for head dims without an MFMA instantiation and fp32 main
+// keys that need a per-row sequence lookup.  Probabilities are rounded to T before P.V like the MFMA path.
 // ---------------------------------------------------------------------------
 template <int D>
 struct SimtCfg {
@@ -2158,6 +2408,12 @@ static Launch simt_launch() {
   return Launch{C::RPW, C::NT, C::LDS_BYTES, (const void*)&attn_simt_kernel<T, D>};
 }
 
+template <int D, int QB>
+static Launch f32_launch() {
+  typedef F32Cfg<D, QB> C;
+  return Launch{C::BQ, C::NT, C::LDS_BYTES, (const void*)&attn_f32_kernel<D, QB>, true};
+}
+
 template <typename T, int D, int QB, int NW, int BK, int PPB = 0>
 static Launch mfma3_launch(bool paged) {
   typedef Mfma3Cfg<T, D, QB, NW, BK, PPB> C;
@@ -2265,13 +2521,33 @@ static bool pick_simt(int D, Launch& L) {
   }
 }
 
+// fp32 on the matrix cores, D <= 256: the widest query tile whose fragments fit two waves
+// per SIMD (wide tiles read each key fewer times: 8 x 12 heads x 512, D = 128, 141 us with
+// 32-row tiles, 172 with 16).  A small batch takes 16-row tiles, twice the workgroups: at
+// D = 64 below 256 tiles of 32 rows (2 x 8 heads x 128: 6.4 us); at D = 128 below 64, since
+// long contexts split anyway and wide tiles then merge less (4 x 8 x 100 queries, 1000
+// context rows: 32 us against 38).
+static bool pick_f32(const fmlm_attn_params& p, Launch& L) {
+  if ((p.flags & FMLM_FLAG_CAUSAL_SEQ) && p.cu_seqlens_q && p.kv_layout != FMLM_LAYOUT_PACKED) return false;
+  const int64_t rows = p.cu_seqlens_q ? p.total_q : (int64_t)p.B * p.N;
+  const bool small = p.H * rows < (p.D == 64 ? 256 : 64) * 32;
+  switch (p.D) {
+    case 16: L = f32_launch<16, 4>(); return true;
+    case 32: L = f32_launch<32, 2>(); return true;
+    case 64: L = small ? f32_launch<64, 1>() : f32_launch<64, 2>(); return true;
+    case 128: L = small ? f32_launch<128, 1>() : f32_launch<128, 2>(); return true;
+    case 256: L = f32_launch<256, 1>(); return true;
+    default: return false;
+  }
+}
+
 static int pick_launch(const fmlm_attn_params& p, Launch& L) {
   bool ok = false;
   if (p.tile_config < 0) return FMLM_E_ARG;
   switch (p.dtype) {
     case FMLM_DTYPE_BF16: ok = pick_mfma<bf16>(p, L) || (p.tile_config <= 1 && pick_simt<bf16>(p.D, L)); break;
     case FMLM_DTYPE_F16: ok = pick_mfma<f16>(p, L) || (p.tile_config <= 1 && pick_simt<f16>(p.D, L)); break;
-    case FMLM_DTYPE_F32: ok = pick_simt<float>(p.D, L); break;
+    case FMLM_DTYPE_F32: ok = pick_f32(p, L) || pick_simt<float>(p.D, L); break;
     default: return FMLM_E_DTYPE;
   }
   if (!ok) return p.tile_config > 1 ? FMLM_E_ARG : FMLM_E_HEAD_DIM;
@@ -2497,8 +2773,10 @@ static int launch_attention(const fmlm_attn_params& p, const Launch& L, const Sp
     const dim3 mg((unsigned)std::min<int64_t>(groups * merge_chunks(p, L.bq, hp), 4096));
     if (p.dtype == FMLM_DTYPE_BF16)
       hipLaunchKernelGGL(merge_kernel<bf16>, mg, dim3(kMergeThreads), 0, s, p, L.bq, (const int32_t*)header, spa, hp);
-    else
+    else if (p.dtype == FMLM_DTYPE_F16)
       hipLaunchKernelGGL(merge_kernel<f16>, mg, dim3(kMergeThreads), 0, s, p, L.bq, (const int32_t*)header, spa, hp);
+    else
+      hipLaunchKernelGGL(merge_kernel<float>, mg, dim3(kMergeThreads), 0, s, p, L.bq, (const int32_t*)header, spa, hp);
   }
   return launch_status();
 }

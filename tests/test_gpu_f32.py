@@ -1,0 +1,63 @@
+"""GPU tests of the fp32 kernels (matrix cores) at the sizes where their tiles end, against
+the float64 oracle on the same inputs.
+
+Tolerance: a score is a sum of D products of values around 1 in fp32, off by up to about
+sqrt(D) * 2^-24 * its size (at most 8 here), which is its weight's relative error; the
+output, at most about 3, is then off by less than 16 * 8 * 6e-8 * 3 = 2.3e-5 at D = 256."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from flash_mlm import InferenceCache, build_pack_metadata, flash_attn_mlm_compressed, unpack_from_kernel
+from oracle import attention_ref as ar
+
+pytestmark = pytest.mark.gpu
+TOL = 2.5e-5
+
+
+def _np(t):
+    return t.detach().cpu().numpy().astype(np.float64)
+
+
+def _case(device, D, H, lengths, ctx, seed, mla=False, grad=False):
+    gen = torch.Generator().manual_seed(seed)
+    B, N = len(lengths), max(lengths)
+    r = lambda *shape: torch.randn(shape, generator=gen).to(device).requires_grad_(grad)  # noqa: E731
+    q, k, v = (r(B, H, N, D) for _ in range(3))
+    cu = [0, *np.cumsum(ctx).tolist()]
+    hk = 1 if mla else H
+    kc, vc = r(hk * cu[-1], D), None if mla else r(hk * cu[-1], D)
+    cache = InferenceCache()
+    cache.prefill_kv_cache(0, k_cache=kc, v_cache=vc, total_context_len=cu[-1], context_batch_size=len(ctx),
+                           cu_seqlens_kv=torch.tensor(cu, dtype=torch.int32, device=device), is_mla=mla,
+                           num_heads=H, head_dim=D)
+    meta = build_pack_metadata(torch.tensor(lengths, dtype=torch.int32, device=device), N, 64)
+    return q, k, v, kc, vc, cu, cache, meta
+
+
+# sequence lengths around the 16- and 32-row query tiles and the 16- and 64-key tiles, with
+# context lengths that leave none, some or all of a tile's waves without keys; (H, lengths,
+# ctx) of the last case fill the chip with wide query tiles
+EDGES = [
+    (3, [1, 15, 16, 17, 33, 64, 65], [0, 1, 16, 63, 64, 65, 130]),
+    (2, [31, 0, 5], [48]),
+    (16, [200, 129, 256], [17, 300, 0]),
+]
+
+
+@pytest.mark.parametrize("causal,mla", [(False, False), (True, False), (False, True)])
+@pytest.mark.parametrize("H,lengths,ctx", EDGES)
+@pytest.mark.parametrize("D", [16, 32, 64, 128, 256])
+def test_f32_forward_edges(D, H, lengths, ctx, causal, mla, device):
+    q, k, v, kc, vc, cu, cache, meta = _case(device, D, H, lengths, ctx, D + H, mla)
+    scale = D ** -0.5
+    out = flash_attn_mlm_compressed(q, k, v, H, meta, scale, cache, 0, is_mla=mla, block_n=64,
+                                    causal_query_seq_attn=causal)
+    ref = ar.mlm_attention_packed(_np(q), _np(k), _np(k if mla else v), lengths, scale, is_mla=mla,
+                                  causal_query_seq_attn=causal, k_cache=_np(kc),
+                                  v_cache=None if mla else _np(vc), cu_seqlens_kv=cu, total_context_len=cu[-1],
+                                  context_batch_size=len(ctx))
+    np.testing.assert_allclose(_np(unpack_from_kernel(out, meta, H)), ref, atol=TOL, rtol=TOL)

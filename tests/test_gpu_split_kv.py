@@ -39,6 +39,7 @@ DENSE = [
     (1, 1, 128, 256, 640, 1, torch.float16),
     (3, 2, 130, 32, 449, 3, torch.bfloat16),
     (1, 3, 600, 16, 1, 1, torch.float16),
+    (1, 2, 33, 64, 2050, 1, torch.float32),
 ]
 
 
