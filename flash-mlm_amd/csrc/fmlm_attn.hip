@@ -1906,8 +1906,6 @@ __global__ __launch_bounds__(MlaRowsCfg::NT, 1) void attn_mla_rows_kernel(
 // TFLOP/s (D = 128: 92; a library fp32 product reaches 154); the SIMT kernel below ran at
 // 13.  With loops in place of `skip` the compiler moved V's loads behind the S MFMAs: 85 us.
 // ---------------------------------------------------------------------------
-FMLM_DEV f32x4 mfma_f32(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
-
 template <int D, int QB>
 struct F32Cfg {
   static constexpr int NW = 4;
@@ -1923,21 +1921,6 @@ struct F32Cfg {
   static constexpr int WPS = D >= 256 ? 1 : 2;
   static_assert(BK == NW * 16, "16 keys of a tile per wave");
 };
-
-// E consecutive floats
-template <int E>
-struct FloatN {
-  typedef float type __attribute__((ext_vector_type(E)));
-};
-template <>
-struct FloatN<1> {
-  typedef float type;
-};
-template <int E>
-FMLM_DEV float elem_of(const typename FloatN<E>::type& x, int e) {
-  if constexpr (E == 1) return x;
-  else return x[e];
-}
 
 template <int D, int QB>
 __global__ __launch_bounds__(256, (F32Cfg<D, QB>::WPS)) void attn_f32_kernel(

@@ -1568,8 +1568,8 @@ __global__ __launch_bounds__(kBwdNW * 64, BwdCfg<D>::WPS) void attn_bwd_dkv_kern
 }
 
 // ---------------------------------------------------------------------------
-// SIMT backward (fp32 inputs, and head dims without an MFMA kernel): the same two-kernel
-// split as above.  TPR threads per query row (dq) or per key row (dK / dV), each holding
+// SIMT backward (head dims and modes without an MFMA kernel): the same two-kernel split as
+// above.  TPR threads per query row (dq) or per key row (dK / dV), each holding
 // DPT dims; a row's partial dot products meet through xor shuffles inside its TPR lanes,
 // and the staged tiles are fp32 in LDS, read as float4.
 // ---------------------------------------------------------------------------
@@ -1828,6 +1828,415 @@ __global__ __launch_bounds__(256) void attn_bwd_dkv_simt_kernel(const fmlm_attn_
 }
 
 // ---------------------------------------------------------------------------
+// fp32 backward on the matrix cores (v_mfma_f32_16x16x4_f32; head dims up to 256,
+// contiguous contexts), bound by the MFMAs like the fp32 forward and built like it: no LDS
+// in the loops, fragments straight from L1 / L2 in its two forms, "row" (lane (j + 16g):
+// row j, columns 16s + 4g .. +4, contracted over the columns) and "col" (row 4g + r, E
+// consecutive columns, contracted over the rows), each loaded behind the MFMAs of another.
+// The 4 waves of a workgroup split the contraction's long side (dq: 16 keys of every 64;
+// dK / dV: 16 query rows of every 64) and add their sums up through LDS at the end.
+// ---------------------------------------------------------------------------
+template <int D>
+struct F32BwdCfg {
+  static constexpr int DS = D / 16;               // 16-column steps of a row fragment
+  static constexpr int E = D >= 64 ? 4 : D / 16;  // columns per lane of a col fragment
+  static constexpr int NG = D / (16 * E);         // column groups
+  static constexpr int OP = D + 4;                // LDS row pitch (floats)
+  // 16-row query blocks of a dq workgroup, 16-key blocks of a dK / dV workgroup: as many as
+  // fit two waves per SIMD (8 x 12 heads x 512, D = 64: two of each 275 us; one query block
+  // 292, one key block 306)
+  static constexpr int QB = D == 16 ? 4 : D <= 64 ? 2 : 1;
+  static constexpr int KB = QB;
+  static constexpr int BQ = 16 * QB, KEYS = 16 * KB;
+  static constexpr int DQ_LDS = kBwdNW * BQ * (OP + 3) * 4;
+  static constexpr int DKV_LDS = kBwdNW * KEYS * OP * 4;
+  // waves per SIMD: 256 columns take more than 256 registers
+  static constexpr int WPS = D >= 256 ? 1 : 2;
+};
+
+// the row fragments of one row (src: its column 4g)
+template <int D>
+FMLM_DEV void load_row_frag(const float* src, f32x4 (&x)[F32BwdCfg<D>::DS]) {
+#pragma unroll
+  for (int ds = 0; ds < F32BwdCfg<D>::DS; ++ds) x[ds] = *(const f32x4*)(src + 16 * ds);
+}
+// acc[i] += A B over the columns, A's row fragments a and B's b[i]
+template <int D, int N>
+FMLM_DEV void mma_rows(const f32x4 (&a)[F32BwdCfg<D>::DS], const f32x4 (&b)[N][F32BwdCfg<D>::DS], f32x4 (&acc)[N]) {
+#pragma unroll
+  for (int ds = 0; ds < F32BwdCfg<D>::DS; ++ds)
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int i = 0; i < N; ++i) acc[i] = mfma_f32(a[ds][e], b[i][ds][e], acc[i]);
+}
+// o[i] += X^T b[i] over 16 rows, X's col fragments x: row 4g + r against b[i][r]
+template <int D, int N>
+FMLM_DEV void mma_cols(const typename FloatN<F32BwdCfg<D>::E>::type (&x)[4][F32BwdCfg<D>::NG], const f32x4 (&b)[N],
+                       f32x4 (&o)[N][F32BwdCfg<D>::NG][F32BwdCfg<D>::E]) {
+  typedef F32BwdCfg<D> C;
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int dg = 0; dg < C::NG; ++dg)
+#pragma unroll
+      for (int e = 0; e < C::E; ++e)
+#pragma unroll
+        for (int i = 0; i < N; ++i) o[i][dg][e] = mfma_f32(elem_of<C::E>(x[r][dg], e), b[i][r], o[i][dg][e]);
+}
+// the lane's columns of accumulator o, row l16 of its block, to an LDS row
+template <int D>
+FMLM_DEV void store_cols(const f32x4 (&o)[F32BwdCfg<D>::NG][F32BwdCfg<D>::E], float* row, int g) {
+  typedef F32BwdCfg<D> C;
+  typedef typename FloatN<C::E>::type vE;
+#pragma unroll
+  for (int dg = 0; dg < C::NG; ++dg)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      vE x;
+      if constexpr (C::E == 1) x = o[dg][0][r];
+      else
+#pragma unroll
+        for (int e = 0; e < C::E; ++e) x[e] = o[dg][e][r];
+      *(vE*)(row + 4 * C::E * g + 16 * C::E * dg + C::E * r) = x;
+    }
+}
+
+template <int D>
+__global__ __launch_bounds__(256, F32BwdCfg<D>::WPS) void attn_bwd_dq_f32_kernel(const fmlm_attn_params p,
+                                                                                 const fmlm_attn_grads g_,
+                                                                                 const int32_t* qrec, int nq) {
+  typedef F32BwdCfg<D> C;
+  typedef typename FloatN<C::E>::type vE;
+  constexpr int QB = C::QB, BK = 64;
+  extern __shared__ __align__(16) char smem_raw[];
+  float* const ob = (float*)smem_raw;                 // [NW][BQ][OP]
+  float* const mb = ob + kBwdNW * C::BQ * C::OP;      // [NW][BQ]
+  float* const lb = mb + kBwdNW * C::BQ;              // [NW][BQ]
+  float* const delta_s = lb + kBwdNW * C::BQ;         // [BQ]
+
+  int u, h;
+  grid_unit((unsigned)p.H, u, h);
+  if (u >= nq) return;
+  int rec[9];  // the unit's record (query_record)
+  load_record(qrec + (int64_t)u * kRecInts, rec);
+  const int b = rec[0];
+  if (b < 0) return;
+  const int qpos0 = rec[1];
+  const SeqInfo si = rec_seq_info(rec + 2);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, g = lane >> 4;
+  const float c = p.scale * kLog2e;
+
+  f32x4 q[QB][C::DS], dof[QB][C::DS];
+  float delta[QB];
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb) {
+    const int row = qb * 16 + l16, pos = min(qpos0 + row, si.len - 1);
+    const float* qp = (const float*)p.q + row_at(p.q_layout, b, h, si.q0, pos, p.q_sb, p.q_sh, p.q_sn) + 4 * g;
+    const float* dp = (const float*)g_.dout + row_at(p.o_layout, b, h, si.q0, pos, g_.do_sb, g_.do_sh, g_.do_sn) + 4 * g;
+    const float* op = (const float*)p.o + row_at(p.o_layout, b, h, si.q0, pos, p.o_sb, p.o_sh, p.o_sn) + 4 * g;
+    load_row_frag<D>(qp, q[qb]);
+    load_row_frag<D>(dp, dof[qb]);
+    float d = 0.f;
+#pragma unroll
+    for (int ds = 0; ds < C::DS; ++ds) {
+      const f32x4 o4 = *(const f32x4*)(op + 16 * ds);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) d = fmaf(dof[qb][ds][e], o4[e], d);
+    }
+    d += __shfl_xor(d, 16);
+    delta[qb] = d + __shfl_xor(d, 32);
+    if (wave == 0 && g == 0) delta_s[row] = delta[qb];
+  }
+
+  const BSeg sc = ctx_seg_at(p, g_, rec[6], h, rec[7], rec[8]);
+  const BSeg sm = main_seg_at(p, g_, b, h, si);
+  const int nt0 = (sc.n + BK - 1) / BK, ntiles = nt0 + (sm.n + BK - 1) / BK;
+  // this wave's first key of tile t; a segment's last tile may have no keys of this wave
+  auto key0 = [&](int t) { return (t < nt0 ? t : t - nt0) * BK + wave * 16; };
+  auto nkeys = [&](int t) { return t < nt0 ? sc.n : sm.n; };
+  const int skip = wave * 16 >= sc.n - (nt0 - 1) * BK ? nt0 - 1 : -1;
+  const int end = ntiles > nt0 && key0(ntiles - 1) >= sm.n ? ntiles - 1 : ntiles;
+  auto from = [&](int t) { return t == skip ? t + 1 : t; };
+  // rows past the segment's end repeat its last row (their scores are masked)
+  auto row_of = [&](int t, int key, bool v) {
+    const bool cx = t < nt0;
+    const float* base = cx ? (const float*)(v ? sc.v : sc.k) + (v ? sc.vbase : sc.kbase)
+                           : (const float*)(v ? sm.v : sm.k) + (v ? sm.vbase : sm.kbase);
+    const int64_t sn = cx ? (v ? sc.vsn : sc.ksn) : (v ? sm.vsn : sm.ksn);
+    return base + (uint64_t)(uint32_t)min(key, nkeys(t) - 1) * (uint32_t)sn;
+  };
+
+  f32x4 acc[QB][C::NG][C::E];
+  float m_i[QB], l_i[QB];
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb) {
+    m_i[qb] = -INFINITY;
+    l_i[qb] = 0.f;
+#pragma unroll
+    for (int dg = 0; dg < C::NG; ++dg)
+#pragma unroll
+      for (int e = 0; e < C::E; ++e) acc[qb][dg][e] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  int t = from(0);
+  if (t < end) {
+    f32x4 kr[C::DS], vr[C::DS];
+    vE kc[4][C::NG];
+    load_row_frag<D>(row_of(t, key0(t) + l16, false) + 4 * g, kr);
+    while (t < end) {
+      load_row_frag<D>(row_of(t, key0(t) + l16, true) + 4 * g, vr);
+      __builtin_amdgcn_sched_barrier(0);  // loads stay ahead of the MFMAs that cover them
+      f32x4 s[QB], dp[QB];
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) s[qb] = dp[qb] = f32x4{0.f, 0.f, 0.f, 0.f};
+      mma_rows<D, QB>(kr, q, s);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float* src = row_of(t, key0(t) + 4 * g + r, false) + C::E * l16;
+#pragma unroll
+        for (int dg = 0; dg < C::NG; ++dg) kc[r][dg] = *(const vE*)(src + 16 * C::E * dg);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      mma_rows<D, QB>(vr, dof, dp);
+      __builtin_amdgcn_sched_barrier(0);
+      const int lim = nkeys(t) - key0(t) - 4 * g;  // key 4g + r is valid iff r < lim
+      const int tn = from(t + 1);
+      const int tl = tn < end ? tn : t;
+      load_row_frag<D>(row_of(tl, key0(tl) + l16, false) + 4 * g, kr);
+      __builtin_amdgcn_sched_barrier(0);
+      bool grow = false;
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) s[qb][r] = r < lim ? s[qb][r] * c : -INFINITY;
+        grow |= fmaxf(fmaxf(s[qb][0], s[qb][1]), fmaxf(s[qb][2], s[qb][3])) > m_i[qb] + kRescaleSlack;
+      }
+      if (__builtin_amdgcn_ballot_w64(grow)) {  // lazy rescale (kRescaleSlack)
+#pragma unroll
+        for (int qb = 0; qb < QB; ++qb) {
+          const float mx = lane_max_xor16_32(fmaxf(fmaxf(s[qb][0], s[qb][1]), fmaxf(s[qb][2], s[qb][3])));
+          const float m_new = mx > m_i[qb] + kRescaleSlack ? mx : m_i[qb];
+          const float alpha = m_new == m_i[qb] ? 1.f : fast_exp2(m_i[qb] - m_new);
+          m_i[qb] = m_new;
+          l_i[qb] *= alpha;
+#pragma unroll
+          for (int dg = 0; dg < C::NG; ++dg)
+#pragma unroll
+            for (int e = 0; e < C::E; ++e) acc[qb][dg][e] *= alpha;
+        }
+      }
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) {
+        const float mref = m_i[qb] == -INFINITY ? 0.f : m_i[qb];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          s[qb][r] = fast_exp2(s[qb][r] - mref);
+          dp[qb][r] = s[qb][r] * (dp[qb][r] - delta[qb]);
+        }
+        l_i[qb] += (s[qb][0] + s[qb][1]) + (s[qb][2] + s[qb][3]);
+      }
+      mma_cols<D, QB>(kc, dp, acc);
+      t = tn;
+    }
+  }
+
+  // ---- the waves' sums to LDS, then the rows' sums over the waves
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb) {
+    const int row = qb * 16 + l16;
+    float l = l_i[qb];
+    l += __shfl_xor(l, 16);
+    l += __shfl_xor(l, 32);
+    if (g == 0) {
+      mb[wave * C::BQ + row] = m_i[qb];
+      lb[wave * C::BQ + row] = l;
+    }
+    store_cols<D>(acc[qb], ob + (wave * C::BQ + row) * C::OP, g);
+  }
+  __syncthreads();
+  float* const st_lse = (float*)g_.workspace;
+  for (int i = tid; i < C::BQ * (D / 4); i += 256) {
+    const int row = i / (D / 4), col = (i % (D / 4)) * 4, pos = qpos0 + row;
+    if (pos >= si.len) break;
+    float m[kBwdNW], M = -INFINITY, L = 0.f;
+#pragma unroll
+    for (int w = 0; w < kBwdNW; ++w) {
+      m[w] = mb[w * C::BQ + row];
+      M = fmaxf(M, m[w]);
+    }
+    f32x4 sum = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < kBwdNW; ++w) {
+      const float a = m[w] == M ? 1.f : fast_exp2(m[w] - M);
+      L += a * lb[w * C::BQ + row];
+      sum += a * *(const f32x4*)(ob + (w * C::BQ + row) * C::OP + col);
+    }
+    float* dst = (float*)g_.dq + row_at(p.q_layout, b, h, si.q0, pos, g_.dq_sb, g_.dq_sh, g_.dq_sn);
+    *(f32x4*)(dst + col) = sum * (L > 0.f ? p.scale / L : 0.f);
+    if (col == 0) {
+      const int64_t at = (int64_t)h * p.total_q + si.q0 + pos;
+      st_lse[at] = L > 0.f ? M + __log2f(L) : INFINITY;
+      st_lse[(int64_t)p.H * p.total_q + at] = delta_s[row];
+    }
+  }
+}
+
+template <int D, bool CAUSAL>
+__global__ __launch_bounds__(256, F32BwdCfg<D>::WPS) void attn_bwd_dkv_f32_kernel(const fmlm_attn_params p,
+                                                                                  const fmlm_attn_grads g_, int n_ctx,
+                                                                                  const int32_t* krec, int nk) {
+  typedef F32BwdCfg<D> C;
+  typedef typename FloatN<C::E>::type vE;
+  constexpr int KB = C::KB, QS = kBwdNW * 16;
+  extern __shared__ __align__(16) char smem_raw[];
+  float* const red = (float*)smem_raw;  // [NW][KEYS][OP]
+
+  const bool mla = p.flags & FMLM_FLAG_MLA;
+  KeyUnit ku;
+  if (!resolve_key_unit<CAUSAL>(p, g_, n_ctx, krec, nk, ku)) return;
+  const BSeg& s = ku.s;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, g = lane >> 4;
+  const float c = p.scale * kLog2e;
+  // the row statistics: the forward's log2-sum-exp when it stored them, else the dq
+  // kernel's; delta from the dq kernel
+  const float* const st_delta = (const float*)g_.workspace + (int64_t)p.H * p.total_q;
+  const float* const st_lse = p.lse ? (const float*)p.lse : (const float*)g_.workspace;
+
+  f32x4 kf[KB][C::DS], vf[KB][C::DS];
+  f32x4 dk[KB][C::NG][C::E], dv[KB][C::NG][C::E];
+#pragma unroll
+  for (int kb = 0; kb < KB; ++kb) {
+    const int key = min(ku.j0 + kb * 16 + l16, s.n - 1);  // past the end: the last key, its P is 0
+    load_row_frag<D>((const float*)s.k + s.kbase + (int64_t)key * s.ksn + 4 * g, kf[kb]);
+    load_row_frag<D>((const float*)s.v + s.vbase + (int64_t)key * s.vsn + 4 * g, vf[kb]);
+#pragma unroll
+    for (int dg = 0; dg < C::NG; ++dg)
+#pragma unroll
+      for (int e = 0; e < C::E; ++e) dk[kb][dg][e] = dv[kb][dg][e] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+
+  const int hq_lo = ku.shared ? 0 : ku.kh, hq_hi = ku.shared ? p.H : ku.kh + 1;
+  const QuerySteps steps{&p, &ku, hq_hi, QS};
+  // each wave walks the steps that have rows of it (rows p0 + 16 wave ..) by itself
+  auto mine = [&](QStep st, SeqInfo& si) {
+    while (st.hq < hq_hi) {
+      si = seq_info(p, st.b);
+      if (st.p0 + wave * 16 < si.len) break;
+      st = steps.next(st, si.len);
+    }
+    return st;
+  };
+  auto q_row = [&](const QStep& st, const SeqInfo& si, int pos) {
+    return (const float*)p.q + row_at(p.q_layout, st.b, st.hq, si.q0, min(pos, si.len - 1), p.q_sb, p.q_sh, p.q_sn);
+  };
+  auto o_row = [&](const QStep& st, const SeqInfo& si, int pos) {
+    return (const float*)g_.dout +
+           row_at(p.o_layout, st.b, st.hq, si.q0, min(pos, si.len - 1), g_.do_sb, g_.do_sh, g_.do_sn);
+  };
+  SeqInfo si{};
+  QStep cur = mine(steps.first_from(hq_lo, ku.b_lo), si);
+  if (cur.hq < hq_hi) {
+    f32x4 qr[C::DS], dr[C::DS];
+    vE qc[4][C::NG], oc[4][C::NG];
+    load_row_frag<D>(q_row(cur, si, cur.p0 + wave * 16 + l16) + 4 * g, qr);
+    load_row_frag<D>(o_row(cur, si, cur.p0 + wave * 16 + l16) + 4 * g, dr);
+    while (true) {
+      const int r0 = cur.p0 + wave * 16 + 4 * g;  // rows r0 + r in this lane's accumulators
+      float lse[4], dl[4];
+      {
+        const int64_t at = (int64_t)cur.hq * p.total_q + si.q0;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          lse[r] = st_lse[at + min(r0 + r, si.len - 1)];
+          dl[r] = st_delta[at + min(r0 + r, si.len - 1)];
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      f32x4 sa[KB], dp[KB];
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb) sa[kb] = dp[kb] = f32x4{0.f, 0.f, 0.f, 0.f};
+      mma_rows<D, KB>(qr, kf, sa);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float* src = q_row(cur, si, r0 + r) + C::E * l16;
+#pragma unroll
+        for (int dg = 0; dg < C::NG; ++dg) qc[r][dg] = *(const vE*)(src + 16 * C::E * dg);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      mma_rows<D, KB>(dr, vf, dp);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float* src = o_row(cur, si, r0 + r) + C::E * l16;
+#pragma unroll
+        for (int dg = 0; dg < C::NG; ++dg) oc[r][dg] = *(const vE*)(src + 16 * C::E * dg);
+      }
+      SeqInfo sn = si;
+      const QStep nxt = mine(steps.next(cur, si.len), sn);
+      const bool more = nxt.hq < hq_hi;
+      const QStep ld = more ? nxt : cur;  // unconditional loads: a branch would lengthen the waits
+      const SeqInfo sl = more ? sn : si;
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb) {
+        const int key = ku.j0 + kb * 16 + l16;
+        const bool kvalid = key < s.n && (!ku.causal_main || key < si.mainlen);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float pv = kvalid && r0 + r < si.len ? fast_exp2(fmaf(sa[kb][r], c, -lse[r])) : 0.f;
+          sa[kb][r] = pv;
+          dp[kb][r] = pv * (dp[kb][r] - dl[r]) * p.scale;
+        }
+      }
+      mma_cols<D, KB>(qc, dp, dk);
+      __builtin_amdgcn_sched_barrier(0);
+      load_row_frag<D>(q_row(ld, sl, ld.p0 + wave * 16 + l16) + 4 * g, qr);
+      if constexpr (D < 256) load_row_frag<D>(o_row(ld, sl, ld.p0 + wave * 16 + l16) + 4 * g, dr);
+      __builtin_amdgcn_sched_barrier(0);
+      mma_cols<D, KB>(oc, sa, dv);
+      // 256 columns: behind the next S instead, for want of registers
+      if constexpr (D >= 256) load_row_frag<D>(o_row(ld, sl, ld.p0 + wave * 16 + l16) + 4 * g, dr);
+      if (!more) break;
+      cur = nxt;
+      si = sn;
+    }
+  }
+
+  // ---- the waves' sums through LDS; with MLA V is K and both gradients are dK's
+#pragma unroll
+  for (int out = 0; out < 2; ++out) {
+    if (out == 1 && mla) break;
+    if (out == 1) __syncthreads();
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+      if (out == 0 && mla) {
+#pragma unroll
+        for (int dg = 0; dg < C::NG; ++dg)
+#pragma unroll
+          for (int e = 0; e < C::E; ++e) dk[kb][dg][e] += dv[kb][dg][e];
+      }
+      store_cols<D>(out == 0 ? dk[kb] : dv[kb], red + (wave * C::KEYS + kb * 16 + l16) * C::OP, g);
+    }
+    __syncthreads();
+    for (int i = tid; i < C::KEYS * (D / 4); i += 256) {
+      const int row = i / (D / 4), col = (i % (D / 4)) * 4, key = ku.j0 + row;
+      if (key >= s.n) break;
+      f32x4 sum = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int w = 0; w < kBwdNW; ++w) sum += *(const f32x4*)(red + (w * C::KEYS + row) * C::OP + col);
+      float* dst = out == 0 ? (float*)s.dk + s.dkbase + (int64_t)key * s.dksn : (float*)s.dv + s.dvbase + (int64_t)key * s.dvsn;
+      *(f32x4*)(dst + col) = sum;
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
 struct BwdFns {
@@ -1863,7 +2272,30 @@ static BwdFns bwd_simt_fns() {
                 C::R};
 }
 
-// SIMT kernels: fp32, and head dims or modes without an MFMA backward
+template <int D>
+static BwdFns bwd_f32_fns() {
+  typedef F32BwdCfg<D> C;
+  return BwdFns{(const void*)attn_bwd_dq_f32_kernel<D>,
+                {(const void*)attn_bwd_dkv_f32_kernel<D, false>, (const void*)attn_bwd_dkv_f32_kernel<D, true>},
+                C::DQ_LDS,
+                C::DKV_LDS,
+                C::BQ,
+                C::KEYS};
+}
+
+static bool pick_bwd_f32(const fmlm_attn_params& p, BwdFns& f) {
+  if (p.ctx_block_table) return false;
+  switch (p.D) {
+    case 16: f = bwd_f32_fns<16>(); return true;
+    case 32: f = bwd_f32_fns<32>(); return true;
+    case 64: f = bwd_f32_fns<64>(); return true;
+    case 128: f = bwd_f32_fns<128>(); return true;
+    case 256: f = bwd_f32_fns<256>(); return true;
+    default: return false;
+  }
+}
+
+// SIMT kernels: head dims or modes without an MFMA backward
 template <typename T>
 static bool pick_bwd_simt(int D, BwdFns& f) {
   switch (D) {
@@ -1921,7 +2353,7 @@ static int check_bwd(const fmlm_attn_params& p, const fmlm_attn_grads& g, BwdFns
   } else if (p.dtype == FMLM_DTYPE_F16) {
     picked = mfma_ok ? pick_bwd<f16>(p.D, f) : pick_bwd_simt<f16>(p.D, f);
   } else if (p.dtype == FMLM_DTYPE_F32) {
-    picked = pick_bwd_simt<float>(p.D, f);
+    picked = pick_bwd_f32(p, f) || pick_bwd_simt<float>(p.D, f);
   } else {
     return FMLM_E_DTYPE;
   }

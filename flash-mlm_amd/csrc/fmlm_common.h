@@ -133,6 +133,24 @@ struct Mfma<f16> {
   }
 };
 
+// ---- MFMA 16x16x4 on fp32 operands and the fp32 kernels' fragments
+FMLM_DEV f32x4 mfma_f32(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+
+// E consecutive floats
+template <int E>
+struct FloatN {
+  typedef float type __attribute__((ext_vector_type(E)));
+};
+template <>
+struct FloatN<1> {
+  typedef float type;
+};
+template <int E>
+FMLM_DEV float elem_of(const typename FloatN<E>::type& x, int e) {
+  if constexpr (E == 1) return x;
+  else return x[e];
+}
+
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 #define FMLM_LDS __attribute__((address_space(3)))
 

@@ -61,3 +61,26 @@ def test_f32_forward_edges(D, H, lengths, ctx, causal, mla, device):
                                   v_cache=None if mla else _np(vc), cu_seqlens_kv=cu, total_context_len=cu[-1],
                                   context_batch_size=len(ctx))
     np.testing.assert_allclose(_np(unpack_from_kernel(out, meta, H)), ref, atol=TOL, rtol=TOL)
+
+
+@pytest.mark.parametrize("causal,mla", [(False, False), (True, False), (False, True)])
+@pytest.mark.parametrize("H,lengths,ctx", EDGES)
+@pytest.mark.parametrize("D", [16, 32, 64, 128, 256])
+def test_f32_backward_edges(D, H, lengths, ctx, causal, mla, device):
+    """Gradients within 2e-5 of the largest entry: dS = P (dP - delta) with P off by at most
+    16 * 8 * 6e-8 = 8e-6 of itself (above) and dP - delta by about as much of its range."""
+    q, k, v, kc, vc, cu, cache, meta = _case(device, D, H, lengths, ctx, D + H, mla, grad=True)
+    scale = D ** -0.5
+    out = flash_attn_mlm_compressed(q, k, v, H, meta, scale, cache, 0, is_mla=mla, block_n=64,
+                                    causal_query_seq_attn=causal)
+    dout = torch.randn(out.shape, generator=torch.Generator().manual_seed(1)).to(device)
+    leaves = [q, k, kc] if mla else [q, k, v, kc, vc]
+    got = torch.autograd.grad(out, leaves, dout)
+    ref = ar.mlm_attention_packed_backward(
+        _np(q), _np(k), _np(k if mla else v), _np(unpack_from_kernel(dout, meta, H)), lengths, scale, is_mla=mla,
+        causal_query_seq_attn=causal, k_cache=_np(kc), v_cache=None if mla else _np(vc), cu_seqlens_kv=cu,
+        total_context_len=cu[-1], context_batch_size=len(ctx))
+    ref = [ref[0], ref[1], ref[3]] if mla else ref
+    for name, g, r in zip(["q", "k", "kc"] if mla else ["q", "k", "v", "kc", "vc"], got, ref):
+        worst = np.abs(_np(g) - r).max() / np.abs(r).max()
+        assert worst <= 2e-5, (name, worst)
