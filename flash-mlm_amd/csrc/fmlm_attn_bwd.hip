@@ -320,6 +320,28 @@ struct UnitTables {
   int32_t* c;     // [n_ctx + 1]
 };
 
+// the tables as a record's resolution reads them: in global memory, written by an earlier
+// launch (read through ldc), or in LDS
+struct ConstTab {
+  const int32_t* a;
+  FMLM_DEV int operator[](int i) const { return ldc(a, i); }
+};
+template <typename Tab>
+struct UnitTabs {
+  Tab perm, q, k, c;
+};
+// the last entry s of the n + 1 non-decreasing entries of t with t[s] <= j, s < n
+template <typename Tab>
+FMLM_DEV int find_tab(const Tab& t, int n, int j) {
+  int lo = 0, hi = n - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (t[mid] <= j) lo = mid;
+    else hi = mid - 1;
+  }
+  return lo;
+}
+
 FMLM_DEV UnitTables unit_tables(const fmlm_attn_params& p, const fmlm_attn_grads& g) {
   UnitTables t;
   t.perm = (int32_t*)((char*)g.workspace + 2 * (int64_t)p.H * p.total_q * 4);
@@ -374,11 +396,9 @@ FMLM_DEV int dq_keys(const fmlm_attn_params& p, int b) {
 // grid runs in unit order, grid_unit) are the short ones.  More sequences keep their order.
 constexpr int kRankMax = 1024;
 
-__global__ __launch_bounds__(kScanThreads) void bwd_units_kernel(const fmlm_attn_params p, const fmlm_attn_grads g,
-                                                                 int bq, int bk, int n_ctx) {
-  __shared__ int32_t part[kScanThreads];
-  __shared__ int32_t s_keys[kRankMax], s_perm[kRankMax];
-  const UnitTables t = unit_tables(p, g);
+// s_perm: the sequences by rank (B <= kRankMax); q, k, c: the unit tables
+FMLM_DEV void scan_units(const fmlm_attn_params& p, int bq, int bk, int n_ctx, int32_t* s_keys, int32_t* s_perm,
+                         int32_t* q, int32_t* k, int32_t* c, int32_t* part) {
   const int tid = threadIdx.x;
   const bool ranked = p.B <= kRankMax;
   if (ranked) {
@@ -392,14 +412,22 @@ __global__ __launch_bounds__(kScanThreads) void bwd_units_kernel(const fmlm_attn
     }
     __syncthreads();
   }
-  for (int r = tid; r < p.B; r += kScanThreads) t.perm[r] = ranked ? s_perm[r] : r;
-  scan_tiles(p.B, bq, [&](int r) { return seq_info(p, ranked ? s_perm[r] : r).len; }, t.q, part);
-  scan_tiles(p.B, bk, [&](int b) { return seq_info(p, b).len; }, t.k, part);
+  scan_tiles(p.B, bq, [&](int r) { return seq_info(p, ranked ? s_perm[r] : r).len; }, q, part);
+  scan_tiles(p.B, bk, [&](int b) { return seq_info(p, b).len; }, k, part);
   scan_tiles(n_ctx, bk, [&](int cb) {
     int c0, c1;
     ctx_range(p, cb, c0, c1);
     return c1 - c0;
-  }, t.c, part);
+  }, c, part);
+}
+
+__global__ __launch_bounds__(kScanThreads) void bwd_units_kernel(const fmlm_attn_params p, const fmlm_attn_grads g,
+                                                                 int bq, int bk, int n_ctx) {
+  __shared__ int32_t part[kScanThreads];
+  __shared__ int32_t s_keys[kRankMax], s_perm[kRankMax];
+  const UnitTables t = unit_tables(p, g);
+  scan_units(p, bq, bk, n_ctx, s_keys, s_perm, t.q, t.k, t.c, part);
+  for (int r = threadIdx.x; r < p.B; r += kScanThreads) t.perm[r] = p.B <= kRankMax ? s_perm[r] : r;
 }
 
 // ---------------------------------------------------------------------------
@@ -477,16 +505,16 @@ FMLM_DEV SeqInfo rec_seq_info(const int* f) {
   return si;
 }
 
-FMLM_DEV void query_record(const fmlm_attn_params& p, const fmlm_attn_grads& g, int bq, int u, int32_t (&r)[kRecInts]) {
-  const UnitTables ut = unit_tables(p, g);
+template <typename Tab>
+FMLM_DEV void query_record(const fmlm_attn_params& p, const UnitTabs<Tab>& ut, int bq, int u, int32_t (&r)[kRecInts]) {
 #pragma unroll
   for (int i = 0; i < kRecInts; ++i) r[i] = 0;
   r[0] = -1;
-  if (u >= ldc(ut.q, p.B)) return;
-  const int rk = find_seq(ut.q, p.B, u);  // table entry: sequences by key count, largest first
-  const int b = ldc(ut.perm, rk);
+  if (u >= ut.q[p.B]) return;
+  const int rk = find_tab(ut.q, p.B, u);  // table entry: sequences by key count, largest first
+  const int b = ut.perm[rk];
   const SeqInfo si = seq_info(p, b);
-  const int qpos0 = (u - ldc(ut.q, rk)) * bq;
+  const int qpos0 = (u - ut.q[rk]) * bq;
   if (qpos0 >= si.len) return;
   const int cb = ctx_batch_of(p, b);
   int c0, c1;
@@ -511,19 +539,19 @@ FMLM_DEV bool seq_attends(const fmlm_attn_params& p, bool is_ctx, bool causal_ma
   return si.len > 0 && (!causal_main || si.mainlen > j0);  // causal: tokens < cu[b+1]
 }
 
-FMLM_DEV void key_record(const fmlm_attn_params& p, const fmlm_attn_grads& g, int n_ctx, int keys, bool causal,
+template <typename Tab>
+FMLM_DEV void key_record(const fmlm_attn_params& p, const UnitTabs<Tab>& ut, int n_ctx, int keys, bool causal,
                          int u, int32_t (&r)[kRecInts]) {
   const int32_t* cu = p.cu_seqlens_q;
-  const UnitTables ut = unit_tables(p, g);
 #pragma unroll
   for (int i = 0; i < kRecInts; ++i) r[i] = 0;
-  const int n_main = causal ? (min(ldc(cu, p.B), p.total_q) + keys - 1) / keys : ldc(ut.k, p.B);
-  const int n_cunits = n_ctx > 0 ? ldc(ut.c, n_ctx) : 0;
+  const int n_main = causal ? (min(ldc(cu, p.B), p.total_q) + keys - 1) / keys : ut.k[p.B];
+  const int n_cunits = n_ctx > 0 ? ut.c[n_ctx] : 0;
   int kind = 0, slot = 0, j0 = 0, n = 0, row0 = 0, b_lo = p.B, b_hi = p.B;
   if (u < n_cunits) {
     kind = 1;
-    slot = find_seq(ut.c, n_ctx, u);
-    j0 = (u - ldc(ut.c, slot)) * keys;
+    slot = find_tab(ut.c, n_ctx, u);
+    j0 = (u - ut.c[slot]) * keys;
     int c0, c1;
     ctx_range(p, slot, c0, c1);
     n = ctx_seg_keys(p, c0, c1);
@@ -541,8 +569,8 @@ FMLM_DEV void key_record(const fmlm_attn_params& p, const fmlm_attn_grads& g, in
       n = min(ldc(cu, p.B), p.total_q);
       b_lo = j0 < n ? find_seq(cu, p.B, j0) : p.B;
     } else {
-      slot = find_seq(ut.k, p.B, um);
-      j0 = (um - ldc(ut.k, slot)) * keys;
+      slot = find_tab(ut.k, p.B, um);
+      j0 = (um - ut.k[slot]) * keys;
       const SeqInfo si = seq_info(p, slot);
       n = si.len;
       row0 = si.q0;
@@ -570,24 +598,47 @@ FMLM_DEV void key_record(const fmlm_attn_params& p, const fmlm_attn_grads& g, in
   }
 }
 
-// one thread per unit of either grid
-__global__ __launch_bounds__(256) void bwd_records_kernel(const fmlm_attn_params p, const fmlm_attn_grads g, int bq,
-                                                          int bk, int n_ctx, int32_t* qrec, int nq, int32_t* krec,
-                                                          int nk) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
+// the records of unit i of both grids
+template <typename Tab>
+FMLM_DEV void write_records(const fmlm_attn_params& p, const UnitTabs<Tab>& ut, int bq, int bk, int n_ctx, int i,
+                            int32_t* qrec, int nq, int32_t* krec, int nk) {
   int32_t r[kRecInts];
   if (i < nq) {
-    query_record(p, g, bq, i, r);
+    query_record(p, ut, bq, i, r);
     int4* d = (int4*)(qrec + (int64_t)i * kRecInts);
 #pragma unroll
     for (int j = 0; j < kRecInts / 4; ++j) d[j] = make_int4(r[4 * j], r[4 * j + 1], r[4 * j + 2], r[4 * j + 3]);
   }
   if (i < nk) {
-    key_record(p, g, n_ctx, bk, (p.flags & FMLM_FLAG_CAUSAL_SEQ) != 0, i, r);
+    key_record(p, ut, n_ctx, bk, (p.flags & FMLM_FLAG_CAUSAL_SEQ) != 0, i, r);
     int4* d = (int4*)(krec + (int64_t)i * kRecInts);
 #pragma unroll
     for (int j = 0; j < kRecInts / 4; ++j) d[j] = make_int4(r[4 * j], r[4 * j + 1], r[4 * j + 2], r[4 * j + 3]);
   }
+}
+
+// one thread per unit of either grid
+__global__ __launch_bounds__(256) void bwd_records_kernel(const fmlm_attn_params p, const fmlm_attn_grads g, int bq,
+                                                          int bk, int n_ctx, int32_t* qrec, int nq, int32_t* krec,
+                                                          int nk) {
+  const UnitTables t = unit_tables(p, g);
+  const UnitTabs<ConstTab> ut{{t.perm}, {t.q}, {t.k}, {t.c}};
+  write_records(p, ut, bq, bk, n_ctx, blockIdx.x * 256 + threadIdx.x, qrec, nq, krec, nk);
+}
+
+// The unit tables (in LDS) and the records in one launch of one workgroup, for batches of
+// up to kRankMax sequences and context batches and kPlanUnits units: both kernels are
+// chains of dependent metadata loads (5 us each at any size), and a launch lies between.
+constexpr int kPlanUnits = 8 * kScanThreads;
+__global__ __launch_bounds__(kScanThreads) void bwd_plan_kernel(const fmlm_attn_params p, int bq, int bk, int n_ctx,
+                                                                int32_t* qrec, int nq, int32_t* krec, int nk) {
+  __shared__ int32_t part[kScanThreads];
+  __shared__ int32_t s_keys[kRankMax], s_perm[kRankMax];
+  __shared__ int32_t s_q[kRankMax + 1], s_k[kRankMax + 1], s_c[kRankMax + 1];
+  scan_units(p, bq, bk, n_ctx, s_keys, s_perm, s_q, s_k, s_c, part);
+  const UnitTabs<const int32_t*> ut{s_perm, s_q, s_k, s_c};
+  for (int i = threadIdx.x; i < max(nq, nk); i += kScanThreads)
+    write_records(p, ut, bq, bk, n_ctx, i, qrec, nq, krec, nk);
 }
 
 // unit u of key head kh (grid_unit) from its record (krec: nk records); false for a
@@ -655,6 +706,61 @@ struct QuerySteps {
 };
 
 // ---------------------------------------------------------------------------
+// Zero fill (fmlm_attn_bwd_fill): the gradient rows that no unit writes, by workgroups
+// appended to the dq kernel's grid, so that their stores run beside its last units' math
+// instead of in passes over whole gradients before it.  Fill unit f < B of head h zeroes
+// the padding rows [len, N) of sequence f of dq, dk and dv; fill unit B the rows of packed
+// tensors before the first and after the last sequence, and the context's outside its
+// batches.  Keys shared by all heads are left to the caller.
+// ---------------------------------------------------------------------------
+// rows [r0, r1) of elements of es bytes from base + off
+FMLM_DEV void zero_rows(void* base, int es, int64_t off, int64_t sn, int r0, int r1, int D) {
+  const int cpr = D * es / 16;  // 16-byte chunks per row
+  const int64_t n = (int64_t)max(r1 - r0, 0) * cpr;
+  char* const b = (char*)base + (off + (int64_t)r0 * sn) * es;
+  for (int64_t i = threadIdx.x; i < n; i += kBwdNW * 64) {
+    const int64_t r = i / cpr;
+    *(u32x4*)(b + r * sn * es + (i - r * cpr) * 16) = u32x4{0u, 0u, 0u, 0u};
+  }
+}
+
+__host__ __device__ inline int fill_units(const fmlm_attn_params& p) { return p.cu_seqlens_q ? p.B + 1 : 0; }
+
+FMLM_DEV void fill_unit(const fmlm_attn_params& p, const fmlm_attn_grads& g, int f, int h) {
+  const int es = p.dtype == FMLM_DTYPE_F32 ? 4 : 2;
+  const bool mla = p.flags & FMLM_FLAG_MLA;
+  if (f < p.B) {
+    const int len = seq_info(p, f).len;
+    if (p.q_layout == FMLM_LAYOUT_PADDED) zero_rows(g.dq, es, f * g.dq_sb + h * g.dq_sh, g.dq_sn, len, p.N, p.D);
+    if (p.kv_layout == FMLM_LAYOUT_PADDED && g.dk_sh) {
+      zero_rows(g.dk, es, f * g.dk_sb + h * g.dk_sh, g.dk_sn, len, p.N, p.D);
+      if (!mla) zero_rows(g.dv, es, f * g.dv_sb + h * g.dv_sh, g.dv_sn, len, p.N, p.D);
+    }
+    return;
+  }
+  const int c0 = min(max(ldc(p.cu_seqlens_q, 0), 0), p.total_q);
+  const int c1 = min(max(ldc(p.cu_seqlens_q, p.B), c0), p.total_q);
+  auto ends = [&](void* x, int64_t sh, int64_t sn, int lo, int hi, int rows) {
+    zero_rows(x, es, h * sh, sn, 0, min(lo, rows), p.D);
+    zero_rows(x, es, h * sh, sn, hi, rows, p.D);
+  };
+  if (p.q_layout == FMLM_LAYOUT_PACKED) ends(g.dq, g.dq_sh, g.dq_sn, c0, c1, (int)(g.dq_sh / max(g.dq_sn, (int64_t)1)));
+  if (p.kv_layout == FMLM_LAYOUT_PACKED && g.dk_sh) {
+    // causal main keys start at token 0
+    const int k0 = (p.flags & FMLM_FLAG_CAUSAL_SEQ) ? 0 : c0;
+    ends(g.dk, g.dk_sh, g.dk_sn, k0, c1, (int)(g.dk_sh / max(g.dk_sn, (int64_t)1)));
+    if (!mla) ends(g.dv, g.dv_sh, g.dv_sn, k0, c1, (int)(g.dv_sh / max(g.dv_sn, (int64_t)1)));
+  }
+  if (g.dk_ctx && p.cu_seqlens_kv && !p.ctx_block_table && (p.c_sh || h == 0)) {
+    const int n = max(p.ctx_batch, 1);
+    const int x0 = min(max(ldc(p.cu_seqlens_kv, 0), 0), p.ctx_rows);
+    const int x1 = min(max(ldc(p.cu_seqlens_kv, n), x0), p.ctx_rows);
+    ends(g.dk_ctx, p.c_sh, p.c_sn, x0, x1, p.ctx_rows);
+    if (!mla) ends(g.dv_ctx, p.c_sh, p.c_sn, x0, x1, p.ctx_rows);
+  }
+}
+
+// ---------------------------------------------------------------------------
 // dq kernel: grid (query-tile units, H), kBwdNW waves, QB blocks of 16 rows per wave.
 // LSE: the forward stored each row's log2-sum-exp (p.lse), so P = 2^(z - lse) needs no
 // running max, no row sum and no rescale.
@@ -662,7 +768,7 @@ struct QuerySteps {
 template <typename T, int D, bool LSE>
 __global__ __launch_bounds__(kBwdNW * 64, BwdCfg<D>::WPS) void attn_bwd_dq_kernel(const fmlm_attn_params p,
                                                                      const fmlm_attn_grads g,
-                                                                     const int32_t* qrec, int nq) {
+                                                                     const int32_t* qrec, int nq, int nfill) {
   typedef BwdCfg<D> C;
   typedef typename Mfma<T>::v8 v8;
   constexpr int QB = C::QB;
@@ -670,7 +776,10 @@ __global__ __launch_bounds__(kBwdNW * 64, BwdCfg<D>::WPS) void attn_bwd_dq_kerne
 
   int u, h;
   grid_unit((unsigned)p.H, u, h);
-  if (u >= nq) return;
+  if (u >= nq) {
+    if (u - nq < nfill) fill_unit(p, g, u - nq, h);
+    return;
+  }
   int rec[9];  // the unit's record (query_record)
   load_record(qrec + (int64_t)u * kRecInts, rec);
   const int b = rec[0];
@@ -1605,7 +1714,7 @@ FMLM_DEV float row_sum(float x) {
 
 template <typename T, int D>
 __global__ __launch_bounds__(256) void attn_bwd_dq_simt_kernel(const fmlm_attn_params p, const fmlm_attn_grads g,
-                                                               const int32_t* qrec, int nq) {
+                                                               const int32_t* qrec, int nq, int nfill) {
   typedef SimtBwdCfg<D> C;
   extern __shared__ __align__(16) char smem_raw[];
   float* const Kf = (float*)smem_raw;
@@ -1613,7 +1722,10 @@ __global__ __launch_bounds__(256) void attn_bwd_dq_simt_kernel(const fmlm_attn_p
 
   int u, h;
   grid_unit((unsigned)p.H, u, h);
-  if (u >= nq) return;
+  if (u >= nq) {
+    if (u - nq < nfill) fill_unit(p, g, u - nq, h);
+    return;
+  }
   int rec[9];  // the unit's record (query_record)
   load_record(qrec + (int64_t)u * kRecInts, rec);
   const int b = rec[0];
@@ -1905,7 +2017,8 @@ FMLM_DEV void store_cols(const f32x4 (&o)[F32BwdCfg<D>::NG][F32BwdCfg<D>::E], fl
 template <int D>
 __global__ __launch_bounds__(256, F32BwdCfg<D>::WPS) void attn_bwd_dq_f32_kernel(const fmlm_attn_params p,
                                                                                  const fmlm_attn_grads g_,
-                                                                                 const int32_t* qrec, int nq) {
+                                                                                 const int32_t* qrec, int nq,
+                                                                                 int nfill) {
   typedef F32BwdCfg<D> C;
   typedef typename FloatN<C::E>::type vE;
   constexpr int QB = C::QB, BK = 64;
@@ -1917,7 +2030,10 @@ __global__ __launch_bounds__(256, F32BwdCfg<D>::WPS) void attn_bwd_dq_f32_kernel
 
   int u, h;
   grid_unit((unsigned)p.H, u, h);
-  if (u >= nq) return;
+  if (u >= nq) {
+    if (u - nq < nfill) fill_unit(p, g_, u - nq, h);
+    return;
+  }
   int rec[9];  // the unit's record (query_record)
   load_record(qrec + (int64_t)u * kRecInts, rec);
   const int b = rec[0];
@@ -2437,7 +2553,7 @@ extern "C" int64_t fmlm_attn_bwd_workspace_bytes(const fmlm_attn_params* p) {
   return bwd_layout(*p, kMinUnitRows, kMinUnitRows, n_ctx).bytes;
 }
 
-extern "C" int fmlm_attn_bwd(const fmlm_attn_params* pp, const fmlm_attn_grads* gp, void* stream) {
+static int attn_bwd(const fmlm_attn_params* pp, const fmlm_attn_grads* gp, bool fill, void* stream) {
   if (!pp || !gp) return FMLM_E_ARG;
   const fmlm_attn_params& p = *pp;
   const fmlm_attn_grads& g = *gp;
@@ -2453,8 +2569,10 @@ extern "C" int fmlm_attn_bwd(const fmlm_attn_params* pp, const fmlm_attn_grads* 
   const BwdLayout l = bwd_layout(p, f.bq, f.dkv_keys, n_ctx);
   if (!g.workspace || g.workspace_bytes < fmlm_attn_bwd_workspace_bytes(pp) || g.workspace_bytes < l.bytes)
     return FMLM_E_WORKSPACE;
+  int nfill = fill ? fill_units(p) : 0;
   dim3 qgrid, kgrid;
-  if (!unit_grid(l.qunits, (unsigned)p.H, qgrid) || !unit_grid(l.kunits, dkv_heads(p, n_ctx), kgrid)) return FMLM_E_ARG;
+  if (!unit_grid(l.qunits + nfill, (unsigned)p.H, qgrid) || !unit_grid(l.kunits, dkv_heads(p, n_ctx), kgrid))
+    return FMLM_E_ARG;
   hipStream_t s = (hipStream_t)stream;
   fmlm_attn_params pc = p;
   fmlm_attn_grads gc = g;
@@ -2463,16 +2581,21 @@ extern "C" int fmlm_attn_bwd(const fmlm_attn_params* pp, const fmlm_attn_grads* 
   int nq = (int)l.qunits, nk = (int)l.kunits;
 
   // 0. unit tables, then the records of both grids' units
-  hipLaunchKernelGGL(bwd_units_kernel, dim3(1), dim3(kScanThreads), 0, s, p, g, f.bq, f.dkv_keys, n_ctx);
-  if ((rc = launch_status())) return rc;
   const int64_t nrec = std::max(l.qunits, l.kunits);
-  hipLaunchKernelGGL(bwd_records_kernel, dim3((unsigned)((nrec + 255) / 256)), dim3(256), 0, s, p, g, f.bq, f.dkv_keys,
-                     n_ctx, qrec, nq, krec, nk);
+  if (p.B <= kRankMax && n_ctx <= kRankMax && nrec <= kPlanUnits) {
+    hipLaunchKernelGGL(bwd_plan_kernel, dim3(1), dim3(kScanThreads), 0, s, p, f.bq, f.dkv_keys, n_ctx, qrec, nq, krec,
+                       nk);
+  } else {
+    hipLaunchKernelGGL(bwd_units_kernel, dim3(1), dim3(kScanThreads), 0, s, p, g, f.bq, f.dkv_keys, n_ctx);
+    if ((rc = launch_status())) return rc;
+    hipLaunchKernelGGL(bwd_records_kernel, dim3((unsigned)((nrec + 255) / 256)), dim3(256), 0, s, p, g, f.bq,
+                       f.dkv_keys, n_ctx, qrec, nq, krec, nk);
+  }
   if ((rc = launch_status())) return rc;
   // 1. dq (+ the row statistics: delta, and the log2-sum-exp unless the forward stored it)
   const void* const dq_fn = p.lse && f.dq_lse ? f.dq_lse : f.dq;
   if ((rc = raise_lds(dq_fn, f.dq_lds))) return rc;
-  void* args[] = {(void*)&pc, (void*)&gc, (void*)&qrec, (void*)&nq};
+  void* args[] = {(void*)&pc, (void*)&gc, (void*)&qrec, (void*)&nq, (void*)&nfill};
   hipError_t e = hipLaunchKernel(dq_fn, qgrid, dim3(kBwdNW * 64), args, (size_t)f.dq_lds, s);
   if (e != hipSuccess) return (int)e;
   // 2. dK / dV, context keys then main keys in one launch
@@ -2481,4 +2604,12 @@ extern "C" int fmlm_attn_bwd(const fmlm_attn_params* pp, const fmlm_attn_grads* 
   e = hipLaunchKernel(f.dkv[causal ? 1 : 0], kgrid, dim3(kBwdNW * 64), kargs, (size_t)f.dkv_lds, s);
   if (e != hipSuccess) return (int)e;
   return launch_status();
+}
+
+extern "C" int fmlm_attn_bwd(const fmlm_attn_params* pp, const fmlm_attn_grads* gp, void* stream) {
+  return attn_bwd(pp, gp, false, stream);
+}
+
+extern "C" int fmlm_attn_bwd_fill(const fmlm_attn_params* pp, const fmlm_attn_grads* gp, void* stream) {
+  return attn_bwd(pp, gp, true, stream);
 }

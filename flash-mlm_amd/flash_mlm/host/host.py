@@ -295,10 +295,10 @@ def _attention_backward(plan: AttnLaunch, out: torch.Tensor, dout: torch.Tensor,
     """Gradients (dq, dk, dv, dk_cache, dv_cache) of the prepared call ``plan`` whose
     output is ``out``, shaped like the caller's tensors (dv None for MLA: V is K and both
     gradients are in dk)."""
-    g, (dq, dk, dv, dkc, dvc, _ws, _dout) = _backward_args(plan, out, dout, want_ctx)
+    g, (dq, dk, dv, dkc, dvc, _ws, _dout) = _backward_args(plan, out, dout, want_ctx, zeroed=False)
     with _device_scope(out.device):
-        rc = plan.lib.fmlm_attn_bwd(plan.params, g, plan.stream)
-    _lib.check(rc, "fmlm_attn_bwd")
+        rc = plan.lib.fmlm_attn_bwd_fill(plan.params, g, plan.stream)
+    _lib.check(rc, "fmlm_attn_bwd_fill")
     if plan.unpack_kv is not None:
         mla = bool(plan.params.flags & _lib.FLAG_MLA)
         dk = _unpack_kv_grad(plan.lib, dk, plan, mla)
@@ -309,9 +309,11 @@ def _attention_backward(plan: AttnLaunch, out: torch.Tensor, dout: torch.Tensor,
     return dq, dk, dv, dkc, dvc
 
 
-def _backward_args(plan: AttnLaunch, out: torch.Tensor, dout: torch.Tensor, want_ctx: bool):
-    """The fmlm_attn_grads block of one backward call and the tensors it points to:
-    zeroed gradients shaped like the tensors the kernel read, the workspace and dout."""
+def _backward_args(plan: AttnLaunch, out: torch.Tensor, dout: torch.Tensor, want_ctx: bool, zeroed: bool = True):
+    """The fmlm_attn_grads block of one backward call and the tensors it points to: gradients
+    shaped like the tensors the kernel read, the workspace and dout.  ``zeroed``: the
+    gradients start as zeros (for fmlm_attn_bwd), else only those of which
+    fmlm_attn_bwd_fill does not reach every row."""
     p, lib = plan.params, plan.lib
     q_, _, k_, v_, k_ctx, v_ctx = plan.keep[:6]
     mla = bool(p.flags & _lib.FLAG_MLA)
@@ -321,7 +323,9 @@ def _backward_args(plan: AttnLaunch, out: torch.Tensor, dout: torch.Tensor, want
         raise ValueError("gradient of the attention output has the wrong shape")
 
     def grad_of(x: torch.Tensor, strides):
-        gx = torch.zeros(x.shape, dtype=x.dtype, device=x.device)
+        # a head stride of 0 (rows shared by all heads): the kernel fills the shared rows only
+        make = torch.zeros if zeroed or strides[1] == 0 else torch.empty
+        gx = make(x.shape, dtype=x.dtype, device=x.device)
         if x.ndim == 4:  # padded [B, H, N, D]; head stride 0 = rows shared by all heads
             return gx, (gx.stride(0), 0 if strides[1] == 0 else gx.stride(1), gx.stride(2))
         return gx, strides  # packed rows of a contiguous tensor
@@ -341,10 +345,11 @@ def _backward_args(plan: AttnLaunch, out: torch.Tensor, dout: torch.Tensor, want
         # a paged context's gradient is accumulated in float32 (a page can serve several
         # context batches); _attention_backward rounds it to the cache dtype
         acc = torch.float32 if p.ctx_block_table else k_ctx.dtype
-        dkc = torch.zeros(k_ctx.shape, dtype=acc, device=k_ctx.device)
+        make = torch.zeros if zeroed or p.ctx_block_table else torch.empty
+        dkc = make(k_ctx.shape, dtype=acc, device=k_ctx.device)
         g.dk_ctx = dkc.data_ptr()
         if not mla:
-            dvc = torch.zeros(v_ctx.shape, dtype=acc, device=v_ctx.device)
+            dvc = make(v_ctx.shape, dtype=acc, device=v_ctx.device)
             g.dv_ctx = dvc.data_ptr()
     nbytes = int(lib.fmlm_attn_bwd_workspace_bytes(p))
     _lib.check(nbytes if nbytes < 0 else 0, "fmlm_attn_bwd_workspace_bytes")

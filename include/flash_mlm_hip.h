@@ -328,6 +328,13 @@ typedef struct fmlm_attn_grads {
 FMLM_API int fmlm_attn_grads_size(void);  /* sizeof(fmlm_attn_grads), for bindings */
 FMLM_API int64_t fmlm_attn_bwd_workspace_bytes(const fmlm_attn_params* p);
 FMLM_API int fmlm_attn_bwd(const fmlm_attn_params* p, const fmlm_attn_grads* g, void* stream);
+/* The same for gradients that were not zeroed: the rows that fmlm_attn_bwd does not write
+ * become zero too, namely the padding rows [L_b, N) of padded q / k / v gradients, the rows
+ * of packed ones (and of a packed context's) before the first and after the last sequence
+ * (context batch).  Rows per head of a packed gradient: its head stride / row stride.
+ * Gradients of keys shared by all heads (head stride 0) and of paged contexts still have to
+ * be zeroed by the caller. */
+FMLM_API int fmlm_attn_bwd_fill(const fmlm_attn_params* p, const fmlm_attn_grads* g, void* stream);
 
 #ifdef __cplusplus
 }

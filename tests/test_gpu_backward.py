@@ -560,3 +560,47 @@ def test_backward_dense_repeated_call(with_context, device):
 
     for first, again in zip(grads(), grads()):
         assert torch.equal(first, again)
+
+
+@pytest.mark.parametrize("case", ["padded", "causal", "precompressed", "mla", "dense"])
+@pytest.mark.parametrize("dtype,D", [(torch.float16, 64), (torch.float32, 64), (torch.bfloat16, 16)])
+def test_backward_fill_writes_every_row(case, dtype, D, device):
+    """fmlm_attn_bwd_fill over gradients full of NaN gives what fmlm_attn_bwd gives over
+    zeros, on the MFMA, the fp32 and the SIMT kernels: padding rows, empty sequences (at
+    either end too), packed rows past the last sequence and spare context rows."""
+    import ctypes
+
+    from flash_mlm import _lib
+    from flash_mlm.host import host as hh
+
+    gen = torch.Generator().manual_seed(41)
+    lengths, ctx_lens, H, N = [0, 70, 0, 5, 0], [3, 0, 80, 17, 2], 3, 80
+    B, mla = len(lengths), case == "mla"
+    cache, kc, _, cu, _ = _packed_cache(ctx_lens, H=H, D=D, mla=mla, dtype=dtype, device=device, gen=gen)
+    q, k, v = (_leaf((B, H, N, D), dtype, device, gen).detach() for _ in range(3))
+    meta = build_pack_metadata(torch.tensor(lengths, dtype=torch.int32, device=device), N, 64)
+    if case == "dense":
+        out, plan = hh._dense_impl(q, k, v, 0.125, None, None, False, None, False)
+    elif case == "precompressed":
+        T = meta.total_tokens + 9
+        qp, kp, vp = (_leaf((H * T, D), dtype, device, gen).detach() for _ in range(3))
+        out, plan = hh._precompressed_impl(qp, kp, vp, H, T, meta.cu_seqlens, meta.batch_ids_q, meta.q_tile_starts_q,
+                                           0.125, cache, 0, False, None, False, False, None)
+        out[:] = out.nan_to_num()  # its padding rows are not written
+    else:
+        out, plan = hh._compressed_impl(q, k, v, H, meta, 0.125, cache, 0, mla, None, 64, 64, False, False,
+                                        case == "causal", owned_buffers=True)
+    dout = torch.randn(out.shape, generator=gen).to(dtype).to(device)
+    results = []
+    for fill in (False, True):
+        g, keep = hh._backward_args(plan, out, dout, True)
+        grads = [t for t in keep[:5] if t is not None]
+        if fill:
+            for t in grads:
+                if not (mla and t is keep[1]):  # rows shared by all heads are left to the caller
+                    t.fill_(float("nan"))
+        fn = plan.lib.fmlm_attn_bwd_fill if fill else plan.lib.fmlm_attn_bwd
+        _lib.check(fn(ctypes.byref(plan.params), ctypes.byref(g), plan.stream), "backward")
+        results.append(grads)
+    for zeroed, filled in zip(*results):
+        assert torch.equal(zeroed, filled)
