@@ -228,7 +228,9 @@ def dtype_code(dtype: torch.dtype) -> int:
 
 
 def stream_of(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    # the raw handle: building a torch.cuda.Stream object took 2 us of a 12 us call
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def ptr(t: torch.Tensor | None) -> int | None:

@@ -142,22 +142,22 @@ def _launch(*, run: bool = True, **kw) -> AttnLaunch:
 
 # ---------------------------------------------------------------------------
 # Launch memo.  A call that matches an earlier one in everything its checks and its
-# parameter block depend on (the q/k/v pointers, shapes, strides, dtype and device, the
-# arguments, the cached layer entry, the tile configuration) reuses that call's parameter
-# block: it allocates the output, re-packs K/V where the call packs them, and launches,
-# skipping the Python-side validation and the ~45 field writes of the block.  The cache
-# replaces a layer's entry on prefill and append, never mutating it, so the entry object
-# stands for its contents; the memo refers to it (and to the cache) weakly and holds no
-# input tensor, only the small index tensors the call derived (int32 offsets, an empty
-# context's zero offsets).  Compressed calls keep their memo on the PackMetadata, dense
-# calls in a module-level table.
+# parameter block depend on (the q/k/v shapes, strides, dtype, device and 16-byte
+# alignment, the arguments, the cached layer entry, the tile configuration) reuses that
+# call's parameter block with its own tensors' addresses: it allocates the output, re-packs
+# K/V where the call packs them, and launches, skipping the Python-side validation and the
+# ~45 field writes of the block.  The cache replaces a layer's entry on prefill and append,
+# never mutating it, so the entry object stands for its contents; the memo refers to it
+# (and to the cache) weakly and holds no input tensor, only the small index tensors the
+# call derived (int32 offsets, an empty context's zero offsets).  Compressed calls keep
+# their memo on the PackMetadata, dense calls in a module-level table.
 # ---------------------------------------------------------------------------
 _MEMO_MAX = 16
 _DENSE_MEMO: dict = {}
 
 
 def _tkey(t: torch.Tensor):
-    return (t.data_ptr(), t.shape, t.stride(), t.dtype, t.get_device())
+    return (t.data_ptr() % 16 == 0, t.shape, t.stride(), t.dtype, t.get_device())
 
 
 class _Memo:
@@ -192,22 +192,22 @@ def _memo_store(memo: dict, key, m: _Memo) -> None:
 
 
 def _memo_run(m: _Memo, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, entry):
-    """Run a memoised call on this call's q/k/v (the same tensors, by the memo key)."""
+    """Run a memoised call on this call's q/k/v (laid out alike, by the memo key)."""
     out = torch.empty(m.out_shape, dtype=q.dtype, device=q.device)
     p = _lib.AttnParams.from_buffer_copy(m.params)
-    p.o = out.data_ptr()
+    p.q, p.o = q.data_ptr(), out.data_ptr()
     # the first six as _prepare keeps them: the backward reads them (q, out, k, v, context)
     kc, vc = (entry.k_cache, entry.v_cache) if entry is not None and p.k_ctx else (None, None)
-    keep = [q, out, k, v, kc, vc, m.extra]
-    if entry is not None:
-        keep.append((entry.cu_seqlens_kv, entry.block_table))
     if m.repack is not None:
         packed = m.repack(k, v)
         if packed is None:
             return None
-        k_pk, v_pk = packed
-        p.k, p.v = k_pk.data_ptr(), v_pk.data_ptr()
-        keep.append(packed)
+        k, v = packed
+    mla = p.flags & _lib.FLAG_MLA
+    p.k, p.v = k.data_ptr(), (k if mla else v).data_ptr()
+    keep = [q, out, k, None if mla else v, kc, vc, m.extra]
+    if entry is not None:
+        keep.append((entry.cu_seqlens_kv, entry.block_table))
     plan = AttnLaunch(_lib.load(), p, _lib.stream_of(q.device), q.device, tuple(keep))
     plan.unpack_kv, plan.records = m.unpack_kv, m.records
     plan()
@@ -234,7 +234,11 @@ def _cache_tensors(inference_cache, layer_id, prefill: bool):
 
 
 def _wants_grad(*tensors) -> bool:
-    return torch.is_grad_enabled() and any(isinstance(t, torch.Tensor) and t.requires_grad for t in tensors)
+    if torch.is_grad_enabled():
+        for t in tensors:
+            if isinstance(t, torch.Tensor) and t.requires_grad:
+                return True
+    return False
 
 
 def _backward_unsupported(q: torch.Tensor, d: int, entry, is_mla: bool) -> str | None:
@@ -728,13 +732,14 @@ def _compressed_impl(
 ):
     """Body of :func:`flash_attn_mlm_compressed`; returns (out, prepared launch or None)."""
     memo = memo_key = entry = None
-    if (run and not prefill and not owned_buffers and context_index is None and isinstance(q_meta, PackMetadata)
+    if (run and not prefill and context_index is None and isinstance(q_meta, PackMetadata)
             and isinstance(q, torch.Tensor)):
         memo = q_meta.launch_memo
         entry = _entry_of(inference_cache, layer_id)
         memo_key = (_tkey(q), _tkey(k), _tkey(v), num_heads, float(scale), is_mla, context_batch_size, block_m,
                     block_n, auto_tune_tiles, causal_query_seq_attn, _TILE_CONFIG,
-                    None if entry is None else id(entry), inference_cache is None)
+                    None if entry is None else id(entry), inference_cache is None,
+                    owned_buffers and causal_query_seq_attn)
         m = _memo_lookup(memo, memo_key, entry)
         if m is not None:
             res = _memo_run(m, q, k, v, entry)
@@ -911,7 +916,7 @@ def _compressed_impl(
             and plan.keep[10] is None and (causal_query_seq_attn or (k_ is k and v_ is v))):
         repack = None
         if causal_query_seq_attn:
-            repack = _causal_repack(inference_cache, is_mla=is_mla, num_heads=num_heads, b=b, n=n, d=d, T=T,
+            repack = _causal_repack(None if owned_buffers else inference_cache, is_mla=is_mla, num_heads=num_heads, b=b, n=n, d=d, T=T,
                                     cu_q=cu_q)
         # the offsets the launch reads when they are not the metadata's or the entry's own
         extra = (cu_q, cu_kv, k_cache if entry is None else None, v_cache if entry is None else None)

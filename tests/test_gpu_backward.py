@@ -604,3 +604,40 @@ def test_backward_fill_writes_every_row(case, dtype, D, device):
         results.append(grads)
     for zeroed, filled in zip(*results):
         assert torch.equal(zeroed, filled)
+
+
+@pytest.mark.parametrize("grad", [False, True])
+@pytest.mark.parametrize("way", ["dense", "packed", "causal", "mla"])
+def test_repeated_layout_reads_the_new_tensors(way, grad, device):
+    """A call laid out like an earlier one reuses its parameter block, but reads its own
+    tensors: outputs and gradients equal those of the same inputs called first."""
+    B, H, N, D = 2, 3, 40, 64
+    gen = torch.Generator().manual_seed(77)
+    sets = [[_leaf((B, H, N, D), torch.float16, device, gen).requires_grad_(grad) for _ in range(3)] for _ in range(2)]
+    dout_gen = torch.Generator().manual_seed(5)
+
+    def run(meta, q, k, v):
+        if way == "dense":
+            out = flash_attn_mlm(q, k, v, 0.125)
+        else:
+            out = flash_attn_mlm_compressed(q, k, v, H, meta, 0.125, is_mla=way == "mla", block_n=64,
+                                            causal_query_seq_attn=way == "causal")
+        if not grad:
+            return [out]
+        dout = torch.randn(out.shape, generator=dout_gen.manual_seed(5)).half().to(device)
+        leaves = [q, k] if way == "mla" else [q, k, v]
+        return [out.detach(), *torch.autograd.grad(out, leaves, dout)]
+
+    def meta():
+        return build_pack_metadata(torch.tensor([N, 13], dtype=torch.int32, device=device), N, 64)
+
+    fresh = [run(meta(), *s) for s in sets]  # dense calls keep their block between metadata too
+    shared = meta()
+    again = [run(shared, *s) for s in (sets[0], sets[1], sets[0])]
+    for got, want in zip(again, (fresh[0], fresh[1], fresh[0])):
+        for a, b in zip(got, want):
+            assert torch.equal(a, b)
+    assert not torch.equal(fresh[0][0], fresh[1][0])
+    if way == "dense" and not grad:  # the second set's first call already ran from the first's block
+        ref = ar.mlm_attention_dense(*(_np(t) for t in sets[1]), 0.125)
+        np.testing.assert_allclose(_np(fresh[1][0]), ref, atol=1e-2, rtol=1e-2)
