@@ -145,14 +145,13 @@ __global__ __launch_bounds__(kSchedThreads) void schedule_kernel(const fmlm_attn
         float kmax = 0.f;
         for (int b = 0; b < B; ++b) kmax = fmaxf(kmax, s_tiles[b] > 0 ? s_work[b] : 0.f);
         const float chunk = fmaxf((float)kMinHpackTiles, ceilf(kmax / (tid + 1)));
-        float parts = 0.f, recs = 0.f;
+        float parts = 0.f;
         for (int b = 0; b < B; ++b) {
           const float S = fminf(kMaxSplits, fmaxf(1.f, ceilf(s_work[b] / chunk)));
           parts += s_tiles[b] * S;
-          if (S > 1.f) recs += s_tiles[b] * S;
         }
         float cost = ceilf(parts / slots) * (chunk + kHpackPartCost);
-        if (recs > (float)rec_cap || tid >= kMaxSplits) cost = INFINITY;
+        if (parts > (float)rec_cap || tid >= kMaxSplits) cost = INFINITY;  // a record per part
         float best = cost;
 #pragma unroll
         for (int off = 1; off < 64; off <<= 1) best = fminf(best, __shfl_xor(best, off));
@@ -221,6 +220,63 @@ __global__ __launch_bounds__(kSchedThreads) void schedule_kernel(const fmlm_attn
     const long long i = num <= 0 ? 0 : (num + 8 * k - 1) / (8 * k);
     return (int)min(i, (long long)s_tiles[s_order[r]]);
   };
+  if (by_seq && s_chunk > 0) {
+    int n = 0;  // parts of XCD x by that placement
+    for (int r = lane; r < B; r += 64) n += (first_tile(r, x + 1) - first_tile(r, x)) * s_split[s_order[r]];
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) n += __shfl_xor(n, off);
+    if (lane == 0) s_len[x] = n;
+    __syncthreads();
+    int all = 0, most = 0;
+    for (int i = 0; i < kXcds; ++i) {
+      all += s_len[i];
+      most = max(most, s_len[i]);
+    }
+    __syncthreads();
+    const int per_round = max(slots / kXcds, 1);
+    if (most > (all + slots - 1) / max(slots, 1) * per_round || most > 2 * ((all + kXcds - 1) / kXcds)) {
+      // An XCD has more parts than CUs for the round(s) that all parts take (40 for 32: 16
+      // sequences of 8 tokens, 64 heads, 2000-6000 latent rows took 152 us, so 103), or over
+      // twice its share (one sequence: 31 us on one XCD, 28 on all): the parts in rank order,
+      // those of a tile together, are cut into kXcds runs of equal count instead.  s_pre:
+      // parts before each rank.
+      if (tid == 0) {
+        long long acc = 0;
+        for (int r = 0; r < B; ++r) {
+          s_pre[r] = acc;
+          acc += (long long)s_tiles[s_order[r]] * s_split[s_order[r]];
+        }
+        s_pre[B] = acc;
+      }
+      __syncthreads();
+      const int n = (int)s_pre[B];
+      auto start = [&](int xx) { return (int)(((long long)xx * n + kXcds - 1) / kXcds); };
+      for (int r = tid; r < B; r += kSchedThreads) {  // a rank's groups; part i's record is record i
+        const int b = s_order[r], S = s_split[b], tiles = s_tiles[b];
+        const int gid0 = S > 1 ? atomicAdd(&s_groups, tiles) : 0, rec0 = (int)s_pre[r];
+        for (int j = 0; S > 1 && j < tiles; ++j) groups[gid0 + j] = make_int4(b, j << 16, rec0 + j * S, S);
+        for (int i = 0; i < tiles * S; ++i) {
+          const int j = i / S, sp = i - j * S, pos = rec0 + i;
+          const int xx = min((int)((long long)pos * kXcds / max(n, 1)), kXcds - 1);
+          const int qpos = pos - start(xx);
+          if (qpos >= 0 && qpos < cap_q)
+            units[(int64_t)xx * cap_q + qpos] =
+                make_int4(b, j << 16, rec0 + j * S, S > 1 ? (gid0 + j) | (sp << 20) | ((S - 1) << 25) : -1);
+        }
+      }
+      __syncthreads();
+      if (tid < kXcds) header[kHdrQueueLen + tid] = min(start(tid + 1) - start(tid), cap_q);
+      if (tid == 0) {
+        header[kHdrUnits] = n;
+        header[kHdrGroups] = s_groups;
+        header[kHdrGroupsOff] = groups_off;
+        header[kHdrRecordsOff] = records_off;
+        header[kHdrRecBytes] = rec_bytes;
+        header[kHdrCap] = cap_q;
+      }
+      return;
+    }
+  }
   const int K = kXcds / min(H & -H, kXcds);
   const int PX = H * K / kXcds;
   const int nrank = (B + K - 1) / K;
@@ -1587,12 +1643,20 @@ struct MlaRowsCfg {
   static constexpr int LDS_BYTES = 2 * TILEB;
 };
 
-template <typename T, bool PAGED, bool LSE, bool SPLIT>
+// SPLIT: the launch may split key ranges over workgroups.  KH (key halves, 2 only with
+// SPLIT): a tile of 64 query rows, waves 0-3 taking keys 0-31 of every latent tile and waves
+// 4-7 keys 32-63, for calls of few rows (see mla_rows_launch): with 128 rows per tile a
+// sequence of 64 (head, position) rows leaves one working wave per SIMD, bound by the
+// latency of its own LDS reads.  The halves' sums are added through LDS at the end.
+template <typename T, bool PAGED, bool LSE, bool SPLIT, int KH>
 __global__ __launch_bounds__(MlaRowsCfg::NT, 1) void attn_mla_rows_kernel(
     const fmlm_attn_params p, const int4* __restrict__ units, const int32_t* __restrict__ hdr, const SplitArgs spa) {
   typedef MlaRowsCfg C;
   typedef typename Mfma<T>::v8 v8;
   constexpr int D = C::D, BK = C::BK;
+  constexpr int BQ = C::BQ / KH;        // query rows per workgroup
+  constexpr int ROWW = C::NW / KH;      // waves side by side over the rows
+  static_assert(KH == 1 || SPLIT, "key halves only in launches that may split");
   extern __shared__ __align__(16) char smem_raw[];
 
   // packed calls use head-packed tiles: 128 consecutive rows of the sequence's H*len
@@ -1604,15 +1668,16 @@ __global__ __launch_bounds__(MlaRowsCfg::NT, 1) void attn_mla_rows_kernel(
   // other kernels
   const int u = !hpack ? (int)blockIdx.x : SPLIT ? workgroup_unit(hdr) : queue_first(hdr, blockIdx.x);
   WorkItem w;
-  if (u < 0 || !resolve_work(p, units, u, C::BQ, w, SPLIT ? spa : SplitArgs{nullptr, 0, 1}, hpack)) return;
+  if (u < 0 || !resolve_work(p, units, u, BQ, w, SPLIT ? spa : SplitArgs{nullptr, 0, 1}, hpack)) return;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15;
   const int g = lane >> 4;
-  const int row = wave * 16 + l16;  // the query row of this lane's S^T / O^T column
-  const bool wave_active = wave * 16 < w.qcount;
+  const int rw = KH == 1 ? wave : wave % ROWW, kh = KH == 1 ? 0 : wave / ROWW;
+  const int row = rw * 16 + l16;  // the query row of this lane's S^T / O^T column
+  const bool wave_active = rw * 16 < w.qcount;
   // element offsets of this lane's q and o rows
   int64_t q_off, o_off;
   {
@@ -1791,6 +1856,73 @@ __global__ __launch_bounds__(MlaRowsCfg::NT, 1) void attn_mla_rows_kernel(
             }
         }
       };
+      if constexpr (KH == 2) {
+        // this wave's 32 keys of the tile: S of the two key blocks, softmax, P V
+        const int nk = (t < nt0 ? min(BK, w.seg[0].n - t * BK) : min(BK, w.seg[1].n - (t - nt0) * BK)) - 32 * kh;
+        if (nk > 0) {
+          const uint32_t kt = lds_addr(tile) + kk + kh * 32 * C::ROWB, vt = lds_addr(tile) + vv + kh * 32 * C::ROWB;
+          constexpr int HL = 5;  // fragment reads in flight
+          auto fread2 = [&](int f) -> v8 {
+            if (f < 32) {
+              const int kc = f >> 1;
+              return *(const FMLM_LDS v8*)(uintptr_t)((kt ^ (64 * (kc & 3))) + (f & 1) * 16 * C::ROWB + 256 * (kc >> 2));
+            }
+            const int db = f - 32;
+            const uint32_t a = (vt ^ (32 * (db & 7))) + 256 * (db >> 3);
+            const s16x4 lo = lds_read_tr16_at(a);
+            const s16x4 hi = lds_read_tr16_at(a + 16 * C::ROWB);
+            return __builtin_bit_cast(v8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+          };
+          f32x4 s2[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+          u32x4 pk;
+          v8 fr[HL + 1];
+#pragma unroll
+          for (int r = 0; r < HL; ++r) fr[r] = fread2(r);
+          __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+          for (int f = 0; f < 32; ++f) {
+            fr[(f + HL) % (HL + 1)] = fread2(f + HL);
+            s2[f & 1] = Mfma<T>::run(fr[f % (HL + 1)], qf[f >> 1], s2[f & 1]);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          __builtin_amdgcn_s_setprio(0);
+          if (nk < 32) {
+            const int lim = nk - 4 * g;  // key 16 kb + 4g + r is valid iff 16 kb + r < lim
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+              for (int r = 0; r < 4; ++r)
+                if (kb * 16 + r >= lim) s2[kb][r] = -INFINITY;
+          }
+          float mx = vmax(vmax(vmax(s2[0][0], s2[0][1]), vmax(s2[0][2], s2[0][3])),
+                          vmax(vmax(s2[1][0], s2[1][1]), vmax(s2[1][2], s2[1][3])));
+          mx = lane_max_xor16_32(mx) * c;  // log2 units (c > 0)
+          const bool grow = mx > m_i + kRescaleSlack;
+          if (__builtin_amdgcn_ballot_w64(grow)) {
+            const float m_new = grow ? mx : m_i;
+            const float alpha = grow ? fast_exp2(m_i - m_new) : 1.f;
+            m_i = m_new;
+            l_i *= alpha;
+#pragma unroll
+            for (int db = 0; db < C::NDB; ++db) o[db] *= alpha;
+          }
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const f32x2 x = f32x2{fast_exp2(fmaf(s2[e >> 1][(e & 1) * 2], c, -m_i)),
+                                  fast_exp2(fmaf(s2[e >> 1][(e & 1) * 2 + 1], c, -m_i))};
+            l_i += x[0] + x[1];
+            pk[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(x, typename Pair<T>::type));
+          }
+          __builtin_amdgcn_s_setprio(2);
+#pragma unroll
+          for (int f = 32; f < 64; ++f) {
+            if (f + HL < 64) fr[(f + HL) % (HL + 1)] = fread2(f + HL);
+            o[f - 32] = Mfma<T>::run(fr[f % (HL + 1)], __builtin_bit_cast(v8, pk), o[f - 32]);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          __builtin_amdgcn_s_setprio(0);
+        }
+      } else {
       constexpr int NF = 128;
       v8 fr[LEAD + 1];
 #pragma unroll
@@ -1835,6 +1967,7 @@ __global__ __launch_bounds__(MlaRowsCfg::NT, 1) void attn_mla_rows_kernel(
 #pragma unroll
       for (int f = 96; f < 128; ++f) slot(f);
       __builtin_amdgcn_s_setprio(0);
+      }
     }
     __builtin_amdgcn_s_waitcnt(0);  // tile t+1 landed
     __syncthreads();                // and every wave is done with tile t
@@ -1843,21 +1976,41 @@ __global__ __launch_bounds__(MlaRowsCfg::NT, 1) void attn_mla_rows_kernel(
   // ---- epilogue: l over the 4 lanes holding the row's keys, O /= l, store the row
   l_i += __shfl_xor(l_i, 16);
   l_i += __shfl_xor(l_i, 32);
+  if constexpr (KH == 2) {  // keys 32-63's sums join keys 0-31's (the tile buffers are free)
+    int ln = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+    float* const xo = (float*)smem_raw + (rw * C::NDB * 64 + ln) * 4;             // [row wave][db][lane] x 4
+    float* const xm = (float*)(smem_raw + 2 * C::TILEB) + (rw * 64 + ln) * 2;  // m and l
+    if (kh == 1) {
+#pragma unroll
+      for (int db = 0; db < C::NDB; ++db) *(f32x4*)(xo + db * 256) = o[db];
+      xm[0] = m_i;
+      xm[1] = l_i;
+    }
+    __syncthreads();
+    if (kh == 1) return;
+    const float m1 = xm[0], l1 = xm[1];
+    const float M = fmaxf(m_i, m1);
+    const float a0 = m_i == M ? 1.f : fast_exp2(m_i - M), a1 = m1 == M ? 1.f : fast_exp2(m1 - M);
+#pragma unroll
+    for (int db = 0; db < C::NDB; ++db) o[db] = o[db] * a0 + *(const f32x4*)(xo + db * 256) * a1;
+    m_i = M;
+    l_i = l_i * a0 + l1 * a1;
+  }
   if (SPLIT && w.split_n > 1) {  // this part's record (O / l, then m and l per row, fp32) for merge_kernel
     char* const mine = split_record(hdr, spa, w.rec0 + w.split_s);
     // the lane's row and group computed anew: kept across the tile loop they would spill
     int ln = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
     asm volatile("" : "+v"(ln));
-    const int rr = wave * 16 + (ln & 15), rg = ln >> 4;
+    const int rr = rw * 16 + (ln & 15), rg = ln >> 4;
     if (!mine || rr >= w.qcount) return;
     const float inv = l_i > 0.f ? 1.f / l_i : 0.f;
     float* const dst = (float*)mine + rr * D + rg * 4;
 #pragma unroll
     for (int db = 0; db < C::NDB; ++db) *(f32x4*)(dst + db * 16) = o[db] * inv;
     if (rg == 0) {
-      float* const ml = (float*)mine + C::BQ * D;
+      float* const ml = (float*)mine + BQ * D;
       ml[rr] = m_i;
-      ml[C::BQ + rr] = l_i;
+      ml[BQ + rr] = l_i;
     }
     return;
   }
@@ -2354,13 +2507,21 @@ __global__ __launch_bounds__(kMergeThreads) void merge_kernel(const fmlm_attn_pa
       const int row = idx / (D / 8), c8 = idx - row * (D / 8);
       const char* src = rec0 + ((int64_t)(r0 + row) * D + c8 * 8) * 4;
       f32x4 a0 = f32x4{0.f, 0.f, 0.f, 0.f}, a1 = a0;
-#pragma unroll 4
-      for (int sp = 0; sp < S; ++sp) {
-        const f32x4 x0 = *(const f32x4*)(src + sp * rec_bytes);
-        const f32x4 x1 = *(const f32x4*)(src + sp * rec_bytes + 16);
-        const float ws = s_w[row][sp];
-        a0 += ws * x0;
-        a1 += ws * x1;
+      // eight parts' loads in flight (the last part's again past the end, at weight 0)
+      for (int s0 = 0; s0 < S; s0 += 8) {
+        f32x4 x0[8], x1[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const char* at = src + min(s0 + i, S - 1) * rec_bytes;
+          x0[i] = *(const f32x4*)at;
+          x1[i] = *(const f32x4*)(at + 16);
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const float ws = s0 + i < S ? s_w[row][s0 + i] : 0.f;
+          a0 += ws * x0[i];
+          a1 += ws * x1[i];
+        }
       }
       store8<T>((char*)p.o + (s_o[row] + c8 * 8) * (int64_t)sizeof(T), a0, a1);
     }
@@ -2414,19 +2575,27 @@ static Launch mfma3_launch(bool paged) {
 // the paged instantiation only for paged contexts: the page lookup costs registers the
 // contiguous kernel (at 256 VGPRs) does not have; the LSE one only for calls that store
 // the row statistics
-template <typename T, bool SPLIT>
+template <typename T, bool SPLIT, int KH>
 static const void* mla_rows_fn(bool paged, bool lse) {
-  return paged ? (lse ? (const void*)&attn_mla_rows_kernel<T, true, true, SPLIT>
-                      : (const void*)&attn_mla_rows_kernel<T, true, false, SPLIT>)
-               : (lse ? (const void*)&attn_mla_rows_kernel<T, false, true, SPLIT>
-                      : (const void*)&attn_mla_rows_kernel<T, false, false, SPLIT>);
+  return paged ? (lse ? (const void*)&attn_mla_rows_kernel<T, true, true, SPLIT, KH>
+                      : (const void*)&attn_mla_rows_kernel<T, true, false, SPLIT, KH>)
+               : (lse ? (const void*)&attn_mla_rows_kernel<T, false, true, SPLIT, KH>
+                      : (const void*)&attn_mla_rows_kernel<T, false, false, SPLIT, KH>);
 }
 template <typename T>
-static Launch mla_rows_launch(bool paged, bool lse) {
+static Launch mla_rows_launch(const fmlm_attn_params& p) {
   static_assert(MlaRowsCfg::BK == FMLM_PAGE_ROWS, "a paged context tile is one page");
-  Launch L{MlaRowsCfg::BQ, MlaRowsCfg::NT, MlaRowsCfg::LDS_BYTES, mla_rows_fn<T, false>(paged, lse), true, true, true};
-  L.split_fn = mla_rows_fn<T, true>(paged, lse);
-  return L;
+  const bool paged = p.ctx_block_table != nullptr, lse = p.lse != nullptr;
+  // Key halves for calls of up to 4096 (head, position) rows, 64 tiles of 64: 16 sequences of
+  // 1-4 tokens, 64 heads, 1400-7800 latent rows 50 us (128-row tiles 59); 4 sequences of 8,
+  // 32 heads 39 (47).  At 8192 rows (16 sequences of 8 tokens, 64 heads) they are slower, 115
+  // us against 103: every latent tile is then read by twice the workgroups.
+  if (p.cu_seqlens_q && (int64_t)p.H * p.total_q <= 4096) {
+    const void* fn = mla_rows_fn<T, true, 2>(paged, lse);
+    return Launch{MlaRowsCfg::BQ / 2, MlaRowsCfg::NT, MlaRowsCfg::LDS_BYTES + 2048, fn, true, true, true, fn};
+  }
+  return Launch{MlaRowsCfg::BQ, MlaRowsCfg::NT, MlaRowsCfg::LDS_BYTES, mla_rows_fn<T, false, 1>(paged, lse), true,
+                true, true, mla_rows_fn<T, true, 1>(paged, lse)};
 }
 
 // MFMA kernels by head dim.  The pipelined kernel and the 512-wide latent kernel need
@@ -2485,7 +2654,7 @@ static bool pick_mfma(const fmlm_attn_params& p, Launch& L) {
       return true;
     case 512:
       if (!(p.flags & FMLM_FLAG_MLA) || k != 1) return false;
-      L = mla_rows_launch<T>(p.ctx_block_table != nullptr, p.lse != nullptr);
+      L = mla_rows_launch<T>(p);
       return true;
     default: return false;
   }
@@ -2619,9 +2788,10 @@ static SplitCfg split_cfg(const fmlm_attn_params& p, const Launch& L) {
   if (min_units >= (int64_t)(kSplitRounds * sc.slots)) return SplitCfg{};
   sc.rec_cap = 3 * sc.slots;
   // The latent kernel: one or two whole rounds (see schedule_kernel), by the most units there
-  // can be.  16 sequences of 1-4 tokens, 64 heads, 1400-7800 latent rows each: 22 tiles took
-  // 261 us unsplit on as many CUs; split 47 us and the merge 10.  Up to 32 parts instead of
-  // 16: 15% slower (a part's fp32 record costs as much traffic as 8 tiles of keys).
+  // can be.  16 sequences of 1-4 tokens, 64 heads, 1400-7800 latent rows each: 22 tiles of
+  // 128 rows took 261 us unsplit on as many CUs; split 39 us and the merge 9.  Up to 32 parts
+  // instead of 16 change nothing there (a part's fp32 record costs as much traffic as 8
+  // tiles of keys).
   if (L.hpack)
     sc.rec_cap = (((int64_t)p.H * p.total_q + L.bq - 1) / L.bq + p.B <= sc.slots ? 1 : 2) * sc.slots;
   sc.rec_bytes = rec_bytes;
