@@ -23,6 +23,7 @@
 #include "fmlm_common.h"
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 #include <mutex>
 
@@ -84,7 +85,7 @@ constexpr int kHdrQueueLen = 8;   // [8, 16): entries of queue x
 
 __global__ __launch_bounds__(kSchedThreads) void schedule_kernel(const fmlm_attn_params p, int BQ,
                                                                  int cap_q, int slots,
-                                                                 int rec_cap,
+                                                                 int rec_cap, int split_min,
                                                                  int4* __restrict__ units,
                                                                  int32_t* __restrict__ header,
                                                                  int4* __restrict__ groups,
@@ -98,7 +99,7 @@ __global__ __launch_bounds__(kSchedThreads) void schedule_kernel(const fmlm_attn
   __shared__ unsigned char s_split[kSortMax];
   __shared__ int s_len[kXcds];
   __shared__ float s_sum[2];
-  __shared__ int s_chunk, s_groups, s_recs;
+  __shared__ int s_chunk, s_groups, s_recs, s_kmax;
   const int tid = threadIdx.x;
   const int B = p.B, H = p.H;
   const bool sorted = B <= kSortMax;
@@ -117,6 +118,7 @@ __global__ __launch_bounds__(kSchedThreads) void schedule_kernel(const fmlm_attn
     s_chunk = 0;
     s_groups = 0;
     s_recs = 0;
+    s_kmax = 0;
   }
   __syncthreads();
   if (sorted) {
@@ -131,9 +133,11 @@ __global__ __launch_bounds__(kSchedThreads) void schedule_kernel(const fmlm_attn
       s_work[b] = (float)ktiles;
       atomicAdd(&s_sum[0], units);
       atomicAdd(&s_sum[1], units * ktiles);
+      if (tiles > 0) atomicMax(&s_kmax, ktiles);
     }
     __syncthreads();
-    // split only when the units are too few to fill the slots for kSplitRounds rounds;
+    // split only when the units are too few to fill the slots for kSplitRounds rounds and
+    // the longest key range has more than split_min tiles (split_min_tiles);
     // parts of about total / (kSplitRounds * slots) key tiles, at least kMinSplitTiles,
     // the part size doubling until the records fit
     if (hpack) {
@@ -142,8 +146,7 @@ __global__ __launch_bounds__(kSchedThreads) void schedule_kernel(const fmlm_attn
       // long) as rounds x (key tiles of a part + what a part costs besides), and the
       // cheapest is taken.
       if (tid < 64 && rec_cap > 0 && s_sum[0] < kSplitRounds * slots) {
-        float kmax = 0.f;
-        for (int b = 0; b < B; ++b) kmax = fmaxf(kmax, s_tiles[b] > 0 ? s_work[b] : 0.f);
+        const float kmax = (float)s_kmax;
         const float chunk = fmaxf((float)kMinHpackTiles, ceilf(kmax / (tid + 1)));
         float parts = 0.f;
         for (int b = 0; b < B; ++b) {
@@ -157,7 +160,7 @@ __global__ __launch_bounds__(kSchedThreads) void schedule_kernel(const fmlm_attn
         for (int off = 1; off < 64; off <<= 1) best = fminf(best, __shfl_xor(best, off));
         if (cost == best && chunk < kmax) atomicMax(&s_chunk, (int)chunk);
       }
-    } else if (tid == 0 && rec_cap > 0 && s_sum[0] < kSplitRounds * slots) {
+    } else if (tid == 0 && rec_cap > 0 && s_sum[0] < kSplitRounds * slots && s_kmax > split_min) {
       int chunk = max(kMinSplitTiles, (int)ceilf(s_sum[1] / (kSplitRounds * slots)));
       for (int it = 0; it < 24; ++it, chunk *= 2) {
         float recs = 0.f;
@@ -2538,6 +2541,7 @@ struct Launch {
   bool hpack = false;  // packed tiles span (head, position) rows (MLA: one latent for all heads)
   bool paged = false;  // kernel reads a paged context (key tile = FMLM_PAGE_ROWS rows)
   const void* split_fn = nullptr;
+  float tile_us = 1.f;  // measured time of a 64-key tile, about one workgroup per CU
 };
 
 template <typename T, int D, int QB, int NW, int BK>
@@ -2555,7 +2559,9 @@ static Launch simt_launch() {
 template <int D, int QB>
 static Launch f32_launch() {
   typedef F32Cfg<D, QB> C;
-  return Launch{C::BQ, C::NT, C::LDS_BYTES, (const void*)&attn_f32_kernel<D, QB>, true};
+  Launch L{C::BQ, C::NT, C::LDS_BYTES, (const void*)&attn_f32_kernel<D, QB>, true};
+  L.tile_us = 0.3f + 0.6f * QB * D / 64;
+  return L;
 }
 
 template <typename T, int D, int QB, int NW, int BK, int PPB = 0>
@@ -2569,7 +2575,10 @@ static Launch mfma3_launch(bool paged) {
   } else if (paged) {  // the ping-pong configurations read contiguous contexts only
     fn = nullptr;
   }
-  return Launch{C::BQ, C::NT, C::LDS_BYTES, fn, true, false, true};
+  Launch L{C::BQ, C::NT, C::LDS_BYTES, fn, true, false, true};
+  // D = 64: 0.6 / 0.8 us with one / two row blocks per wave, D = 128: 0.86 / 1.12, D = 256: 1.7
+  L.tile_us = QB == 2 ? 0.48f + 0.005f * D : D <= 128 ? 0.34f + 0.0041f * D : 1.7f;
+  return L;
 }
 
 // the paged instantiation only for paged contexts: the page lookup costs registers the
@@ -2592,10 +2601,10 @@ static Launch mla_rows_launch(const fmlm_attn_params& p) {
   // us against 103: every latent tile is then read by twice the workgroups.
   if (p.cu_seqlens_q && (int64_t)p.H * p.total_q <= 4096) {
     const void* fn = mla_rows_fn<T, true, 2>(paged, lse);
-    return Launch{MlaRowsCfg::BQ / 2, MlaRowsCfg::NT, MlaRowsCfg::LDS_BYTES + 2048, fn, true, true, true, fn};
+    return Launch{MlaRowsCfg::BQ / 2, MlaRowsCfg::NT, MlaRowsCfg::LDS_BYTES + 2048, fn, true, true, true, fn, 2.f};
   }
   return Launch{MlaRowsCfg::BQ, MlaRowsCfg::NT, MlaRowsCfg::LDS_BYTES, mla_rows_fn<T, false, 1>(paged, lse), true,
-                true, true, mla_rows_fn<T, true, 1>(paged, lse)};
+                true, true, mla_rows_fn<T, true, 1>(paged, lse), 3.4f};
 }
 
 // MFMA kernels by head dim.  The pipelined kernel and the 512-wide latent kernel need
@@ -2622,9 +2631,22 @@ static bool pick_mfma(const fmlm_attn_params& p, Launch& L) {
   // workgroup would then leave half its waves without rows, one working wave per SIMD.
   // Measured 19-28% faster for 16-64 rows per sequence against a shared context, level at
   // 48-80 rows or where per-sequence contexts make the launch HBM-bound, 12-20% slower
-  // at 64-128 rows.  128-row workgroups (two blocks per wave) otherwise.
-  const bool short_q = (int64_t)p.total_q <= 64LL * p.B;
-  const int k = p.tile_config > 0 ? p.tile_config : ((p.D == 64 || p.D == 128) && short_q ? 3 : 1);
+  // at 64-128 rows.  The same for a dense call whose 128-row workgroups would fill at most
+  // half of the slots (512 at D = 128, 768 at 64): fp16 D = 128, 4 x 16 heads x 256 with
+  // 1000 context rows 30.2 us with 128-row workgroups, 24.0 with 64; 6 x 16 x 512 without
+  // context (384 workgroups of 128 rows) 24.2 against 27.3.  128-row workgroups (two blocks
+  // per wave) otherwise.
+  const bool short_q = p.cu_seqlens_q ? (int64_t)p.total_q <= 64LL * p.B
+                                      : (int64_t)p.total_q <= 64LL * p.B ||
+                                            (int64_t)p.B * p.H * ((p.N + 127) / 128) <= (p.D == 128 ? 256 : 384);
+  // D = 256 fills a CU's LDS with one workgroup: 8 waves (128 rows) as soon as 64-row ones
+  // would be more than one per CU, and longer sequences than they hold (8 sequences of 100-512, 16 heads: 62.9 us with 64-row
+  // workgroups, 54.8 with 128; 8 of 100-300, 8 heads, 232 of the former: 23.8 against 27.0).
+  const int64_t rows64 = p.cu_seqlens_q ? p.total_q / 64 + p.B / 2 : (int64_t)p.B * ((p.N + 63) / 64);
+  const int k = p.tile_config > 0                            ? p.tile_config
+                : (p.D == 64 || p.D == 128) && short_q       ? 3
+                : p.D == 256 && p.H * rows64 > 256 && (int64_t)p.total_q > 64LL * p.B ? 2
+                                                             : 1;
   switch (p.D) {
     case 16:
       if (k == 1) L = mfma3_launch<T, 16, 2, 4, 64>(paged); else return false;
@@ -2757,23 +2779,51 @@ struct SplitCfg {
   int dense_parts = 1;    // dense call: parts per query tile
 };
 
+// Key ranges of up to this many tiles are not split: two parts save half of them, the merge
+// costs 5 us and its launch's gap, so 20 us of key tiles (bf16 D = 128, 20 sequences of
+// 40-100 queries, 8 heads, 500-1000 context rows: 30 us whole, 34 in two).
+static int split_min_tiles(const Launch& L) {
+  return L.hpack ? kMinHpackTiles : std::max(kMinSplitTiles, (int)std::ceil(20.f / L.tile_us));
+}
+
+// key tiles of a packed call's query tile, at most
+static int64_t max_key_tiles(const fmlm_attn_params& p) {
+  const int64_t main = (p.flags & FMLM_FLAG_CAUSAL_SEQ) || p.N <= 0 ? p.total_q : std::min(p.N, p.total_q);
+  int64_t ctx = 0;
+  if (!(p.flags & FMLM_FLAG_PREFILL))
+    ctx = p.ctx_block_table ? (int64_t)std::max(p.ctx_pages_per_batch, 0) * FMLM_PAGE_ROWS
+          : p.cu_seqlens_kv ? std::max(p.ctx_rows, 0)
+                            : p.ctx_len;
+  return (ctx + kSplitBK - 1) / kSplitBK + (main + kSplitBK - 1) / kSplitBK;
+}
+
 static SplitCfg split_cfg(const fmlm_attn_params& p, const Launch& L) {
   SplitCfg sc;
-  if (!L.split || L.bq > kMergeRows) return sc;
+  if (!L.split || L.bq > kMergeRows || (p.flags & FMLM_FLAG_NOSPLIT)) return sc;
   sc.slots = resident_slots(L);
   if (sc.slots == 0) return sc;
   const int64_t rec_bytes = ((int64_t)L.bq * (p.D * 4 + 8) + 15) / 16 * 16;
   if (!p.cu_seqlens_q) {
     // Every query tile has the same keys: S equal parts each, when the tiles fill at most
-    // half of the slots (from there on the parts' records and merge cost what the idle slots
-    // do: 512 tiles on 768 slots were slower split).  Bf16, 16 heads, 24 queries, D = 128,
-    // 6000 context rows: 16 tiles, one workgroup each, took 80 us unsplit; 11 parts each
-    // 19.7, 16 parts 19.0, 32 parts 22.8.
+    // half of the slots.  S is the cheapest by a price in us: the key tiles of a part, and
+    // with S > 1 the merge (5 us) and the records' write and read at about 5 TB/s; a gain
+    // below 2 us is not taken.  Bf16, 16 heads, 24 queries, D = 128, 6000 context rows: 16
+    // tiles, one workgroup each, took 80 us unsplit, 18.5 in 16 parts; 3 x 16 heads x 512
+    // with 8 key tiles 17.7 us unsplit, 30 in two parts.
     const int64_t tiles = (int64_t)p.B * p.H * ((p.N + L.bq - 1) / L.bq);
     if (p.cu_seqlens_kv || tiles < 1 || 2 * tiles > sc.slots) return SplitCfg{};
     const int64_t ctx = (p.flags & FMLM_FLAG_PREFILL) ? 0 : p.ctx_len;
     const int64_t ktiles = (ctx + kSplitBK - 1) / kSplitBK + (p.N + kSplitBK - 1) / kSplitBK;
-    const int64_t S = std::min({(int64_t)kMaxSplits, sc.slots / tiles, ktiles / kMinDenseTiles});
+    const int64_t most = std::min({(int64_t)kMaxSplits, sc.slots / tiles, ktiles / kMinDenseTiles});
+    int64_t S = 1;
+    float best = L.tile_us * ktiles - 2.f;
+    for (int64_t n = 2; n <= most; ++n) {
+      const float cost = L.tile_us * ((ktiles + n - 1) / n) + 5.f + 2.f * tiles * n * rec_bytes / 5e6f;
+      if (cost < best) {
+        best = cost;
+        S = n;
+      }
+    }
     if (S < 2) return SplitCfg{};
     sc.dense_parts = (int)S;
     sc.rec_cap = (int)(tiles * S);
@@ -2887,7 +2937,7 @@ static int launch_schedule(const fmlm_attn_params& p, const Launch& L, const Spl
   // a buffer without room for the records: each launch brings its own (split_record)
   const int64_t records_off = bytes >= l.bytes ? l.records_off : 0;
   hipLaunchKernelGGL(schedule_kernel, dim3(1), dim3(kSchedThreads), 0, s, p, L.bq, (int)l.cap,
-                     sc.slots, sc.rec_cap, (int4*)(sched + l.units_off), header,
+                     sc.slots, sc.rec_cap, split_min_tiles(L), (int4*)(sched + l.units_off), header,
                      (int4*)(sched + l.groups_off), (int)l.groups_off, (int)records_off,
                      (int)sc.rec_bytes, (int)L.hpack);
   return launch_status();
@@ -3028,6 +3078,8 @@ extern "C" int64_t fmlm_attn_records_bytes(const fmlm_attn_params* p) {
   Launch L;
   const int rc = pick_launch(*p, L);
   if (rc) return rc;
+  // a packed call whose longest key range is one part at most cannot split
+  if (p->cu_seqlens_q && max_key_tiles(*p) <= split_min_tiles(L)) return 0;
   return records_for(split_cfg(*p, L));
 }
 

@@ -25,6 +25,7 @@ DTYPE_F32 = 2
 FLAG_MLA = 1
 FLAG_PREFILL = 2
 FLAG_CAUSAL_SEQ = 4
+FLAG_NOSPLIT = 8
 
 LAYOUT_PADDED = 0
 LAYOUT_PACKED = 1

@@ -443,15 +443,17 @@ def _prepare(
     p.k_ctx = k_ctx.data_ptr() if k_ctx.numel() else None
     p.v_ctx = v_ctx.data_ptr() if (v_ctx is not None and v_ctx.numel()) else p.k_ctx
     p.c_sb, p.c_sh, p.c_sn = c_strides
-    ws_bytes = int(lib.fmlm_attn_workspace_bytes(p))
-    _lib.check(ws_bytes if ws_bytes < 0 else 0, "fmlm_attn_workspace_bytes")
+    records = int(lib.fmlm_attn_records_bytes(p))
+    _lib.check(records if records < 0 else 0, "fmlm_attn_records_bytes")
+    if records == 0:
+        p.flags |= _lib.FLAG_NOSPLIT
+    # a dense call needs a workspace for split partial results only
+    ws_bytes = records if cu_seqlens_q is None else int(lib.fmlm_attn_workspace_bytes(p))
     stream = _lib.stream_of(q.device)
     sched = ws = None
-    records = 0
     if cu_seqlens_q is None:
-        records = ws_bytes  # a dense call needs a workspace for split partial results only
+        pass
     elif ws_bytes > 0 and schedule_cache is not None:
-        records = int(lib.fmlm_attn_records_bytes(p))
         # what the unit list depends on: the kernel (dtype, head dim, flags, K/V
         # layout, paged context or not), whose tile size and occupancy fix the slots,
         # the split records and the grid, and the shape (B, H, N, total_q); context
@@ -470,6 +472,7 @@ def _prepare(
         ws = _workspace(inference_cache, ws_bytes, q.device)
         p.workspace = ws.data_ptr()
         p.workspace_bytes = ws_bytes
+        records = 0  # part of the workspace
     keep = (q, out, k, v, k_ctx, v_ctx, cu_seqlens_q, cu_seqlens_kv, ctx_index, block_table, ws, sched)
     plan = AttnLaunch(lib, p, stream, q.device, keep)
     plan.records = records

@@ -51,7 +51,9 @@ enum {
 enum {
   FMLM_FLAG_MLA = 1,        /* V is K (one shared latent head for main and context) */
   FMLM_FLAG_PREFILL = 2,    /* skip the cached-context segment */
-  FMLM_FLAG_CAUSAL_SEQ = 4  /* sequence b attends to main tokens [0, cu_q[b+1]) */
+  FMLM_FLAG_CAUSAL_SEQ = 4, /* sequence b attends to main tokens [0, cu_q[b+1]) */
+  FMLM_FLAG_NOSPLIT = 8     /* key ranges are not split (no records, no merge launch); a
+                               schedule is then built with this flag too               */
 };
 
 /* row layouts of a [*, D] tensor addressed by (sequence b, head h, position p) */
@@ -235,9 +237,10 @@ typedef struct fmlm_attn_params {
   int64_t ctx_page_stride;
   int32_t ctx_pages_per_batch;
   /* Tile configuration of the bf16/f16 attention kernel: 0 = chosen by the library from
-   * the head dim and the query rows per sequence (D = 64 and 128: configuration 3 when
-   * total_q <= 64 * B, i.e. sequences of at most 64 query rows on average, else 1; other
-   * head dims: 1); k >= 1
+   * the head dim and the query rows (D = 64 and 128: configuration 3 when total_q <=
+   * 64 * B, i.e. sequences of at most 64 query rows on average, or when the 128-row
+   * workgroups of a dense call would fill at most half of the GPU, else 1; D = 256: 2 when
+   * 64-row workgroups would be more than 256 and total_q > 64 * B, else 1; other head dims: 1); k >= 1
    * forces compiled configuration k of the head dim (fmlm_attn_workspace_bytes returns
    * FMLM_E_ARG for a k that does not exist).  Configurations, as (query rows per
    * workgroup, waves per workgroup): D = 16, 32: 1 = (128, 4); D = 64: 1 = (128, 4),
@@ -263,8 +266,10 @@ typedef struct fmlm_attn_params {
  * (cu_seqlens_q == NULL) also runs without: its key ranges are then not split. */
 FMLM_API int64_t fmlm_attn_workspace_bytes(const fmlm_attn_params* p);
 
-/* The part of fmlm_attn_workspace_bytes that holds split partial results (0 when the call
- * never splits), or < 0 as above.  A schedule buffer without that part serves calls that
+/* The part of fmlm_attn_workspace_bytes that holds split partial results, or < 0 as above.
+ * 0 when the call cannot split: with FMLM_FLAG_NOSPLIT set it then does the same with one
+ * launch less, in a smaller schedule and workspace (for a packed call by its own context
+ * sizes: without the flag it must still run a schedule built for longer contexts).  A schedule buffer without that part serves calls that
  * bring a workspace of this many bytes. */
 FMLM_API int64_t fmlm_attn_records_bytes(const fmlm_attn_params* p);
 

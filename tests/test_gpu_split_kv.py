@@ -33,12 +33,12 @@ def _randn(gen, shape, dtype, device, std=1.0):
 DENSE = [
     # B, H, N, D, context rows, context batches, dtype: part counts that divide the key
     # tiles unevenly, one query row, a row past a tile, one row short of a key tile
-    (1, 4, 1, 64, 511, 1, torch.bfloat16),
-    (2, 3, 65, 64, 1000, 2, torch.float16),
+    (1, 4, 1, 64, 2047, 1, torch.bfloat16),
+    (2, 3, 65, 64, 2500, 2, torch.float16),
     (1, 2, 17, 128, 6001, 1, torch.bfloat16),
-    (1, 1, 128, 256, 640, 1, torch.float16),
-    (3, 2, 130, 32, 449, 3, torch.bfloat16),
-    (1, 3, 600, 16, 1, 1, torch.float16),
+    (1, 1, 128, 256, 1300, 1, torch.float16),
+    (3, 2, 130, 32, 2049, 3, torch.bfloat16),
+    (1, 3, 600, 16, 3001, 1, torch.float16),
     (1, 2, 33, 64, 2050, 1, torch.float32),
 ]
 
