@@ -2045,22 +2045,22 @@ __global__ __launch_bounds__(MlaRowsCfg::NT, 1) void attn_mla_rows_kernel(
 
 // ---------------------------------------------------------------------------
 // fp32 kernel on the matrix cores (v_mfma_f32_16x16x4_f32: fp32 operands and accumulation,
-// 32 cycles each, so the products cost 16 times the 16-bit kernels' and bound the kernel:
-// nothing is staged in LDS, every fragment comes straight from L1 / L2).  One workgroup is
+// 32 cycles each, so the products cost 16 times the 16-bit kernels' and bound the kernel).
+// One workgroup is
 // one (query tile of QB*16 rows, head); its 4 waves split every 64-key tile, 16 keys each,
 // and add up their partial results through LDS at the end, so that a call of a few query
 // rows still has 4 waves per tile at work.  Lane (j + 16g) of a fragment:
-//   K (A of S^T = K Q^T), Q (B)  row j, columns 16s + 4g .. +4 as one 16-byte load: MFMA e
+//   K (A of S^T = K Q^T), Q (B)  row j, columns 16s + 4g .. +4 as one 16-byte read: MFMA e
 //                                of step s contracts columns 16s + 4g' + e, g' = 0..3
 //   S^T                          key 4g + r of query j in register r, which is the B
 //                                operand of the MFMA that contracts keys 4g' + r
-//   V^T (A of O^T = V^T P^T)     E consecutive columns of key row 4g + r in one load; MFMA
+//   V^T (A of O^T = V^T P^T)     E consecutive columns of key row 4g + r in one read; MFMA
 //                                e builds the columns E*i + e (i < 16) of a 16E-wide group
 // so a lane ends up with 4E consecutive columns of O per group.
-// The next tile's K is loaded behind this tile's S, V behind the previous tile's P V: one
-// register copy of each.  Bound by the MFMAs: 8 x 12 heads x 512 x 512, D = 64, 73 us, 88
-// TFLOP/s (D = 128: 92; a library fp32 product reaches 154); the SIMT kernel below ran at
-// 13.  With loops in place of `skip` the compiler moved V's loads behind the S MFMAs: 85 us.
+// The next tile's K is loaded (F32Tile) once this tile's S has read the buffer, V once its
+// P V has: each has the other product's time.  8 x 12 heads x 512 x 512, D = 64: 70.7 us, 91
+// TFLOP/s (D = 128: 96; a library fp32 product reaches 154); with fragments straight from
+// L1 / L2 73.5; the SIMT kernel below ran at 13 TFLOP/s.
 // ---------------------------------------------------------------------------
 template <int D, int QB>
 struct F32Cfg {
@@ -2068,11 +2068,11 @@ struct F32Cfg {
   static constexpr int NT = NW * 64;
   static constexpr int BQ = 16 * QB;
   static constexpr int BK = kSplitBK;             // keys per tile, 16 per wave
-  static constexpr int DS = D / 16;               // 16-column steps of S^T
-  static constexpr int E = D >= 64 ? 4 : D / 16;  // columns per lane and V load
-  static constexpr int NG = D / (16 * E);         // column groups of O^T
-  static constexpr int OP = D + 4;                // LDS row pitch (floats): 16 rows on distinct banks
-  static constexpr int LDS_BYTES = NW * BQ * (OP + 2) * 4;
+  static constexpr int DS = F32Tile<D>::DS, E = F32Tile<D>::E, NG = F32Tile<D>::NG;
+  static constexpr int OP = D + 4;                // LDS row pitch of the sums (floats): 16 rows on distinct banks
+  static constexpr int TILES = NW * 2 * F32Tile<D>::BYTES;  // a K and a V tile per wave
+  static constexpr int SUMS = NW * BQ * (OP + 2) * 4;       // the waves' sums, after the loop
+  static constexpr int LDS_BYTES = TILES > SUMS ? TILES : SUMS;
   // waves per SIMD: the fragments of 256 columns take more than 256 registers
   static constexpr int WPS = D >= 256 ? 1 : 2;
   static_assert(BK == NW * 16, "16 keys of a tile per wave");
@@ -2082,7 +2082,6 @@ template <int D, int QB>
 __global__ __launch_bounds__(256, (F32Cfg<D, QB>::WPS)) void attn_f32_kernel(
     const fmlm_attn_params p, const int4* __restrict__ units, const int32_t* __restrict__ hdr, const SplitArgs spa) {
   typedef F32Cfg<D, QB> C;
-  typedef typename FloatN<C::E>::type vE;
   extern __shared__ __align__(16) char smem_raw[];
   float* const ob = (float*)smem_raw;             // [NW][BQ][OP]
   float* const mb = ob + C::NW * C::BQ * C::OP;   // [NW][BQ]
@@ -2123,23 +2122,17 @@ __global__ __launch_bounds__(256, (F32Cfg<D, QB>::WPS)) void attn_f32_kernel(
   const int skip = wave * 16 >= n0 - (nt0 - 1) * C::BK ? nt0 - 1 : -1;
   const int end = te == ntiles && te > nt0 && key0(te - 1) >= n1 ? te - 1 : te;
   auto from = [&](int t) { return t == skip ? t + 1 : t; };
-  // row pitches lie below 2^22 elements (check_params): one 32 x 32 bit product
-  auto row_off = [](int key, int64_t sn) { return (uint64_t)(uint32_t)key * (uint32_t)sn; };
-  // rows past the segment's end repeat its last row (their scores are masked)
-  auto load_k = [&](int t, f32x4(&k)[C::DS]) {
-    const int key = min(key0(t) + l16, nkeys(t) - 1);
-    const float* src = (t < nt0 ? kp0 : kp1) + row_off(key, t < nt0 ? w.seg[0].ksn : w.seg[1].ksn) + 4 * g;
-#pragma unroll
-    for (int ds = 0; ds < C::DS; ++ds) k[ds] = *(const f32x4*)(src + 16 * ds);
-  };
-  auto load_v = [&](int t, vE(&v)[4][C::NG]) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int key = min(key0(t) + 4 * g + r, nkeys(t) - 1);
-      const float* src = (t < nt0 ? vp0 : vp1) + row_off(key, t < nt0 ? w.seg[0].vsn : w.seg[1].vsn) + C::E * l16;
-#pragma unroll
-      for (int dg = 0; dg < C::NG; ++dg) v[r][dg] = *(const vE*)(src + 16 * C::E * dg);
-    }
+  // the loads of this wave's 16 keys of tile t (row pitches lie below 2^22 elements,
+  // check_params); rows past the segment's end repeat its last row, their scores are masked
+  typedef F32Tile<D> TL;
+  const uint32_t kt = lds_addr(smem_raw) + wave * 2 * TL::BYTES, vt = kt + TL::BYTES;
+  auto load = [&](int t, bool v) {
+    const bool cx = t < nt0;
+    const int64_t sn = cx ? (v ? w.seg[0].vsn : w.seg[0].ksn) : (v ? w.seg[1].vsn : w.seg[1].ksn);
+    const float* base = cx ? (v ? vp0 : kp0) : (v ? vp1 : kp1);
+    const int j0 = key0(t);
+    TL::load(uniform_ptr((const char*)(base + (uint64_t)(uint32_t)j0 * (uint32_t)sn)),
+             __builtin_amdgcn_readfirstlane((uint32_t)sn * 4u), nkeys(t) - 1 - j0, v ? vt : kt, lane);
   };
 
   f32x4 o[QB][C::NG][C::E];
@@ -2156,26 +2149,20 @@ __global__ __launch_bounds__(256, (F32Cfg<D, QB>::WPS)) void attn_f32_kernel(
 
   int t = from(tb);
   if (t < end) {
-    f32x4 k[C::DS];
-    vE v[4][C::NG];
-    load_k(t, k);
+    const uint32_t krow = TL::row_base(kt, l16, g);
+    load(t, false);
+    load(t, true);
     while (t < end) {
-      load_v(t, v);
-      __builtin_amdgcn_sched_barrier(0);  // the loads stay ahead of the MFMAs that cover them
       f32x4 s[QB];
 #pragma unroll
       for (int qb = 0; qb < QB; ++qb) s[qb] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int ds = 0; ds < C::DS; ++ds)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-#pragma unroll
-          for (int qb = 0; qb < QB; ++qb) s[qb] = mfma_f32(k[ds][e], q[qb][ds][e], s[qb]);
-      __builtin_amdgcn_sched_barrier(0);
+      wait_loads<TL::NL>();  // K (V's loads came later)
+      mma_rows<D, QB>(krow, q, s);
       const int lim = nkeys(t) - key0(t) - 4 * g;  // key 4g + r is valid iff r < lim
       const int tn = from(t + 1);
-      load_k(tn < end ? tn : t, k);  // unconditional: a branch here would make the wait for V wait for K too
-      __builtin_amdgcn_sched_barrier(0);
+      const int tl = tn < end ? tn : t;  // past the end: once more, unused
+      wait_reads();
+      load(tl, false);
       bool grow = false;
 #pragma unroll
       for (int qb = 0; qb < QB; ++qb) {
@@ -2203,18 +2190,15 @@ __global__ __launch_bounds__(256, (F32Cfg<D, QB>::WPS)) void attn_f32_kernel(
         for (int r = 0; r < 4; ++r) s[qb][r] = fast_exp2(s[qb][r] - (m_i[qb] == -INFINITY ? 0.f : m_i[qb]));
         l_i[qb] += (s[qb][0] + s[qb][1]) + (s[qb][2] + s[qb][3]);
       }
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-#pragma unroll
-        for (int dg = 0; dg < C::NG; ++dg)
-#pragma unroll
-          for (int e = 0; e < C::E; ++e)
-#pragma unroll
-            for (int qb = 0; qb < QB; ++qb)
-              o[qb][dg][e] = mfma_f32(elem_of<C::E>(v[r][dg], e), s[qb][r], o[qb][dg][e]);
+      wait_loads<TL::NL>();  // V (the next K's loads came later)
+      mma_cols<D, QB>(vt, l16, g, s, o);
+      wait_reads();
+      load(tl, true);
       t = tn;
     }
+    wait_loads<0>();
   }
+  __syncthreads();  // the sums below reuse the tiles' memory
 
   // ---- the waves' partial results to LDS, then the rows' sums over the waves
 #pragma unroll
@@ -2227,18 +2211,7 @@ __global__ __launch_bounds__(256, (F32Cfg<D, QB>::WPS)) void attn_f32_kernel(
       mb[wave * C::BQ + row] = m_i[qb];
       lb[wave * C::BQ + row] = l;
     }
-    float* dst = ob + (wave * C::BQ + row) * C::OP + 4 * C::E * g;
-#pragma unroll
-    for (int dg = 0; dg < C::NG; ++dg)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        vE x;
-        if constexpr (C::E == 1) x = o[qb][dg][0][r];
-        else
-#pragma unroll
-          for (int e = 0; e < C::E; ++e) x[e] = o[qb][dg][e][r];
-        *(vE*)(dst + 16 * C::E * dg + C::E * r) = x;
-      }
+    store_cols<D>(o[qb], ob + (wave * C::BQ + row) * C::OP, g);
   }
   __syncthreads();
   char* rec = nullptr;

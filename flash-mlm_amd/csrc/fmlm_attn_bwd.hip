@@ -1941,27 +1941,33 @@ __global__ __launch_bounds__(256) void attn_bwd_dkv_simt_kernel(const fmlm_attn_
 
 // ---------------------------------------------------------------------------
 // fp32 backward on the matrix cores (v_mfma_f32_16x16x4_f32; head dims up to 256,
-// contiguous contexts), bound by the MFMAs like the fp32 forward and built like it: no LDS
-// in the loops, fragments straight from L1 / L2 in its two forms, "row" (lane (j + 16g):
-// row j, columns 16s + 4g .. +4, contracted over the columns) and "col" (row 4g + r, E
-// consecutive columns, contracted over the rows), each loaded behind the MFMAs of another.
+// contiguous contexts), bound by the MFMAs like the fp32 forward and built like it: 16-row
+// tiles private to a wave (F32Tile), read in two forms, "row" (lane (j + 16g): row j,
+// columns 16s + 4g .. +4, contracted over the columns) and "col" (row 4g + r, E consecutive
+// columns, contracted over the rows), both from one load of the tile.
 // The 4 waves of a workgroup split the contraction's long side (dq: 16 keys of every 64;
-// dK / dV: 16 query rows of every 64) and add their sums up through LDS at the end.
+// dK / dV: 16 query rows of every 64) and add their sums up through LDS at the end.  8 x 12
+// heads x 512 x 512: 240 us at D = 64 (67 TFLOP/s of 5 products, 94 of the 7 computed), 457
+// at D = 128; with fragments straight from L1 / L2 275 and 602 us.
 // ---------------------------------------------------------------------------
 template <int D>
 struct F32BwdCfg {
-  static constexpr int DS = D / 16;               // 16-column steps of a row fragment
-  static constexpr int E = D >= 64 ? 4 : D / 16;  // columns per lane of a col fragment
-  static constexpr int NG = D / (16 * E);         // column groups
-  static constexpr int OP = D + 4;                // LDS row pitch (floats)
+  typedef F32Tile<D> TL;
+  static constexpr int DS = TL::DS, E = TL::E, NG = TL::NG;
+  static constexpr int OP = D + 4;  // LDS row pitch of the sums (floats)
   // 16-row query blocks of a dq workgroup, 16-key blocks of a dK / dV workgroup: as many as
   // fit two waves per SIMD (8 x 12 heads x 512, D = 64: two of each 275 us; one query block
   // 292, one key block 306)
   static constexpr int QB = D == 16 ? 4 : D <= 64 ? 2 : 1;
   static constexpr int KB = QB;
   static constexpr int BQ = 16 * QB, KEYS = 16 * KB;
-  static constexpr int DQ_LDS = kBwdNW * BQ * (OP + 3) * 4;
-  static constexpr int DKV_LDS = kBwdNW * KEYS * OP * 4;
+  // tiles per wave: dq K (two, the next one loading during this one's math) and V; dK / dV
+  // Q and dO, two each.  One each where two would leave one workgroup per CU (D >= 128).
+  static constexpr int NBUF = D <= 64 ? 2 : 1;
+  static constexpr int DQ_TILES = kBwdNW * (NBUF + 1) * TL::BYTES, DQ_SUMS = kBwdNW * BQ * (OP + 3) * 4;
+  static constexpr int DKV_TILES = kBwdNW * 2 * NBUF * TL::BYTES, DKV_SUMS = kBwdNW * KEYS * OP * 4;
+  static constexpr int DQ_LDS = DQ_TILES > DQ_SUMS ? DQ_TILES : DQ_SUMS;
+  static constexpr int DKV_LDS = DKV_TILES > DKV_SUMS ? DKV_TILES : DKV_SUMS;
   // waves per SIMD: 256 columns take more than 256 registers
   static constexpr int WPS = D >= 256 ? 1 : 2;
 };
@@ -1972,55 +1978,13 @@ FMLM_DEV void load_row_frag(const float* src, f32x4 (&x)[F32BwdCfg<D>::DS]) {
 #pragma unroll
   for (int ds = 0; ds < F32BwdCfg<D>::DS; ++ds) x[ds] = *(const f32x4*)(src + 16 * ds);
 }
-// acc[i] += A B over the columns, A's row fragments a and B's b[i]
-template <int D, int N>
-FMLM_DEV void mma_rows(const f32x4 (&a)[F32BwdCfg<D>::DS], const f32x4 (&b)[N][F32BwdCfg<D>::DS], f32x4 (&acc)[N]) {
-#pragma unroll
-  for (int ds = 0; ds < F32BwdCfg<D>::DS; ++ds)
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-#pragma unroll
-      for (int i = 0; i < N; ++i) acc[i] = mfma_f32(a[ds][e], b[i][ds][e], acc[i]);
-}
-// o[i] += X^T b[i] over 16 rows, X's col fragments x: row 4g + r against b[i][r]
-template <int D, int N>
-FMLM_DEV void mma_cols(const typename FloatN<F32BwdCfg<D>::E>::type (&x)[4][F32BwdCfg<D>::NG], const f32x4 (&b)[N],
-                       f32x4 (&o)[N][F32BwdCfg<D>::NG][F32BwdCfg<D>::E]) {
-  typedef F32BwdCfg<D> C;
-#pragma unroll
-  for (int r = 0; r < 4; ++r)
-#pragma unroll
-    for (int dg = 0; dg < C::NG; ++dg)
-#pragma unroll
-      for (int e = 0; e < C::E; ++e)
-#pragma unroll
-        for (int i = 0; i < N; ++i) o[i][dg][e] = mfma_f32(elem_of<C::E>(x[r][dg], e), b[i][r], o[i][dg][e]);
-}
-// the lane's columns of accumulator o, row l16 of its block, to an LDS row
-template <int D>
-FMLM_DEV void store_cols(const f32x4 (&o)[F32BwdCfg<D>::NG][F32BwdCfg<D>::E], float* row, int g) {
-  typedef F32BwdCfg<D> C;
-  typedef typename FloatN<C::E>::type vE;
-#pragma unroll
-  for (int dg = 0; dg < C::NG; ++dg)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      vE x;
-      if constexpr (C::E == 1) x = o[dg][0][r];
-      else
-#pragma unroll
-        for (int e = 0; e < C::E; ++e) x[e] = o[dg][e][r];
-      *(vE*)(row + 4 * C::E * g + 16 * C::E * dg + C::E * r) = x;
-    }
-}
-
 template <int D>
 __global__ __launch_bounds__(256, F32BwdCfg<D>::WPS) void attn_bwd_dq_f32_kernel(const fmlm_attn_params p,
                                                                                  const fmlm_attn_grads g_,
                                                                                  const int32_t* qrec, int nq,
                                                                                  int nfill) {
   typedef F32BwdCfg<D> C;
-  typedef typename FloatN<C::E>::type vE;
+  typedef F32Tile<D> TL;
   constexpr int QB = C::QB, BK = 64;
   extern __shared__ __align__(16) char smem_raw[];
   float* const ob = (float*)smem_raw;                 // [NW][BQ][OP]
@@ -2064,7 +2028,6 @@ __global__ __launch_bounds__(256, F32BwdCfg<D>::WPS) void attn_bwd_dq_f32_kernel
     }
     d += __shfl_xor(d, 16);
     delta[qb] = d + __shfl_xor(d, 32);
-    if (wave == 0 && g == 0) delta_s[row] = delta[qb];
   }
 
   const BSeg sc = ctx_seg_at(p, g_, rec[6], h, rec[7], rec[8]);
@@ -2076,13 +2039,17 @@ __global__ __launch_bounds__(256, F32BwdCfg<D>::WPS) void attn_bwd_dq_f32_kernel
   const int skip = wave * 16 >= sc.n - (nt0 - 1) * BK ? nt0 - 1 : -1;
   const int end = ntiles > nt0 && key0(ntiles - 1) >= sm.n ? ntiles - 1 : ntiles;
   auto from = [&](int t) { return t == skip ? t + 1 : t; };
-  // rows past the segment's end repeat its last row (their scores are masked)
-  auto row_of = [&](int t, int key, bool v) {
+  // the loads of this wave's 16 keys of tile t; rows past the segment's end repeat its last
+  // row (their scores are masked)
+  const uint32_t vt = lds_addr(smem_raw) + wave * (C::NBUF + 1) * TL::BYTES, kt0 = vt + TL::BYTES;
+  auto load = [&](int t, bool v, uint32_t dst) {
     const bool cx = t < nt0;
     const float* base = cx ? (const float*)(v ? sc.v : sc.k) + (v ? sc.vbase : sc.kbase)
                            : (const float*)(v ? sm.v : sm.k) + (v ? sm.vbase : sm.kbase);
     const int64_t sn = cx ? (v ? sc.vsn : sc.ksn) : (v ? sm.vsn : sm.ksn);
-    return base + (uint64_t)(uint32_t)min(key, nkeys(t) - 1) * (uint32_t)sn;
+    const int j0 = key0(t);
+    TL::load(uniform_ptr((const char*)(base + (uint64_t)(uint32_t)j0 * (uint32_t)sn)),
+             __builtin_amdgcn_readfirstlane((uint32_t)sn * 4u), nkeys(t) - 1 - j0, dst, lane);
   };
 
   f32x4 acc[QB][C::NG][C::E];
@@ -2098,31 +2065,29 @@ __global__ __launch_bounds__(256, F32BwdCfg<D>::WPS) void attn_bwd_dq_f32_kernel
   }
   int t = from(0);
   if (t < end) {
-    f32x4 kr[C::DS], vr[C::DS];
-    vE kc[4][C::NG];
-    load_row_frag<D>(row_of(t, key0(t) + l16, false) + 4 * g, kr);
+    uint32_t kt = kt0;
+    load(t, false, kt);
+    load(t, true, vt);
     while (t < end) {
-      load_row_frag<D>(row_of(t, key0(t) + l16, true) + 4 * g, vr);
-      __builtin_amdgcn_sched_barrier(0);  // loads stay ahead of the MFMAs that cover them
+      const int tn = from(t + 1);
+      const int tl = tn < end ? tn : t;  // past the end: once more, unused
+      const uint32_t kn = C::NBUF == 2 ? kt0 + (kt == kt0 ? TL::BYTES : 0) : kt;
       f32x4 s[QB], dp[QB];
 #pragma unroll
       for (int qb = 0; qb < QB; ++qb) s[qb] = dp[qb] = f32x4{0.f, 0.f, 0.f, 0.f};
-      mma_rows<D, QB>(kr, q, s);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float* src = row_of(t, key0(t) + 4 * g + r, false) + C::E * l16;
-#pragma unroll
-        for (int dg = 0; dg < C::NG; ++dg) kc[r][dg] = *(const vE*)(src + 16 * C::E * dg);
+      if constexpr (C::NBUF == 2) {
+        wait_loads<TL::NL>();  // K (V's loads came later)
+        load(tl, false, kn);   // the buffer that the last tile's dq read
+        mma_rows<D, QB>(TL::row_base(kt, l16, g), q, s);
+        wait_loads<TL::NL>();  // V (the next K's came later)
+      } else {
+        wait_loads<0>();  // V was loaded before K
+        mma_rows<D, QB>(TL::row_base(kt, l16, g), q, s);
       }
-      __builtin_amdgcn_sched_barrier(0);
-      mma_rows<D, QB>(vr, dof, dp);
-      __builtin_amdgcn_sched_barrier(0);
+      mma_rows<D, QB>(TL::row_base(vt, l16, g), dof, dp);
+      wait_reads();
+      load(tl, true, vt);
       const int lim = nkeys(t) - key0(t) - 4 * g;  // key 4g + r is valid iff r < lim
-      const int tn = from(t + 1);
-      const int tl = tn < end ? tn : t;
-      load_row_frag<D>(row_of(tl, key0(tl) + l16, false) + 4 * g, kr);
-      __builtin_amdgcn_sched_barrier(0);
       bool grow = false;
 #pragma unroll
       for (int qb = 0; qb < QB; ++qb) {
@@ -2154,10 +2119,15 @@ __global__ __launch_bounds__(256, F32BwdCfg<D>::WPS) void attn_bwd_dq_f32_kernel
         }
         l_i[qb] += (s[qb][0] + s[qb][1]) + (s[qb][2] + s[qb][3]);
       }
-      mma_cols<D, QB>(kc, dp, acc);
+      mma_cols<D, QB>(kt, l16, g, dp, acc);
+      wait_reads();
+      if constexpr (C::NBUF == 1) load(tl, false, kt);
+      kt = kn;
       t = tn;
     }
+    wait_loads<0>();
   }
+  __syncthreads();  // the sums below reuse the tiles' memory
 
   // ---- the waves' sums to LDS, then the rows' sums over the waves
 #pragma unroll
@@ -2169,6 +2139,7 @@ __global__ __launch_bounds__(256, F32BwdCfg<D>::WPS) void attn_bwd_dq_f32_kernel
     if (g == 0) {
       mb[wave * C::BQ + row] = m_i[qb];
       lb[wave * C::BQ + row] = l;
+      if (wave == 0) delta_s[row] = delta[qb];
     }
     store_cols<D>(acc[qb], ob + (wave * C::BQ + row) * C::OP, g);
   }
@@ -2205,7 +2176,7 @@ __global__ __launch_bounds__(256, F32BwdCfg<D>::WPS) void attn_bwd_dkv_f32_kerne
                                                                                   const fmlm_attn_grads g_, int n_ctx,
                                                                                   const int32_t* krec, int nk) {
   typedef F32BwdCfg<D> C;
-  typedef typename FloatN<C::E>::type vE;
+  typedef F32Tile<D> TL;
   constexpr int KB = C::KB, QS = kBwdNW * 16;
   extern __shared__ __align__(16) char smem_raw[];
   float* const red = (float*)smem_raw;  // [NW][KEYS][OP]
@@ -2247,20 +2218,24 @@ __global__ __launch_bounds__(256, F32BwdCfg<D>::WPS) void attn_bwd_dkv_f32_kerne
     }
     return st;
   };
-  auto q_row = [&](const QStep& st, const SeqInfo& si, int pos) {
-    return (const float*)p.q + row_at(p.q_layout, st.b, st.hq, si.q0, min(pos, si.len - 1), p.q_sb, p.q_sh, p.q_sn);
-  };
-  auto o_row = [&](const QStep& st, const SeqInfo& si, int pos) {
-    return (const float*)g_.dout +
-           row_at(p.o_layout, st.b, st.hq, si.q0, min(pos, si.len - 1), g_.do_sb, g_.do_sh, g_.do_sn);
+  // the loads of this wave's 16 Q (or dO) rows of a step; rows past the sequence's end repeat
+  // its last one (their P is 0)
+  const uint32_t base_lds = lds_addr(smem_raw) + wave * 2 * C::NBUF * TL::BYTES;
+  auto load = [&](const QStep& st, const SeqInfo& si, bool dout, uint32_t dst) {
+    const int r0 = st.p0 + wave * 16;
+    const char* src = dout ? (const char*)((const float*)g_.dout + row_at(p.o_layout, st.b, st.hq, si.q0, r0, g_.do_sb,
+                                                                          g_.do_sh, g_.do_sn))
+                           : (const char*)((const float*)p.q +
+                                           row_at(p.q_layout, st.b, st.hq, si.q0, r0, p.q_sb, p.q_sh, p.q_sn));
+    TL::load(uniform_ptr(src), __builtin_amdgcn_readfirstlane((uint32_t)(dout ? g_.do_sn : p.q_sn) * 4u),
+             si.len - 1 - r0, dst, lane);
   };
   SeqInfo si{};
   QStep cur = mine(steps.first_from(hq_lo, ku.b_lo), si);
   if (cur.hq < hq_hi) {
-    f32x4 qr[C::DS], dr[C::DS];
-    vE qc[4][C::NG], oc[4][C::NG];
-    load_row_frag<D>(q_row(cur, si, cur.p0 + wave * 16 + l16) + 4 * g, qr);
-    load_row_frag<D>(o_row(cur, si, cur.p0 + wave * 16 + l16) + 4 * g, dr);
+    uint32_t qt = base_lds;  // the step's Q tile; its dO tile is the next one
+    load(cur, si, false, qt);
+    load(cur, si, true, qt + TL::BYTES);
     while (true) {
       const int r0 = cur.p0 + wave * 16 + 4 * g;  // rows r0 + r in this lane's accumulators
       float lse[4], dl[4];
@@ -2272,33 +2247,20 @@ __global__ __launch_bounds__(256, F32BwdCfg<D>::WPS) void attn_bwd_dkv_f32_kerne
           dl[r] = st_delta[at + min(r0 + r, si.len - 1)];
         }
       }
-      __builtin_amdgcn_sched_barrier(0);
-      f32x4 sa[KB], dp[KB];
-#pragma unroll
-      for (int kb = 0; kb < KB; ++kb) sa[kb] = dp[kb] = f32x4{0.f, 0.f, 0.f, 0.f};
-      mma_rows<D, KB>(qr, kf, sa);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float* src = q_row(cur, si, r0 + r) + C::E * l16;
-#pragma unroll
-        for (int dg = 0; dg < C::NG; ++dg) qc[r][dg] = *(const vE*)(src + 16 * C::E * dg);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      mma_rows<D, KB>(dr, vf, dp);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float* src = o_row(cur, si, r0 + r) + C::E * l16;
-#pragma unroll
-        for (int dg = 0; dg < C::NG; ++dg) oc[r][dg] = *(const vE*)(src + 16 * C::E * dg);
-      }
       SeqInfo sn = si;
       const QStep nxt = mine(steps.next(cur, si.len), sn);
       const bool more = nxt.hq < hq_hi;
-      const QStep ld = more ? nxt : cur;  // unconditional loads: a branch would lengthen the waits
-      const SeqInfo sl = more ? sn : si;
-      __builtin_amdgcn_sched_barrier(0);
+      const uint32_t qn = C::NBUF == 2 ? base_lds + (qt == base_lds ? 2 * TL::BYTES : 0) : qt;
+      f32x4 sa[KB], dp[KB];
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb) sa[kb] = dp[kb] = f32x4{0.f, 0.f, 0.f, 0.f};
+      wait_loads<0>();
+      if (C::NBUF == 2 && more) {  // during this step's math, into the buffers of the last one
+        load(nxt, sn, false, qn);
+        load(nxt, sn, true, qn + TL::BYTES);
+      }
+      mma_rows<D, KB>(TL::row_base(qt, l16, g), kf, sa);
+      mma_rows<D, KB>(TL::row_base(qt + TL::BYTES, l16, g), vf, dp);
 #pragma unroll
       for (int kb = 0; kb < KB; ++kb) {
         const int key = ku.j0 + kb * 16 + l16;
@@ -2310,19 +2272,21 @@ __global__ __launch_bounds__(256, F32BwdCfg<D>::WPS) void attn_bwd_dkv_f32_kerne
           dp[kb][r] = pv * (dp[kb][r] - dl[r]) * p.scale;
         }
       }
-      mma_cols<D, KB>(qc, dp, dk);
-      __builtin_amdgcn_sched_barrier(0);
-      load_row_frag<D>(q_row(ld, sl, ld.p0 + wave * 16 + l16) + 4 * g, qr);
-      if constexpr (D < 256) load_row_frag<D>(o_row(ld, sl, ld.p0 + wave * 16 + l16) + 4 * g, dr);
-      __builtin_amdgcn_sched_barrier(0);
-      mma_cols<D, KB>(oc, sa, dv);
-      // 256 columns: behind the next S instead, for want of registers
-      if constexpr (D >= 256) load_row_frag<D>(o_row(ld, sl, ld.p0 + wave * 16 + l16) + 4 * g, dr);
+      mma_cols<D, KB>(qt + TL::BYTES, l16, g, sa, dv);
+      if (C::NBUF == 1 && more) {
+        wait_reads();
+        load(nxt, sn, true, qt + TL::BYTES);
+      }
+      mma_cols<D, KB>(qt, l16, g, dp, dk);
+      wait_reads();
       if (!more) break;
+      if (C::NBUF == 1) load(nxt, sn, false, qt);
+      qt = qn;
       cur = nxt;
       si = sn;
     }
   }
+  __syncthreads();  // the sums below reuse the tiles' memory
 
   // ---- the waves' sums through LDS; with MLA V is K and both gradients are dK's
 #pragma unroll

@@ -245,4 +245,96 @@ FMLM_DEV void dma16_sbase(const char* base, uint32_t off, uint32_t lds) {
 }
 #pragma clang diagnostic pop
 
+// ---- fp32 tiles: 16 rows of D floats in LDS, private to one wave (no barriers: the wave
+// waits for its own loads).  The two fragment forms of the fp32 MFMAs read 16 bytes of 16
+// different rows per 16 lanes (row) or 16E consecutive columns (col); straight from memory
+// a row form load touches 64 cache lines, and the L1 lookups took as long as the MFMAs.
+// Direct loads fill the tile with whole rows instead, its 16-byte chunks swizzled per row
+// so that both forms read it without bank conflicts (D >= 64).
+template <int D>
+struct F32Tile {
+  static constexpr int E = D >= 64 ? 4 : D / 16;  // columns per lane of a col fragment
+  static constexpr int NG = D / (16 * E);         // column groups of 16 E
+  static constexpr int DS = D / 16;               // 16-column steps of a row fragment
+  static constexpr int CPR = D / 4;               // 16-byte chunks per row
+  static constexpr int PITCH = D * 4;
+  static constexpr int BYTES = 16 * PITCH;
+  static constexpr int NL = BYTES / 1024;         // wave-wide direct loads
+  typedef typename FloatN<E>::type vE;
+
+  static FMLM_DEV int swz(int r) { return D >= 64 ? r & 15 : D == 32 ? (r >> 1) & 7 : (r >> 2) & 3; }
+
+  // starts the loads of rows [0, 16) from the wave-uniform row-0 address src at `pitch`
+  // bytes (rows past `last` repeat row `last`) into the tile at LDS byte address lds
+  static FMLM_DEV void load(const char* src, uint32_t pitch, int last, uint32_t lds, int lane) {
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      const int at = i * 64 + lane, r = at / CPR;
+      dma16_sbase(src, (uint32_t)min(r, last) * pitch + 16u * (uint32_t)((at % CPR) ^ swz(r)),
+                  __builtin_amdgcn_readfirstlane(lds + i * 1024));
+    }
+  }
+  // the lane's address of row fragment 0 in the tile at LDS address lds (a multiple of 256)
+  static FMLM_DEV uint32_t row_base(uint32_t lds, int l16, int g) { return lds + l16 * PITCH + 16 * (g ^ swz(l16)); }
+  static FMLM_DEV f32x4 row(uint32_t base, int ds) {  // columns 16ds + 4g .. +4 of row l16
+    return *(const FMLM_LDS f32x4*)(uintptr_t)((base ^ (64 * (ds & 3))) + 256 * (ds >> 2));
+  }
+  static FMLM_DEV vE col(uint32_t lds, int l16, int g, int r, int dg) {  // columns E (l16 + 16dg) .. of row 4g + r
+    const int R = 4 * g + r;
+    const uint32_t a = lds + R * PITCH + 16 * ((E * l16 / 4) ^ swz(R)) + 4 * (E * l16 % 4) + 256 * dg;
+    return *(const FMLM_LDS vE*)(uintptr_t)a;
+  }
+};
+
+// acc[i] += A B over the columns: A's row fragments from the tile (row_base), B's in b[i]
+template <int D, int N>
+FMLM_DEV void mma_rows(uint32_t base, const f32x4 (&b)[N][D / 16], f32x4 (&acc)[N]) {
+#pragma unroll
+  for (int ds = 0; ds < D / 16; ++ds) {
+    const f32x4 a = F32Tile<D>::row(base, ds);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int i = 0; i < N; ++i) acc[i] = mfma_f32(a[e], b[i][ds][e], acc[i]);
+  }
+}
+// o[i] += X^T b[i] over the tile's 16 rows X: row 4g + r against b[i][r]
+template <int D, int N>
+FMLM_DEV void mma_cols(uint32_t lds, int l16, int g, const f32x4 (&b)[N], f32x4 (&o)[N][F32Tile<D>::NG][F32Tile<D>::E]) {
+  typedef F32Tile<D> C;
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int dg = 0; dg < C::NG; ++dg) {
+      const typename C::vE x = C::col(lds, l16, g, r, dg);
+#pragma unroll
+      for (int e = 0; e < C::E; ++e)
+#pragma unroll
+        for (int i = 0; i < N; ++i) o[i][dg][e] = mfma_f32(elem_of<C::E>(x, e), b[i][r], o[i][dg][e]);
+    }
+}
+// the lane's columns of accumulator o (row l16 of its block) to a row of floats
+template <int D>
+FMLM_DEV void store_cols(const f32x4 (&o)[F32Tile<D>::NG][F32Tile<D>::E], float* row, int g) {
+  typedef F32Tile<D> C;
+#pragma unroll
+  for (int dg = 0; dg < C::NG; ++dg)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      typename C::vE x;
+      if constexpr (C::E == 1) x = o[dg][0][r];
+      else
+#pragma unroll
+        for (int e = 0; e < C::E; ++e) x[e] = o[dg][e][r];
+      *(typename C::vE*)(row + 4 * C::E * g + 16 * C::E * dg + C::E * r) = x;
+    }
+}
+// at most N of this wave's direct loads are still in flight
+template <int N>
+FMLM_DEV void wait_loads() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+// this wave's LDS reads are done: their tile may be loaded over
+FMLM_DEV void wait_reads() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
 }  // namespace fmlm
