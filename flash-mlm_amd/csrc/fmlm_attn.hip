@@ -2550,7 +2550,7 @@ static Launch mfma3_launch(bool paged) {
   }
   Launch L{C::BQ, C::NT, C::LDS_BYTES, fn, true, false, true};
   // D = 64: 0.6 / 0.8 us with one / two row blocks per wave, D = 128: 0.86 / 1.12, D = 256: 1.7
-  L.tile_us = QB == 2 ? 0.48f + 0.005f * D : D <= 128 ? 0.34f + 0.0041f * D : 1.7f;
+  L.tile_us = QB == 2 ? 0.55f + 0.0045f * D : D <= 128 ? 0.34f + 0.0041f * D : 1.7f;
   return L;
 }
 
