@@ -2058,9 +2058,10 @@ __global__ __launch_bounds__(MlaRowsCfg::NT, 1) void attn_mla_rows_kernel(
 //                                e builds the columns E*i + e (i < 16) of a 16E-wide group
 // so a lane ends up with 4E consecutive columns of O per group.
 // The next tile's K is loaded (F32Tile) once this tile's S has read the buffer, V once its
-// P V has: each has the other product's time.  8 x 12 heads x 512 x 512, D = 64: 70.7 us, 91
-// TFLOP/s (D = 128: 96; a library fp32 product reaches 154); with fragments straight from
-// L1 / L2 73.5; the SIMT kernel below ran at 13 TFLOP/s.
+// P V has: each has the other product's time.  What the matrix cores lose besides is VALU
+// work, which they do not hide.  8 x 12 heads x 512 x 512, D = 64: 68.5 us, 94 TFLOP/s (D =
+// 128: 95; a library fp32 product reaches 154); with fragments straight from L1 / L2 73.5;
+// the SIMT kernel below ran at 13 TFLOP/s.
 // ---------------------------------------------------------------------------
 template <int D, int QB>
 struct F32Cfg {
@@ -2073,7 +2074,7 @@ struct F32Cfg {
   static constexpr int TILES = NW * 2 * F32Tile<D>::BYTES;  // a K and a V tile per wave
   static constexpr int SUMS = NW * BQ * (OP + 2) * 4;       // the waves' sums, after the loop
   static constexpr int LDS_BYTES = TILES > SUMS ? TILES : SUMS;
-  // waves per SIMD: the fragments of 256 columns take more than 256 registers
+  // waves per SIMD: 256 columns of two row blocks take more than 256 registers
   static constexpr int WPS = D >= 256 ? 1 : 2;
   static_assert(BK == NW * 16, "16 keys of a tile per wave");
 };
@@ -2093,7 +2094,10 @@ __global__ __launch_bounds__(256, (F32Cfg<D, QB>::WPS)) void attn_f32_kernel(
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, g = lane >> 4;
-  const float c = p.scale * kLog2e;
+  // scores in log2 units: c * s, a negative scale in Q's sign (the floor keeps -inf * c ==
+  // -inf for masked keys at scale 0)
+  const float qsign = p.scale < 0.f ? -1.f : 1.f;
+  const float c = fmaxf(fabsf(p.scale) * kLog2e, 1e-30f);
 
   f32x4 q[QB][C::DS];
 #pragma unroll
@@ -2102,7 +2106,7 @@ __global__ __launch_bounds__(256, (F32Cfg<D, QB>::WPS)) void attn_f32_kernel(
     const float* src = (const float*)p.q + w.q_row0 + (int64_t)row * w.q_sn + 4 * g;
 #pragma unroll
     for (int ds = 0; ds < C::DS; ++ds)
-      q[qb][ds] = row < w.qcount ? *(const f32x4*)(src + 16 * ds) : f32x4{0.f, 0.f, 0.f, 0.f};
+      q[qb][ds] = row < w.qcount ? *(const f32x4*)(src + 16 * ds) * qsign : f32x4{0.f, 0.f, 0.f, 0.f};
   }
 
   const int n0 = w.seg[0].n, n1 = w.seg[1].n;
@@ -2126,13 +2130,18 @@ __global__ __launch_bounds__(256, (F32Cfg<D, QB>::WPS)) void attn_f32_kernel(
   // check_params); rows past the segment's end repeat its last row, their scores are masked
   typedef F32Tile<D> TL;
   const uint32_t kt = lds_addr(smem_raw) + wave * 2 * TL::BYTES, vt = kt + TL::BYTES;
+  uint32_t off[TL::NL];  // whole tiles at the main keys' pitch (mostly every tensor's)
+  const uint32_t pitch0 = __builtin_amdgcn_readfirstlane((uint32_t)w.seg[1].ksn * 4u);
+  TL::offsets(pitch0, lane, off);
   auto load = [&](int t, bool v) {
     const bool cx = t < nt0;
     const int64_t sn = cx ? (v ? w.seg[0].vsn : w.seg[0].ksn) : (v ? w.seg[1].vsn : w.seg[1].ksn);
     const float* base = cx ? (v ? vp0 : kp0) : (v ? vp1 : kp1);
     const int j0 = key0(t);
-    TL::load(uniform_ptr((const char*)(base + (uint64_t)(uint32_t)j0 * (uint32_t)sn)),
-             __builtin_amdgcn_readfirstlane((uint32_t)sn * 4u), nkeys(t) - 1 - j0, v ? vt : kt, lane);
+    const char* src = uniform_ptr((const char*)(base + (uint64_t)(uint32_t)j0 * (uint32_t)sn));
+    const uint32_t pitch = __builtin_amdgcn_readfirstlane((uint32_t)sn * 4u);
+    if (pitch == pitch0 && nkeys(t) - j0 >= 16) TL::load_at(src, off, v ? vt : kt);
+    else TL::load(src, pitch, nkeys(t) - 1 - j0, v ? vt : kt, lane);
   };
 
   f32x4 o[QB][C::NG][C::E];
@@ -2154,27 +2163,32 @@ __global__ __launch_bounds__(256, (F32Cfg<D, QB>::WPS)) void attn_f32_kernel(
     load(t, true);
     while (t < end) {
       f32x4 s[QB];
-#pragma unroll
-      for (int qb = 0; qb < QB; ++qb) s[qb] = f32x4{0.f, 0.f, 0.f, 0.f};
       wait_loads<TL::NL>();  // K (V's loads came later)
       mma_rows<D, QB>(krow, q, s);
-      const int lim = nkeys(t) - key0(t) - 4 * g;  // key 4g + r is valid iff r < lim
+      const int nk = nkeys(t) - key0(t);  // this wave's valid keys
       const int tn = from(t + 1);
       const int tl = tn < end ? tn : t;  // past the end: once more, unused
       wait_reads();
       load(tl, false);
+      if (nk < 16) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (4 * g + r >= nk)
+#pragma unroll
+            for (int qb = 0; qb < QB; ++qb) s[qb][r] = -INFINITY;
+      }
+      float mx[QB];  // the lane's largest score of the row
       bool grow = false;
 #pragma unroll
       for (int qb = 0; qb < QB; ++qb) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) s[qb][r] = r < lim ? s[qb][r] * c : -INFINITY;
-        grow |= fmaxf(fmaxf(s[qb][0], s[qb][1]), fmaxf(s[qb][2], s[qb][3])) > m_i[qb] + kRescaleSlack;
+        mx[qb] = fmaxf(fmaxf(s[qb][0], s[qb][1]), fmaxf(s[qb][2], s[qb][3])) * c;
+        grow |= mx[qb] > m_i[qb] + kRescaleSlack;
       }
       if (__builtin_amdgcn_ballot_w64(grow)) {  // lazy rescale (kRescaleSlack)
 #pragma unroll
         for (int qb = 0; qb < QB; ++qb) {
-          const float mx = lane_max_xor16_32(fmaxf(fmaxf(s[qb][0], s[qb][1]), fmaxf(s[qb][2], s[qb][3])));
-          const float m_new = mx > m_i[qb] + kRescaleSlack ? mx : m_i[qb];
+          const float top = lane_max_xor16_32(mx[qb]);
+          const float m_new = top > m_i[qb] + kRescaleSlack ? top : m_i[qb];
           const float alpha = m_new == m_i[qb] ? 1.f : fast_exp2(m_i[qb] - m_new);
           m_i[qb] = m_new;
           l_i[qb] *= alpha;
@@ -2186,8 +2200,9 @@ __global__ __launch_bounds__(256, (F32Cfg<D, QB>::WPS)) void attn_f32_kernel(
       }
 #pragma unroll
       for (int qb = 0; qb < QB; ++qb) {
+        const float mref = m_i[qb] == -INFINITY ? 0.f : m_i[qb];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) s[qb][r] = fast_exp2(s[qb][r] - (m_i[qb] == -INFINITY ? 0.f : m_i[qb]));
+        for (int r = 0; r < 4; ++r) s[qb][r] = fast_exp2(fmaf(s[qb][r], c, -mref));
         l_i[qb] += (s[qb][0] + s[qb][1]) + (s[qb][2] + s[qb][3]);
       }
       wait_loads<TL::NL>();  // V (the next K's loads came later)
@@ -2669,8 +2684,8 @@ static bool pick_simt(int D, Launch& L) {
 }
 
 // fp32 on the matrix cores, D <= 256: the widest query tile whose fragments fit two waves
-// per SIMD (wide tiles read each key fewer times: 8 x 12 heads x 512, D = 128, 141 us with
-// 32-row tiles, 172 with 16).  A small batch takes 16-row tiles, twice the workgroups: at
+// per SIMD, one at D = 256 (wide tiles read each key fewer times: 8 x 12 heads x 512, D =
+// 128, 141 us with 32-row tiles, 172 with 16; 8 x 8, D = 256, 224 and 240).  A small batch takes 16-row tiles, twice the workgroups: at
 // D = 64 below 256 tiles of 32 rows (2 x 8 heads x 128: 6.4 us); at D = 128 below 64, since
 // long contexts split anyway and wide tiles then merge less (4 x 8 x 100 queries, 1000
 // context rows: 32 us against 38).
@@ -2683,7 +2698,7 @@ static bool pick_f32(const fmlm_attn_params& p, Launch& L) {
     case 32: L = f32_launch<32, 2>(); return true;
     case 64: L = small ? f32_launch<64, 1>() : f32_launch<64, 2>(); return true;
     case 128: L = small ? f32_launch<128, 1>() : f32_launch<128, 2>(); return true;
-    case 256: L = f32_launch<256, 1>(); return true;
+    case 256: L = small ? f32_launch<256, 1>() : f32_launch<256, 2>(); return true;
     default: return false;
   }
 }

@@ -1947,7 +1947,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkv_simt_kernel(const fmlm_attn_
 // columns, contracted over the rows), both from one load of the tile.
 // The 4 waves of a workgroup split the contraction's long side (dq: 16 keys of every 64;
 // dK / dV: 16 query rows of every 64) and add their sums up through LDS at the end.  8 x 12
-// heads x 512 x 512: 240 us at D = 64 (67 TFLOP/s of 5 products, 94 of the 7 computed), 457
+// heads x 512 x 512: 239 us at D = 64 (67 TFLOP/s of 5 products, 94 of the 7 computed), 449
 // at D = 128; with fragments straight from L1 / L2 275 and 602 us.
 // ---------------------------------------------------------------------------
 template <int D>
@@ -1957,7 +1957,7 @@ struct F32BwdCfg {
   static constexpr int OP = D + 4;  // LDS row pitch of the sums (floats)
   // 16-row query blocks of a dq workgroup, 16-key blocks of a dK / dV workgroup: as many as
   // fit two waves per SIMD (8 x 12 heads x 512, D = 64: two of each 275 us; one query block
-  // 292, one key block 306)
+  // 292, one key block 306; D = 256 with two query blocks spills, 742 -> 1057)
   static constexpr int QB = D == 16 ? 4 : D <= 64 ? 2 : 1;
   static constexpr int KB = QB;
   static constexpr int BQ = 16 * QB, KEYS = 16 * KB;
@@ -2007,7 +2007,9 @@ __global__ __launch_bounds__(256, F32BwdCfg<D>::WPS) void attn_bwd_dq_f32_kernel
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, g = lane >> 4;
-  const float c = p.scale * kLog2e;
+  // scores in log2 units: c * s, a negative scale in Q's sign (see attn_f32_kernel)
+  const float qsign = p.scale < 0.f ? -1.f : 1.f;
+  const float c = fmaxf(fabsf(p.scale) * kLog2e, 1e-30f);
 
   f32x4 q[QB][C::DS], dof[QB][C::DS];
   float delta[QB];
@@ -2017,8 +2019,11 @@ __global__ __launch_bounds__(256, F32BwdCfg<D>::WPS) void attn_bwd_dq_f32_kernel
     const float* qp = (const float*)p.q + row_at(p.q_layout, b, h, si.q0, pos, p.q_sb, p.q_sh, p.q_sn) + 4 * g;
     const float* dp = (const float*)g_.dout + row_at(p.o_layout, b, h, si.q0, pos, g_.do_sb, g_.do_sh, g_.do_sn) + 4 * g;
     const float* op = (const float*)p.o + row_at(p.o_layout, b, h, si.q0, pos, p.o_sb, p.o_sh, p.o_sn) + 4 * g;
-    load_row_frag<D>(qp, q[qb]);
-    load_row_frag<D>(dp, dof[qb]);
+#pragma unroll
+    for (int ds = 0; ds < C::DS; ++ds) {
+      q[qb][ds] = *(const f32x4*)(qp + 16 * ds) * qsign;
+      dof[qb][ds] = *(const f32x4*)(dp + 16 * ds);
+    }
     float d = 0.f;
 #pragma unroll
     for (int ds = 0; ds < C::DS; ++ds) {
@@ -2042,14 +2047,19 @@ __global__ __launch_bounds__(256, F32BwdCfg<D>::WPS) void attn_bwd_dq_f32_kernel
   // the loads of this wave's 16 keys of tile t; rows past the segment's end repeat its last
   // row (their scores are masked)
   const uint32_t vt = lds_addr(smem_raw) + wave * (C::NBUF + 1) * TL::BYTES, kt0 = vt + TL::BYTES;
+  uint32_t off[TL::NL];  // whole tiles at the main keys' pitch (mostly every tensor's)
+  const uint32_t pitch0 = __builtin_amdgcn_readfirstlane((uint32_t)sm.ksn * 4u);
+  TL::offsets(pitch0, lane, off);
   auto load = [&](int t, bool v, uint32_t dst) {
     const bool cx = t < nt0;
     const float* base = cx ? (const float*)(v ? sc.v : sc.k) + (v ? sc.vbase : sc.kbase)
                            : (const float*)(v ? sm.v : sm.k) + (v ? sm.vbase : sm.kbase);
     const int64_t sn = cx ? (v ? sc.vsn : sc.ksn) : (v ? sm.vsn : sm.ksn);
     const int j0 = key0(t);
-    TL::load(uniform_ptr((const char*)(base + (uint64_t)(uint32_t)j0 * (uint32_t)sn)),
-             __builtin_amdgcn_readfirstlane((uint32_t)sn * 4u), nkeys(t) - 1 - j0, dst, lane);
+    const char* src = uniform_ptr((const char*)(base + (uint64_t)(uint32_t)j0 * (uint32_t)sn));
+    const uint32_t pitch = __builtin_amdgcn_readfirstlane((uint32_t)sn * 4u);
+    if (pitch == pitch0 && nkeys(t) - j0 >= 16) TL::load_at(src, off, dst);
+    else TL::load(src, pitch, nkeys(t) - 1 - j0, dst, lane);
   };
 
   f32x4 acc[QB][C::NG][C::E];
@@ -2073,8 +2083,6 @@ __global__ __launch_bounds__(256, F32BwdCfg<D>::WPS) void attn_bwd_dq_f32_kernel
       const int tl = tn < end ? tn : t;  // past the end: once more, unused
       const uint32_t kn = C::NBUF == 2 ? kt0 + (kt == kt0 ? TL::BYTES : 0) : kt;
       f32x4 s[QB], dp[QB];
-#pragma unroll
-      for (int qb = 0; qb < QB; ++qb) s[qb] = dp[qb] = f32x4{0.f, 0.f, 0.f, 0.f};
       if constexpr (C::NBUF == 2) {
         wait_loads<TL::NL>();  // K (V's loads came later)
         load(tl, false, kn);   // the buffer that the last tile's dq read
@@ -2087,19 +2095,26 @@ __global__ __launch_bounds__(256, F32BwdCfg<D>::WPS) void attn_bwd_dq_f32_kernel
       mma_rows<D, QB>(TL::row_base(vt, l16, g), dof, dp);
       wait_reads();
       load(tl, true, vt);
-      const int lim = nkeys(t) - key0(t) - 4 * g;  // key 4g + r is valid iff r < lim
+      const int nk = nkeys(t) - key0(t);  // this wave's valid keys
+      if (nk < 16) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (4 * g + r >= nk)
+#pragma unroll
+            for (int qb = 0; qb < QB; ++qb) s[qb][r] = -INFINITY;
+      }
+      float mx[QB];  // the lane's largest score of the row
       bool grow = false;
 #pragma unroll
       for (int qb = 0; qb < QB; ++qb) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) s[qb][r] = r < lim ? s[qb][r] * c : -INFINITY;
-        grow |= fmaxf(fmaxf(s[qb][0], s[qb][1]), fmaxf(s[qb][2], s[qb][3])) > m_i[qb] + kRescaleSlack;
+        mx[qb] = fmaxf(fmaxf(s[qb][0], s[qb][1]), fmaxf(s[qb][2], s[qb][3])) * c;
+        grow |= mx[qb] > m_i[qb] + kRescaleSlack;
       }
       if (__builtin_amdgcn_ballot_w64(grow)) {  // lazy rescale (kRescaleSlack)
 #pragma unroll
         for (int qb = 0; qb < QB; ++qb) {
-          const float mx = lane_max_xor16_32(fmaxf(fmaxf(s[qb][0], s[qb][1]), fmaxf(s[qb][2], s[qb][3])));
-          const float m_new = mx > m_i[qb] + kRescaleSlack ? mx : m_i[qb];
+          const float top = lane_max_xor16_32(mx[qb]);
+          const float m_new = top > m_i[qb] + kRescaleSlack ? top : m_i[qb];
           const float alpha = m_new == m_i[qb] ? 1.f : fast_exp2(m_i[qb] - m_new);
           m_i[qb] = m_new;
           l_i[qb] *= alpha;
@@ -2114,7 +2129,7 @@ __global__ __launch_bounds__(256, F32BwdCfg<D>::WPS) void attn_bwd_dq_f32_kernel
         const float mref = m_i[qb] == -INFINITY ? 0.f : m_i[qb];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          s[qb][r] = fast_exp2(s[qb][r] - mref);
+          s[qb][r] = fast_exp2(fmaf(s[qb][r], c, -mref));
           dp[qb][r] = s[qb][r] * (dp[qb][r] - delta[qb]);
         }
         l_i[qb] += (s[qb][0] + s[qb][1]) + (s[qb][2] + s[qb][3]);
@@ -2221,14 +2236,18 @@ __global__ __launch_bounds__(256, F32BwdCfg<D>::WPS) void attn_bwd_dkv_f32_kerne
   // the loads of this wave's 16 Q (or dO) rows of a step; rows past the sequence's end repeat
   // its last one (their P is 0)
   const uint32_t base_lds = lds_addr(smem_raw) + wave * 2 * C::NBUF * TL::BYTES;
+  uint32_t off[TL::NL];  // whole tiles at Q's pitch (mostly dO's too)
+  const uint32_t pitch0 = __builtin_amdgcn_readfirstlane((uint32_t)p.q_sn * 4u);
+  TL::offsets(pitch0, lane, off);
   auto load = [&](const QStep& st, const SeqInfo& si, bool dout, uint32_t dst) {
     const int r0 = st.p0 + wave * 16;
     const char* src = dout ? (const char*)((const float*)g_.dout + row_at(p.o_layout, st.b, st.hq, si.q0, r0, g_.do_sb,
                                                                           g_.do_sh, g_.do_sn))
                            : (const char*)((const float*)p.q +
                                            row_at(p.q_layout, st.b, st.hq, si.q0, r0, p.q_sb, p.q_sh, p.q_sn));
-    TL::load(uniform_ptr(src), __builtin_amdgcn_readfirstlane((uint32_t)(dout ? g_.do_sn : p.q_sn) * 4u),
-             si.len - 1 - r0, dst, lane);
+    const uint32_t pitch = __builtin_amdgcn_readfirstlane((uint32_t)(dout ? g_.do_sn : p.q_sn) * 4u);
+    if (pitch == pitch0 && si.len - r0 >= 16) TL::load_at(uniform_ptr(src), off, dst);
+    else TL::load(uniform_ptr(src), pitch, si.len - 1 - r0, dst, lane);
   };
   SeqInfo si{};
   QStep cur = mine(steps.first_from(hq_lo, ku.b_lo), si);
@@ -2252,8 +2271,6 @@ __global__ __launch_bounds__(256, F32BwdCfg<D>::WPS) void attn_bwd_dkv_f32_kerne
       const bool more = nxt.hq < hq_hi;
       const uint32_t qn = C::NBUF == 2 ? base_lds + (qt == base_lds ? 2 * TL::BYTES : 0) : qt;
       f32x4 sa[KB], dp[KB];
-#pragma unroll
-      for (int kb = 0; kb < KB; ++kb) sa[kb] = dp[kb] = f32x4{0.f, 0.f, 0.f, 0.f};
       wait_loads<0>();
       if (C::NBUF == 2 && more) {  // during this step's math, into the buffers of the last one
         load(nxt, sn, false, qn);
@@ -2262,16 +2279,21 @@ __global__ __launch_bounds__(256, F32BwdCfg<D>::WPS) void attn_bwd_dkv_f32_kerne
       mma_rows<D, KB>(TL::row_base(qt, l16, g), kf, sa);
       mma_rows<D, KB>(TL::row_base(qt + TL::BYTES, l16, g), vf, dp);
 #pragma unroll
-      for (int kb = 0; kb < KB; ++kb) {
-        const int key = ku.j0 + kb * 16 + l16;
-        const bool kvalid = key < s.n && (!ku.causal_main || key < si.mainlen);
+      for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float pv = kvalid && r0 + r < si.len ? fast_exp2(fmaf(sa[kb][r], c, -lse[r])) : 0.f;
-          sa[kb][r] = pv;
-          dp[kb][r] = pv * (dp[kb][r] - dl[r]) * p.scale;
-        }
+        for (int r = 0; r < 4; ++r) sa[kb][r] = fast_exp2(fmaf(sa[kb][r], c, -lse[r]));
+      const int kend = ku.causal_main ? min(s.n, si.mainlen) : s.n;  // keys this step's rows see
+      if (cur.p0 + wave * 16 + 16 > si.len || ku.j0 + C::KEYS > kend) {
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (ku.j0 + kb * 16 + l16 >= kend || r0 + r >= si.len) sa[kb][r] = 0.f;
       }
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) dp[kb][r] = sa[kb][r] * (dp[kb][r] - dl[r]) * p.scale;
       mma_cols<D, KB>(qt + TL::BYTES, l16, g, sa, dv);
       if (C::NBUF == 1 && more) {
         wait_reads();

@@ -274,6 +274,19 @@ struct F32Tile {
                   __builtin_amdgcn_readfirstlane(lds + i * 1024));
     }
   }
+  // the lane's offsets of a whole tile at `pitch`, and its loads with them: a load's offset
+  // otherwise takes four VALU instructions, which the fp32 MFMAs do not hide (below)
+  static FMLM_DEV void offsets(uint32_t pitch, int lane, uint32_t (&off)[NL]) {
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      const int at = i * 64 + lane, r = at / CPR;
+      off[i] = (uint32_t)r * pitch + 16u * (uint32_t)((at % CPR) ^ swz(r));
+    }
+  }
+  static FMLM_DEV void load_at(const char* src, const uint32_t (&off)[NL], uint32_t lds) {
+#pragma unroll
+    for (int i = 0; i < NL; ++i) dma16_sbase(src, off[i], __builtin_amdgcn_readfirstlane(lds + i * 1024));
+  }
   // the lane's address of row fragment 0 in the tile at LDS address lds (a multiple of 256)
   static FMLM_DEV uint32_t row_base(uint32_t lds, int l16, int g) { return lds + l16 * PITCH + 16 * (g ^ swz(l16)); }
   static FMLM_DEV f32x4 row(uint32_t base, int ds) {  // columns 16ds + 4g .. +4 of row l16
@@ -286,16 +299,31 @@ struct F32Tile {
   }
 };
 
-// acc[i] += A B over the columns: A's row fragments from the tile (row_base), B's in b[i]
+// acc[i] = A B over the columns: A's row fragments from the tile (row_base), B's in b[i].
+// Several sums side by side from 64 columns on, so that a score's rounding error does not
+// grow with the whole row (one chain of 128 columns: error of the output against 64 bits up
+// to 1.2 times that of 16 partial sums, the SIMT kernels').
 template <int D, int N>
 FMLM_DEV void mma_rows(uint32_t base, const f32x4 (&b)[N][D / 16], f32x4 (&acc)[N]) {
+  constexpr int NC = D >= 128 ? 4 : D == 64 ? 2 : 1;
+  f32x4 part[NC][N];
+#pragma unroll
+  for (int n = 0; n < NC; ++n)
+#pragma unroll
+    for (int i = 0; i < N; ++i) part[n][i] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int ds = 0; ds < D / 16; ++ds) {
     const f32x4 a = F32Tile<D>::row(base, ds);
 #pragma unroll
     for (int e = 0; e < 4; ++e)
 #pragma unroll
-      for (int i = 0; i < N; ++i) acc[i] = mfma_f32(a[e], b[i][ds][e], acc[i]);
+      for (int i = 0; i < N; ++i) part[ds % NC][i] = mfma_f32(a[e], b[i][ds][e], part[ds % NC][i]);
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    if constexpr (NC == 4) acc[i] = (part[0][i] + part[1][i]) + (part[2][i] + part[3][i]);
+    else if constexpr (NC == 2) acc[i] = part[0][i] + part[1][i];
+    else acc[i] = part[0][i];
   }
 }
 // o[i] += X^T b[i] over the tile's 16 rows X: row 4g + r against b[i][r]
