@@ -135,3 +135,47 @@ def test_split_launches_of_one_schedule_do_not_share_partial_results(device):
     for i in range(2):
         for g in got[i]:
             assert torch.equal(g, want[i])
+
+
+@pytest.mark.parametrize("way", ["dense", "latent"])
+def test_split_call_in_a_graph(way, device):
+    """A captured call that splits (its records come from the graph's own memory) replays to
+    the eager result, with other calls between the replays."""
+    gen = torch.Generator().manual_seed(12)
+    cache, dtype = InferenceCache(), torch.bfloat16
+    if way == "dense":
+        H, D, C = 2, 128, 3000
+        q, k, v = (_randn(gen, (1, H, 20, D), dtype, device) for _ in range(3))
+        kc, vc = (_randn(gen, (H * C, D), dtype, device) for _ in range(2))
+        cache.prefill_kv_cache(0, k_cache=kc, v_cache=vc, context_batch_size=1, is_mla=False, num_heads=H, head_dim=D)
+
+        def call():
+            return flash_attn_mlm(q, k, v, 0.1, inference_cache=cache, layer_id=0)
+    else:
+        B, H, D, C = 2, 16, 512, 1500
+        q, k = (_randn(gen, (B, H, 3, D), dtype, device, 0.5) for _ in range(2))
+        kc = _randn(gen, (B * C, D), dtype, device, 0.5)
+        cu = torch.arange(B + 1, dtype=torch.int32, device=device) * C
+        cache.prefill_kv_cache(0, k_cache=kc, total_context_len=B * C, cu_seqlens_kv=cu, context_batch_size=B,
+                               is_mla=True, num_heads=H, head_dim=D)
+        meta = build_pack_metadata(torch.tensor([3, 1], dtype=torch.int32, device=device), 3, 64)
+
+        def call():
+            return flash_attn_mlm_compressed(q, k, k, H, meta, 0.05, cache, 0, is_mla=True, block_n=64)
+
+    want = call()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        call()
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = call()
+    for _ in range(4):
+        out.zero_()
+        graph.replay()
+        eager = call()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want) and torch.equal(eager, want)
