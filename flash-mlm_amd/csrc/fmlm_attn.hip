@@ -2823,7 +2823,10 @@ static SplitCfg split_cfg(const fmlm_attn_params& p, const Launch& L) {
   // schedule cannot split (and no records or merge launch are needed)
   const int64_t min_units = L.hpack ? ((int64_t)p.H * p.total_q - (int64_t)p.B * L.bq) / L.bq
                                     : (int64_t)p.H * (((int64_t)p.total_q - (int64_t)p.B * L.bq) / L.bq);
-  if (min_units >= (int64_t)(kSplitRounds * sc.slots)) return SplitCfg{};
+  // (the latent kernel, in whole rounds, gains nothing from half a round on, and its split
+  // variant is the slower one per tile: 64 heads x 362 queries over 2431 latent rows, 181
+  // tiles, 148 us, 159 with the variant that may split)
+  if (min_units >= (L.hpack ? sc.slots / 2 : (int64_t)(kSplitRounds * sc.slots))) return SplitCfg{};
   sc.rec_cap = 3 * sc.slots;
   // The latent kernel: one or two whole rounds (see schedule_kernel), by the most units there
   // can be.  16 sequences of 1-4 tokens, 64 heads, 1400-7800 latent rows each: 22 tiles of
