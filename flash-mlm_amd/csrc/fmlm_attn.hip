@@ -2409,6 +2409,10 @@ __global__ __launch_bounds__(SimtCfg<D>::NT) void attn_simt_kernel(
 // ---------------------------------------------------------------------------
 constexpr int kMergeRows = 128;  // largest split-capable query tile
 constexpr int kMergeThreads = 256;
+// Past this many chunks (8 blocks on each CU) a chunk takes twice the rows: the chain of loads
+// in front of a chunk's rows then costs more than blocks add.  8 sequences x 16 heads of up to 600
+// tokens, D = 128: the call 77 us with 16-row chunks throughout, 75 us so (1024 and 512: the same).
+constexpr int kMergeItems = 2048;
 // rows per chunk (at most one per thread / 8)
 __host__ __device__ inline int merge_chunk(int D) { return D <= 64 ? 32 : 2048 / D; }
 
@@ -2435,20 +2439,40 @@ FMLM_DEV void store8(char* dst, const f32x4& a0, const f32x4& a1) {
   }
 }
 
+// a0, a1 += 8 columns of N consecutive records from src, with the weights w
+template <int N>
+FMLM_DEV void merge_parts(const char* src, int64_t rec_bytes, const float* w, f32x4& a0, f32x4& a1) {
+  f32x4 x0[N], x1[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    x0[i] = *(const f32x4*)(src + i * rec_bytes);
+    x1[i] = *(const f32x4*)(src + i * rec_bytes + 16);
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    a0 += w[i] * x0[i];
+    a1 += w[i] * x1[i];
+  }
+}
+
 template <typename T>
 __global__ __launch_bounds__(kMergeThreads) void merge_kernel(const fmlm_attn_params p, int BQ,
                                                     const int32_t* __restrict__ header, const SplitArgs spa,
                                                     int hpack) {
-  __shared__ float s_w[32][kMaxSplits];  // per row: part weights / their sum
-  __shared__ int64_t s_o[32];            // per row: element offset of its output row
+  __shared__ float s_w[kMergeRows][kMaxSplits];  // per row: part weights / their sum
+  __shared__ int64_t s_o[kMergeRows];            // per row: element offset of its output row
   const int nt = (p.N + BQ - 1) / BQ;  // dense: tiles per (sequence, head)
   const int n_groups = header ? ldc(header, kHdrGroups) : p.B * p.H * nt;
-  const int chunks = merge_chunks(p, BQ, hpack);
+  int chunks = merge_chunks(p, BQ, hpack), chunk = merge_chunk(p.D);
+  while (chunks > 1 && chunk * 2 <= kMergeRows && n_groups * chunks > kMergeItems) {
+    chunk *= 2;
+    chunks = (chunks + 1) / 2;
+  }
   const int64_t rec_bytes = spa.rec_bytes;
   const int D = p.D;
   const int64_t ml_off = (int64_t)BQ * D * 4;
   for (int wi = blockIdx.x; wi < n_groups * chunks; wi += gridDim.x) {
-    const int gi = wi / chunks, r0 = (wi % chunks) * merge_chunk(D);
+    const int gi = wi / chunks, r0 = (wi % chunks) * chunk;
     int b, h, tile, S, first;
     if (header) {
       const int4 gr = ldc4((const int4*)((const char*)header + ldc(header, kHdrGroupsOff)), gi);
@@ -2458,7 +2482,7 @@ __global__ __launch_bounds__(kMergeThreads) void merge_kernel(const fmlm_attn_pa
     }
     if (b < 0 || b >= p.B || h >= p.H) continue;
     const SeqInfo si = seq_info(p, b);
-    const int rows = min(min(BQ, (hpack ? p.H : 1) * si.len - tile * BQ) - r0, merge_chunk(D));
+    const int rows = min(min(BQ, (hpack ? p.H : 1) * si.len - tile * BQ) - r0, chunk);
     if (rows <= 0) continue;
     const char* rec0 = split_record(header, spa, first);
     if (!rec0) return;
@@ -2498,22 +2522,18 @@ __global__ __launch_bounds__(kMergeThreads) void merge_kernel(const fmlm_attn_pa
       const int row = idx / (D / 8), c8 = idx - row * (D / 8);
       const char* src = rec0 + ((int64_t)(r0 + row) * D + c8 * 8) * 4;
       f32x4 a0 = f32x4{0.f, 0.f, 0.f, 0.f}, a1 = a0;
-      // eight parts' loads in flight (the last part's again past the end, at weight 0)
-      for (int s0 = 0; s0 < S; s0 += 8) {
-        f32x4 x0[8], x1[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const char* at = src + min(s0 + i, S - 1) * rec_bytes;
-          x0[i] = *(const f32x4*)at;
-          x1[i] = *(const f32x4*)(at + 16);
-        }
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const float ws = s0 + i < S ? s_w[row][s0 + i] : 0.f;
-          a0 += ws * x0[i];
-          a1 += ws * x1[i];
-        }
+      // up to eight parts' loads in flight
+      int s0 = 0;
+      for (; s0 + 8 <= S; s0 += 8) merge_parts<8>(src + s0 * rec_bytes, rec_bytes, &s_w[row][s0], a0, a1);
+      if (S & 4) {
+        merge_parts<4>(src + s0 * rec_bytes, rec_bytes, &s_w[row][s0], a0, a1);
+        s0 += 4;
       }
+      if (S & 2) {
+        merge_parts<2>(src + s0 * rec_bytes, rec_bytes, &s_w[row][s0], a0, a1);
+        s0 += 2;
+      }
+      if (S & 1) merge_parts<1>(src + s0 * rec_bytes, rec_bytes, &s_w[row][s0], a0, a1);
       store8<T>((char*)p.o + (s_o[row] + c8 * 8) * (int64_t)sizeof(T), a0, a1);
     }
     __syncthreads();  // s_w is rewritten for the next chunk
