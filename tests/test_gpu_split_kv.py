@@ -74,6 +74,7 @@ def test_dense_split_matches_oracle_and_unsplit(B, H, N, D, C, cbs, dtype, devic
     (64, [1, 0, 4, 2], [2000, 900, 0, 5]),       # tiles of 64, 128 and 256 rows, short and empty contexts
     (16, [3], [4097]),                           # one tile, the most parts
     (5, [7, 1, 30], [333, 1024, 64 * 9]),        # odd heads: rows of a tile span heads
+    (32, [4, 3] * 40, [640, 517] * 40),          # many groups: the merge takes larger chunks
 ])
 def test_latent_split_matches_oracle(H, lengths, ctx, paged, device):
     gen = torch.Generator().manual_seed(H)
