@@ -21,6 +21,7 @@
 // fp32 inputs have a kernel of their own on the fp32 MFMA (attn_f32_kernel); head dims
 // without an MFMA instantiation use a SIMT kernel with the same addressing.
 #include "fmlm_common.h"
+#include "fmlm_split_plan.h"
 
 #include <algorithm>
 #include <cmath>
@@ -48,7 +49,8 @@ namespace fmlm {
 // is a spare and takes, by its rank among the spares, one of the entries past G_y of the
 // queues y that hold more than G_y (see workgroup_unit).  Placements keep the queues
 // about equally long, so overflow entries are few and most spares exit at once.
-// Head-packed launches run 8 * cap workgroups (every entry its static workgroup's).
+// Head-packed launches that cannot split run 8 * cap workgroups (every entry its static
+// workgroup's, see spread_by_queue).
 //
 // Split-KV: when the units would fill the GPU's workgroup slots for fewer than
 // kSplitRounds rounds, each query tile's key range is cut into S parts (a split group);
@@ -63,16 +65,10 @@ namespace fmlm {
 // bytes, queue capacity, queue lengths), the queues at 256, then the
 // group list (int4: b, h | tile << 16, first record, S), then the records.
 // ---------------------------------------------------------------------------
-constexpr int kXcds = 8;
 constexpr int kSchedThreads = 512;  // one wave per XCD
 constexpr int kSortMax = 2048;      // sequences ordered longest-first up to this many
 constexpr int kSplitBK = 64;        // key tile of the split-capable kernel
-constexpr int kMaxSplits = 16;
-constexpr int kMinSplitTiles = 8;   // key tiles per part at least
-constexpr int kMinDenseTiles = 4;   // the same for a dense call's parts
-constexpr float kSplitRounds = 1.5f;
-constexpr int kMinHpackTiles = 4;      // head-packed: key tiles per part at least
-constexpr float kHpackPartCost = 4.f;  // and a part's start, end and merge, in key tiles
+constexpr int kMinDenseTiles = 4;   // key tiles per part of a dense call at least
 // schedule header fields (int32 index)
 constexpr int kHdrUnits = 0;      // units in all queues
 constexpr int kHdrGroups = 1;     // split groups
@@ -137,46 +133,24 @@ __global__ __launch_bounds__(kSchedThreads) void schedule_kernel(const fmlm_attn
     }
     __syncthreads();
     // split only when the units are too few to fill the slots for kSplitRounds rounds and
-    // the longest key range has more than split_min tiles (split_min_tiles);
-    // parts of about total / (kSplitRounds * slots) key tiles, at least kMinSplitTiles,
-    // the part size doubling until the records fit
+    // the longest key range has more than split_min tiles (split_min_tiles), in parts of
+    // seq_chunk key tiles; head-packed calls take the cheapest of hpack_price's plans (lane
+    // S - 1 prices S parts)
     if (hpack) {
-      // Head-packed tiles fill a CU each (128 KiB of LDS), so parts run in whole rounds of
-      // `slots`: lane S - 1 prices S parts for the longest sequence (the others' parts as
-      // long) as rounds x (key tiles of a part + what a part costs besides), and the
-      // cheapest is taken.
       if (tid < 64 && rec_cap > 0 && s_sum[0] < kSplitRounds * slots) {
-        const float kmax = (float)s_kmax;
-        const float chunk = fmaxf((float)kMinHpackTiles, ceilf(kmax / (tid + 1)));
-        float parts = 0.f;
-        for (int b = 0; b < B; ++b) {
-          const float S = fminf(kMaxSplits, fmaxf(1.f, ceilf(s_work[b] / chunk)));
-          parts += s_tiles[b] * S;
-        }
-        float cost = ceilf(parts / slots) * (chunk + kHpackPartCost);
-        if (parts > (float)rec_cap || tid >= kMaxSplits) cost = INFINITY;  // a record per part
-        float best = cost;
+        const HpackPrice r = hpack_price(s_tiles, s_work, B, s_kmax, tid + 1, slots, rec_cap);
+        float best = r.cost;
 #pragma unroll
         for (int off = 1; off < 64; off <<= 1) best = fminf(best, __shfl_xor(best, off));
-        if (cost == best && chunk < kmax) atomicMax(&s_chunk, (int)chunk);
+        const int chunk = hpack_take(r, best, s_kmax);
+        if (chunk > 0) atomicMax(&s_chunk, chunk);
       }
     } else if (tid == 0 && rec_cap > 0 && s_sum[0] < kSplitRounds * slots && s_kmax > split_min) {
-      int chunk = max(kMinSplitTiles, (int)ceilf(s_sum[1] / (kSplitRounds * slots)));
-      for (int it = 0; it < 24; ++it, chunk *= 2) {
-        float recs = 0.f;
-        for (int b = 0; b < B; ++b) {
-          const int S = min(kMaxSplits, max(1, (int)ceilf(s_work[b] / chunk)));
-          if (S > 1) recs += (float)s_tiles[b] * (hpack ? 1 : H) * S;
-        }
-        if (recs <= (float)rec_cap) {
-          s_chunk = chunk;
-          break;
-        }
-      }
+      s_chunk = seq_chunk(s_tiles, s_work, B, H, s_sum[1], slots, rec_cap);
     }
     __syncthreads();
     for (int b = tid; b < B; b += kSchedThreads) {
-      const int S = s_chunk > 0 ? min(kMaxSplits, max(1, (int)ceilf(s_work[b] / s_chunk))) : 1;
+      const int S = s_chunk > 0 ? split_parts(s_work[b], s_chunk) : 1;
       s_split[b] = (unsigned char)S;
       // longest unit first (key tiles per part), then more tiles first
       s_work[b] = ceilf(s_work[b] / S) * 65536.f + (float)s_tiles[b];
@@ -2778,15 +2752,6 @@ static int resident_slots(const Launch& L) {
   return slots;
 }
 
-// Split-KV sizing: the GPU's workgroup slots for this kernel, the record capacity and
-// the record size.
-struct SplitCfg {
-  int slots = 0;
-  int rec_cap = 0;        // 0: no split
-  int64_t rec_bytes = 0;  // per record: rows x (D fp32 + m + l)
-  int dense_parts = 1;    // dense call: parts per query tile
-};
-
 // Key ranges of up to this many tiles are not split: two parts save half of them, the merge
 // costs 5 us and its launch's gap, so 20 us of key tiles (bf16 D = 128, 20 sequences of
 // 40-100 queries, 8 heads, 500-1000 context rows: 30 us whole, 34 in two).
@@ -2864,20 +2829,6 @@ static int64_t dense_units(const fmlm_attn_params& p, int bq, int parts) {
   return (int64_t)kXcds * (((int64_t)p.B * p.H + kXcds - 1) / kXcds) * ((p.N + bq - 1) / bq) * parts;
 }
 
-// Entries per queue of a packed call: a bound on the launch's units, so that one queue
-// can take all of them whatever the placement.  Sequence b has ceil(L_b / bq) <= L_b / bq
-// + 1 query tiles per head (head-packed: ceil(H L_b / bq) in all); with splits, which
-// happen only below kSplitRounds * slots unsplit units, add every split part.
-static int64_t queue_cap(const fmlm_attn_params& p, int bq, const SplitCfg& sc, bool hpack) {
-  int64_t units = hpack ? ((int64_t)p.H * p.total_q + bq - 1) / bq + p.B
-                        : (int64_t)p.H * (((int64_t)p.total_q + bq - 1) / bq + p.B);
-  if (sc.rec_cap > 0) {
-    const int64_t split_units = std::min(units, (int64_t)(kSplitRounds * sc.slots) + 1) + sc.rec_cap;
-    units = split_units > units ? split_units : units;
-  }
-  return units;
-}
-
 // Head-packed launches that cannot split run every queue entry on its own XCD (8 * cap
 // workgroups): their queues are balanced by work and not by count, and overflow taken onto
 // other XCDs would break the one-latent-per-XCD placement.  One that may split has queues
@@ -2891,23 +2842,6 @@ static int64_t grid_size(const fmlm_attn_params& p, const Launch& L, const Split
   if (!p.cu_seqlens_q) return dense_units(p, L.bq, sc.dense_parts);
   const int64_t cap = queue_cap(p, L.bq, sc, L.hpack);
   return spread_by_queue(L, sc) ? kXcds * cap : cap;
-}
-
-// Schedule buffer layout (see schedule_kernel): header, 8 queues, groups, records.
-struct SchedLayout {
-  int64_t cap, units_off, groups_off, records_off, bytes;
-};
-
-static SchedLayout sched_layout(const fmlm_attn_params& p, int bq, const SplitCfg& sc, bool hpack) {
-  SchedLayout l;
-  l.cap = queue_cap(p, bq, sc, hpack);
-  l.units_off = 256;
-  l.groups_off = l.units_off + kXcds * l.cap * (int64_t)sizeof(int4);
-  l.groups_off = (l.groups_off + 255) / 256 * 256;
-  l.records_off = l.groups_off + (int64_t)sc.rec_cap * (int64_t)sizeof(int4);
-  l.records_off = (l.records_off + 255) / 256 * 256;
-  l.bytes = l.records_off + (int64_t)sc.rec_cap * sc.rec_bytes;
-  return l;
 }
 
 // bytes of the split records of a call (0: it never splits)
@@ -3027,36 +2961,15 @@ static int scratch_on_current_device(char** out) {
 }
 
 // The split sizing of the allocation-free path: as split_cfg, with the record count cut
-// so that the schedule and the records fit the scratch array (no split when fewer than
-// one record per workgroup slot would fit; a dense call's parts are all or none).  Returns
-// false when even the unsplit schedule does not fit.
+// so that the schedule and the records fit the scratch array (fit_records; a dense call's
+// parts are all or none).  Returns false when even the unsplit schedule does not fit.
 static bool split_cfg_within(const fmlm_attn_params& p, const Launch& L, int64_t cap, SplitCfg& sc) {
   sc = split_cfg(p, L);
   if (!p.cu_seqlens_q) {
     if (records_for(sc) > cap) sc = SplitCfg{};
     return true;
   }
-  auto fits = [&](int rec_cap) {
-    SplitCfg t = sc;
-    t.rec_cap = rec_cap;
-    return sched_layout(p, L.bq, t, L.hpack).bytes <= cap;
-  };
-  if (fits(sc.rec_cap)) return true;
-  // the layout grows with the record count: the largest count in [lo, rec_cap) that fits
-  int lo = L.hpack ? 1 : sc.slots, hi = sc.rec_cap - 1;
-  if (sc.rec_cap > 0 && lo <= hi && fits(lo)) {
-    while (lo < hi) {
-      const int mid = lo + (hi - lo + 1) / 2;
-      if (fits(mid))
-        lo = mid;
-      else
-        hi = mid - 1;
-    }
-    sc.rec_cap = lo;
-    return true;
-  }
-  sc.rec_cap = 0;
-  return fits(0);
+  return fit_records(p, L.bq, L.hpack, cap, sc);
 }
 
 }  // namespace fmlm

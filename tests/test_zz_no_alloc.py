@@ -92,3 +92,17 @@ def test_noalloc_dense_and_errors(device):
     p = _lib.AttnParams.from_buffer_copy(plan.params)
     p.D = 48
     assert plan.lib.fmlm_attn_fwd_noalloc(ctypes.byref(p), plan.stream) == -3  # unsupported head dim
+
+
+@pytest.mark.parametrize("B,H,N,ctx", [(16, 64, 8, 4000), (160, 16, 1, 2000), (3, 64, 4, 3000)])
+def test_noalloc_latent_with_more_tiles_than_records(B, H, N, ctx, device):
+    """Latent calls of 64 tiles of 128 rows and 160 of 64: fewer records fit the scratch
+    array than the call has tiles, so it runs unsplit; the last one's 12 tiles split."""
+    out, plan = _case(device, B=B, H=H, N=N, D=512, dtype=torch.bfloat16, lq=(N, N), lc=(ctx, ctx), mla=True, seed=4)
+    plan()
+    got = _noalloc(plan, out)
+    again = _noalloc(plan, out)
+    torch.cuda.synchronize()
+    assert torch.isfinite(got).all()
+    assert torch.equal(got, again)
+    torch.testing.assert_close(got.float(), out.float(), atol=1e-2, rtol=1e-2)
