@@ -2872,15 +2872,15 @@ static int check_params(const fmlm_attn_params& p) {
 }
 
 static int launch_schedule(const fmlm_attn_params& p, const Launch& L, const SplitCfg& sc, char* sched,
-                           int64_t bytes, hipStream_t s) {
+                           bool own_records, hipStream_t s) {
   const SchedLayout l = sched_layout(p, L.bq, sc, L.hpack);
   // the unit's 16-bit tile field: tiles of N rows, or of H*N (H*total_q) rows head-packed;
   // queue entries are addressed with 32-bit indices
   const int64_t rows = L.hpack ? (int64_t)p.H * (p.N > 0 ? p.N : p.total_q) : p.N;
   if (kXcds * l.cap > 0x7fffffff || p.H > 0xffff || (rows + L.bq - 1) / L.bq > 0xffff) return FMLM_E_ARG;
   int32_t* header = (int32_t*)sched;
-  // a buffer without room for the records: each launch brings its own (split_record)
-  const int64_t records_off = bytes >= l.bytes ? l.records_off : 0;
+  // 0: each launch brings its own records (split_record)
+  const int64_t records_off = own_records ? 0 : l.records_off;
   hipLaunchKernelGGL(schedule_kernel, dim3(1), dim3(kSchedThreads), 0, s, p, L.bq, (int)l.cap,
                      sc.slots, sc.rec_cap, split_min_tiles(L), (int4*)(sched + l.units_off), header,
                      (int4*)(sched + l.groups_off), (int)l.groups_off, (int)records_off,
@@ -2889,11 +2889,11 @@ static int launch_schedule(const fmlm_attn_params& p, const Launch& L, const Spl
 }
 
 // The attention launch (plus the split merge) over the schedule at `sched` (packed calls;
-// built first when `build` is set, in `bytes` bytes).  sc must be the split sizing the
-// schedule was (or is) built with; records: where split parts go, NULL for the schedule's
-// own record area.
+// built first, with its own record area, when `build` is set).  sc must be the split sizing
+// the schedule was (or is) built with; records: where split parts go, NULL for the
+// schedule's own record area.
 static int launch_attention(const fmlm_attn_params& p, const Launch& L, const SplitCfg& sc, char* sched,
-                            bool build, int64_t bytes, char* records, hipStream_t s) {
+                            bool build, char* records, hipStream_t s) {
   const void* const fn = sc.rec_cap > 0 && L.split_fn ? L.split_fn : L.fn;
   int rc = allow_lds(fn, L.lds);
   if (rc) return rc;
@@ -2903,7 +2903,7 @@ static int launch_attention(const fmlm_attn_params& p, const Launch& L, const Sp
     header = (int32_t*)sched;
     units = (int4*)(sched + 256);
     if (build) {
-      rc = launch_schedule(p, L, sc, sched, bytes, s);
+      rc = launch_schedule(p, L, sc, sched, false, s);
       if (rc) return rc;
     }
   }
@@ -2983,8 +2983,9 @@ extern "C" int fmlm_attn_schedule(const fmlm_attn_params* pp, void* schedule,
   const int rc = pick_launch(*pp, L);
   if (rc) return rc;
   const SplitCfg sc = split_cfg(*pp, L);
-  if (schedule_bytes < workspace_for(*pp, L, sc) - records_for(sc)) return FMLM_E_WORKSPACE;
-  return launch_schedule(*pp, L, sc, (char*)schedule, schedule_bytes, (hipStream_t)stream);
+  const bool own = pp->flags & FMLM_FLAG_OWN_RECORDS;
+  if (schedule_bytes < workspace_for(*pp, L, sc) - (own ? records_for(sc) : 0)) return FMLM_E_WORKSPACE;
+  return launch_schedule(*pp, L, sc, (char*)schedule, own, (hipStream_t)stream);
 }
 
 extern "C" int fmlm_attn_params_size(void) { return (int)sizeof(fmlm_attn_params); }
@@ -3021,15 +3022,16 @@ extern "C" int fmlm_attn_fwd(const fmlm_attn_params* pp, void* stream) {
   char* const ws = (char*)p.workspace;
   if (!p.cu_seqlens_q) {  // dense: the workspace holds split records only; without one, no split
     if (have < records_for(sc)) sc = SplitCfg{};
-    return launch_attention(p, L, sc, nullptr, false, 0, ws, (hipStream_t)stream);
+    return launch_attention(p, L, sc, nullptr, false, ws, (hipStream_t)stream);
   }
   const int64_t need = workspace_for(p, L, sc);
   if (p.schedule) {
-    char* const records = records_for(sc) > 0 && have >= records_for(sc) ? ws : nullptr;
-    return launch_attention(p, L, sc, (char*)p.schedule, false, 0, records, (hipStream_t)stream);
+    const bool own = p.flags & FMLM_FLAG_OWN_RECORDS;
+    if (own && have < records_for(sc)) return FMLM_E_WORKSPACE;
+    return launch_attention(p, L, sc, (char*)p.schedule, false, own ? ws : nullptr, (hipStream_t)stream);
   }
   if (need > 0 && have < need) return FMLM_E_WORKSPACE;
-  return launch_attention(p, L, sc, ws, true, need, nullptr, (hipStream_t)stream);
+  return launch_attention(p, L, sc, ws, true, nullptr, (hipStream_t)stream);
 }
 
 extern "C" int fmlm_attn_fwd_noalloc(const fmlm_attn_params* pp, void* stream) {
@@ -3049,6 +3051,6 @@ extern "C" int fmlm_attn_fwd_noalloc(const fmlm_attn_params* pp, void* stream) {
     if (rc) return rc;
   }
   // the schedule is always rebuilt: the array holds whatever the previous call left
-  if (!p.cu_seqlens_q) return launch_attention(p, L, sc, nullptr, false, 0, scratch_mem, (hipStream_t)stream);
-  return launch_attention(p, L, sc, scratch_mem, true, kNoAllocScratchBytes, nullptr, (hipStream_t)stream);
+  if (!p.cu_seqlens_q) return launch_attention(p, L, sc, nullptr, false, scratch_mem, (hipStream_t)stream);
+  return launch_attention(p, L, sc, scratch_mem, true, nullptr, (hipStream_t)stream);
 }

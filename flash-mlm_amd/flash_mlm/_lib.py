@@ -26,6 +26,7 @@ FLAG_MLA = 1
 FLAG_PREFILL = 2
 FLAG_CAUSAL_SEQ = 4
 FLAG_NOSPLIT = 8
+FLAG_OWN_RECORDS = 16
 
 LAYOUT_PADDED = 0
 LAYOUT_PACKED = 1

@@ -458,6 +458,8 @@ def _prepare(
         # layout, paged context or not), whose tile size and occupancy fix the slots,
         # the split records and the grid, and the shape (B, H, N, total_q); context
         # lengths only steer where key ranges are split
+        if records:
+            p.flags |= _lib.FLAG_OWN_RECORDS
         key = (p.dtype, D, B, H, N, total_q, p.flags, p.kv_layout, block_table is not None, p.tile_config)
         sched = schedule_cache.get(key)
         if sched is None:

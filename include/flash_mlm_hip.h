@@ -52,8 +52,11 @@ enum {
   FMLM_FLAG_MLA = 1,        /* V is K (one shared latent head for main and context) */
   FMLM_FLAG_PREFILL = 2,    /* skip the cached-context segment */
   FMLM_FLAG_CAUSAL_SEQ = 4, /* sequence b attends to main tokens [0, cu_q[b+1]) */
-  FMLM_FLAG_NOSPLIT = 8     /* key ranges are not split (no records, no merge launch); a
+  FMLM_FLAG_NOSPLIT = 8,    /* key ranges are not split (no records, no merge launch); a
                                schedule is then built with this flag too               */
+  FMLM_FLAG_OWN_RECORDS = 16 /* the schedule has no room for split partial results: every
+                               fmlm_attn_fwd on it has this flag too and brings them in
+                               its workspace                                           */
 };
 
 /* row layouts of a [*, D] tensor addressed by (sequence b, head h, position p) */
@@ -214,14 +217,16 @@ typedef struct fmlm_attn_params {
   void* workspace;         /* device scratch for the work schedule                  */
   int64_t workspace_bytes;
   const void* schedule;    /* NULL, or a schedule built by fmlm_attn_schedule for the same
-                              cu_seqlens_q contents, B, H, total_q, dtype, D, flags and
+                              cu_seqlens_q contents, B, H, total_q, dtype, D, flags (with
+                              others than it was built for, rows stay unwritten) and
                               kv_layout: then fmlm_attn_fwd launches the attention
                               kernel (plus the split merge) only.  Context lengths may
-                              differ; they only steer where key ranges are split.  Split
-                              partial results go to `workspace` when it holds at least
-                              fmlm_attn_records_bytes (launches that overlap then only
-                              need workspaces of their own), else to the schedule buffer
-                              (launches that may overlap need separate ones)          */
+                              differ; they only steer where key ranges are split.  The
+                              buffer also holds split partial results: launches that may
+                              overlap need separate schedule buffers.  With
+                              FMLM_FLAG_OWN_RECORDS they are in `workspace` instead (at
+                              least fmlm_attn_records_bytes, else FMLM_E_WORKSPACE), and
+                              launches that overlap only need workspaces of their own */
   const int32_t* ctx_index;  /* [B] context batch of each sequence, or NULL (see above):
                                 index-mapped context batching.  No counterpart in the
                                 reference, whose roadmap lists it ("variable context
@@ -269,14 +274,13 @@ FMLM_API int64_t fmlm_attn_workspace_bytes(const fmlm_attn_params* p);
 /* The part of fmlm_attn_workspace_bytes that holds split partial results, or < 0 as above.
  * 0 when the call cannot split: with FMLM_FLAG_NOSPLIT set it then does the same with one
  * launch less, in a smaller schedule and workspace (for a packed call by its own context
- * sizes: without the flag it must still run a schedule built for longer contexts).  A schedule buffer without that part serves calls that
- * bring a workspace of this many bytes. */
+ * sizes: without the flag it must still run a schedule built for longer contexts). */
 FMLM_API int64_t fmlm_attn_records_bytes(const fmlm_attn_params* p);
 
 /* Build the work schedule (one entry per query tile of the kernel's own tile size over
- * the real rows of every sequence) into `schedule` (fmlm_attn_workspace_bytes bytes, or
- * that less fmlm_attn_records_bytes) so later fmlm_attn_fwd calls with p->schedule =
- * schedule skip rebuilding it.  No counterpart in the reference (its tile map is PackMetadata.batch_ids_q /
+ * the real rows of every sequence) into `schedule` (fmlm_attn_workspace_bytes bytes, with
+ * FMLM_FLAG_OWN_RECORDS less fmlm_attn_records_bytes; FMLM_E_WORKSPACE when it is smaller)
+ * so later fmlm_attn_fwd calls with p->schedule = schedule skip rebuilding it.  No counterpart in the reference (its tile map is PackMetadata.batch_ids_q /
  * q_tile_starts_q at block_n granularity, host_utils.py:74-107). */
 FMLM_API int fmlm_attn_schedule(const fmlm_attn_params* p, void* schedule, int64_t schedule_bytes,
                                 void* stream);

@@ -180,3 +180,51 @@ def test_split_call_in_a_graph(way, device):
         eager = call()
         torch.cuda.synchronize()
         assert torch.equal(out, want) and torch.equal(eager, want)
+
+
+@pytest.mark.parametrize("D,H,mla", [(64, 4, False), (512, 16, True)])
+def test_schedule_holds_the_records_or_each_call_brings_them(D, H, mla, device):
+    """A schedule without room for the split records is only built, and only run, with
+    FMLM_FLAG_OWN_RECORDS and a workspace for them; without the flag the records are in the
+    schedule buffer, also when the caller passes that buffer as the workspace too."""
+    gen = torch.Generator().manual_seed(21)
+    dtype, lengths, C = torch.bfloat16, [3, 2], 3000
+    N, B = max(lengths), len(lengths)
+    q, k, v = (_randn(gen, (B, H, N, D), dtype, device, 0.5) for _ in range(3))
+    hk = 1 if mla else H
+    kc, vc = _randn(gen, (hk * B * C, D), dtype, device, 0.5), None if mla else _randn(gen, (hk * B * C, D), dtype, device, 0.5)
+    cache = InferenceCache()
+    cache.prefill_kv_cache(0, k_cache=kc, v_cache=vc, total_context_len=B * C, context_batch_size=B, is_mla=mla,
+                           cu_seqlens_kv=torch.arange(B + 1, dtype=torch.int32, device=device) * C, num_heads=H,
+                           head_dim=D)
+    meta = build_pack_metadata(torch.tensor(lengths, dtype=torch.int32, device=device), N, 64)
+    want, plan = hh._compressed_impl(q, k, v, H, meta, D ** -0.5, cache, 0, mla, None, 64, 64, False, False, False,
+                                     run=False)
+    assert plan.records > 0, "the shape is meant to split"
+    plan()
+    lib, stream, e_workspace = plan.lib, plan.stream, -5
+    out = torch.full_like(want, float("nan"))
+
+    def block():
+        p = _lib.AttnParams.from_buffer_copy(plan.params)
+        p.o, p.workspace, p.workspace_bytes = out.data_ptr(), None, 0
+        return p
+
+    p = block()
+    assert p.flags & _lib.FLAG_OWN_RECORDS
+    assert lib.fmlm_attn_fwd(ctypes.byref(p), stream) == e_workspace
+    p = block()
+    p.flags &= ~_lib.FLAG_OWN_RECORDS
+    p.schedule = None
+    nbytes, records = lib.fmlm_attn_workspace_bytes(ctypes.byref(p)), lib.fmlm_attn_records_bytes(ctypes.byref(p))
+    assert records == plan.records
+    buf = torch.empty(nbytes, dtype=torch.uint8, device=device)
+    assert lib.fmlm_attn_schedule(ctypes.byref(p), buf.data_ptr(), nbytes - 1, stream) == e_workspace
+    assert lib.fmlm_attn_schedule(ctypes.byref(p), buf.data_ptr(), nbytes, stream) == 0
+    p.schedule = p.workspace = buf.data_ptr()
+    p.workspace_bytes = nbytes
+    for _ in range(2):  # the first run leaves the schedule as it was
+        out.fill_(float("nan"))
+        assert lib.fmlm_attn_fwd(ctypes.byref(p), stream) == 0
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
