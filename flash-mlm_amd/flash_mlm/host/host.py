@@ -97,10 +97,15 @@ def _workspace(inference_cache: InferenceCache | None, nbytes: int, device: torc
 _ROW_STATS = threading.local()
 
 
+def _torch_stream(handle: int, device: torch.device):
+    # handle 0 is the default stream; ExternalStream(0) would be a new one
+    return torch.cuda.ExternalStream(handle, device=device) if handle else torch.cuda.default_stream(device)
+
+
 class AttnLaunch:
     """A prepared fmlm_attn_fwd call: the parameter block plus the tensors it points to."""
 
-    __slots__ = ("lib", "params", "stream", "device", "keep", "unpack_kv", "lse", "records", "records_buf")
+    __slots__ = ("lib", "params", "stream", "device", "keep", "unpack_kv", "lse", "records")
 
     def __init__(self, lib, params, stream, device, keep):
         self.lib, self.params, self.stream, self.device, self.keep = lib, params, stream, device, keep
@@ -110,9 +115,9 @@ class AttnLaunch:
         self.lse = None  # the row statistics of the last run, when it stored them
         # bytes of split partial results each run brings in a buffer of its own, so that runs
         # of one schedule on several streams or threads never share them (0: none, or the
-        # parameter block's workspace holds them)
+        # parameter block's workspace holds them).  The buffer is the launch's stream's
+        # memory: let go of at once, it is reused behind the launch only
         self.records = 0
-        self.records_buf = None  # kept only by a run on a stream other than the current one
 
     def __call__(self) -> None:
         p = self.params
@@ -124,10 +129,12 @@ class AttnLaunch:
             self.lse = torch.empty(p.H * p.total_q, dtype=torch.float32, device=self.device)
             p.lse = self.lse.data_ptr()
         if self.records:
-            buf = torch.empty(self.records, dtype=torch.uint8, device=self.device)
+            if _lib.stream_of(self.device) == self.stream:
+                buf = torch.empty(self.records, dtype=torch.uint8, device=self.device)
+            else:
+                with torch.cuda.stream(_torch_stream(self.stream, self.device)):
+                    buf = torch.empty(self.records, dtype=torch.uint8, device=self.device)
             p.workspace, p.workspace_bytes = buf.data_ptr(), self.records
-            if _lib.stream_of(self.device) != self.stream:
-                self.records_buf = buf
         with _device_scope(self.device):
             rc = self.lib.fmlm_attn_fwd(p, self.stream)
         _lib.check(rc, "fmlm_attn_fwd")

@@ -228,3 +228,32 @@ def test_schedule_holds_the_records_or_each_call_brings_them(D, H, mla, device):
         assert lib.fmlm_attn_fwd(ctypes.byref(p), stream) == 0
         torch.cuda.synchronize()
         assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("plan_on_side", [True, False])
+def test_records_of_a_run_from_another_stream(plan_on_side, device):
+    """A prepared launch keeps its stream: the records of a run started while another
+    stream is current are that stream's memory, which a new tensor of the current stream
+    never gets while the launch may still be running."""
+    gen = torch.Generator().manual_seed(3)
+    H, D, C = 2, 64, 4000
+    q, k, v = (_randn(gen, (1, H, 9, D), torch.bfloat16, device) for _ in range(3))
+    kc, vc = (_randn(gen, (H * C, D), torch.bfloat16, device) for _ in range(2))
+    cache = InferenceCache()
+    cache.prefill_kv_cache(0, k_cache=kc, v_cache=vc, context_batch_size=1, is_mla=False, num_heads=H, head_dim=D)
+    want = flash_attn_mlm(q, k, v, 0.125, inference_cache=cache, layer_id=0)
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    own, other = (side, torch.cuda.current_stream()) if plan_on_side else (torch.cuda.current_stream(), side)
+    with torch.cuda.stream(own):
+        out, plan = hh._dense_impl(q, k, v, 0.125, cache, 0, False, None, False, run=False)
+    assert plan.records > 0 and plan.stream == own.cuda_stream
+    used = set()
+    with torch.cuda.stream(other):
+        for _ in range(3):
+            plan()
+            used.add(plan.params.workspace)
+        fresh = [torch.empty(plan.records, dtype=torch.uint8, device=device) for _ in range(4)]
+    assert used.isdisjoint(t.data_ptr() for t in fresh)
+    torch.cuda.synchronize()
+    assert torch.equal(out, want)
