@@ -2934,7 +2934,7 @@ static int launch_attention(const fmlm_attn_params& p, const Launch& L, const Sp
 // and the split records live in this library-owned array, one copy per GPU, instead of
 // a caller's workspace.  Host code never uses the array's name as an address: it reads
 // each device's address once with hipGetSymbolAddress (scratch_on_current_device).
-// Every call on a GPU reuses that GPU's array; calls that overlap on one GPU race.
+// Every packed call on a GPU reuses that GPU's array; calls that overlap on one GPU race.
 // ---------------------------------------------------------------------------
 constexpr int64_t kNoAllocScratchBytes = FMLM_NOALLOC_SCRATCH_BYTES;
 __device__ __align__(256) char scratch[kNoAllocScratchBytes];
@@ -2961,14 +2961,15 @@ static int scratch_on_current_device(char** out) {
 }
 
 // The split sizing of the allocation-free path: as split_cfg, with the record count cut
-// so that the schedule and the records fit the scratch array (fit_records; a dense call's
-// parts are all or none).  Returns false when even the unsplit schedule does not fit.
+// so that the schedule and the records fit the scratch array (fit_records).  Dense calls
+// need no schedule and do not split: they leave the array alone, so that they may overlap
+// any other call.  Returns false when even the unsplit schedule does not fit.
 static bool split_cfg_within(const fmlm_attn_params& p, const Launch& L, int64_t cap, SplitCfg& sc) {
-  sc = split_cfg(p, L);
   if (!p.cu_seqlens_q) {
-    if (records_for(sc) > cap) sc = SplitCfg{};
+    sc = SplitCfg{};
     return true;
   }
+  sc = split_cfg(p, L);
   return fit_records(p, L.bq, L.hpack, cap, sc);
 }
 
@@ -3045,12 +3046,10 @@ extern "C" int fmlm_attn_fwd_noalloc(const fmlm_attn_params* pp, void* stream) {
   if (p.B == 0 || p.H == 0) return 0;
   SplitCfg sc;
   if (!split_cfg_within(p, L, kNoAllocScratchBytes, sc)) return FMLM_E_WORKSPACE;
+  if (!p.cu_seqlens_q) return launch_attention(p, L, sc, nullptr, false, nullptr, (hipStream_t)stream);
   char* scratch_mem = nullptr;
-  if (p.cu_seqlens_q || sc.rec_cap > 0) {
-    rc = scratch_on_current_device(&scratch_mem);
-    if (rc) return rc;
-  }
+  rc = scratch_on_current_device(&scratch_mem);
+  if (rc) return rc;
   // the schedule is always rebuilt: the array holds whatever the previous call left
-  if (!p.cu_seqlens_q) return launch_attention(p, L, sc, nullptr, false, scratch_mem, (hipStream_t)stream);
   return launch_attention(p, L, sc, scratch_mem, true, nullptr, (hipStream_t)stream);
 }

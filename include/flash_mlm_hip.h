@@ -295,9 +295,10 @@ FMLM_API int fmlm_attn_fwd(const fmlm_attn_params* p, void* stream);
  * results live in a device array owned by the library, FMLM_NOALLOC_SCRATCH_BYTES per
  * GPU, held until the process ends; the schedule is rebuilt on every call.  When the
  * split records would not fit, fewer key ranges are split (or none); a call whose
- * unsplit schedule does not fit returns FMLM_E_WORKSPACE.  Every call on a GPU shares
- * that GPU's array: calls that may overlap on one GPU (different streams, or host
- * threads) race and must be serialised by the caller.  Allocates nothing.
+ * unsplit schedule does not fit returns FMLM_E_WORKSPACE.  Every packed call on a GPU
+ * shares that GPU's array: calls that may overlap on one GPU (different streams, or host
+ * threads) race and must be serialised by the caller.  Dense calls (cu_seqlens_q == NULL)
+ * do not split and do not use the array: they may overlap any other.  Allocates nothing.
  * ------------------------------------------------------------------------- */
 #define FMLM_NOALLOC_SCRATCH_BYTES (16 << 20)
 

@@ -106,3 +106,28 @@ def test_noalloc_latent_with_more_tiles_than_records(B, H, N, ctx, device):
     assert torch.isfinite(got).all()
     assert torch.equal(got, again)
     torch.testing.assert_close(got.float(), out.float(), atol=1e-2, rtol=1e-2)
+
+
+@pytest.mark.parametrize("D,mla", [(64, False), (512, True)])
+def test_noalloc_dense_does_not_use_the_scratch(D, mla, device):
+    """A dense call that fmlm_attn_fwd splits runs unsplit here, whatever the flags: its
+    result is the unsplit one bit for bit, so that dense calls that overlap share nothing."""
+    gen = torch.Generator().manual_seed(6)
+    H, N, C = 2, 20, 3000
+    q, k, v = ((torch.randn((1, H, N, D), generator=gen) * 0.5).to(torch.bfloat16).to(device) for _ in range(3))
+    kc, vc = ((torch.randn(((1 if mla else H) * C, D), generator=gen) * 0.5).to(torch.bfloat16).to(device) for _ in range(2))
+    cache = InferenceCache()
+    cache.prefill_kv_cache(0, k_cache=kc, v_cache=None if mla else vc, context_batch_size=1, is_mla=mla, num_heads=H,
+                           head_dim=D)
+    out, plan = hh._dense_impl(q, k, v, D ** -0.5, cache, 0, mla, None, False, run=False)
+    assert plan.records > 0, "fmlm_attn_fwd is meant to split this shape"
+    got = _noalloc(plan, out)
+    whole = torch.full_like(out, float("nan"))
+    p = _lib.AttnParams.from_buffer_copy(plan.params)
+    p.o, p.workspace, p.workspace_bytes = whole.data_ptr(), None, 0  # no workspace: unsplit
+    _lib.check(plan.lib.fmlm_attn_fwd(ctypes.byref(p), plan.stream), "fmlm_attn_fwd")
+    plan()
+    torch.cuda.synchronize()
+    assert torch.equal(got, whole)
+    assert not torch.equal(got, out), "the split result is rounded elsewhere: the comparison says nothing"
+    torch.testing.assert_close(got.float(), out.float(), atol=1e-2, rtol=1e-2)
