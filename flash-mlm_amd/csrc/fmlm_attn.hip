@@ -2145,6 +2145,8 @@ __global__ __launch_bounds__(256, (F32Cfg<D, QB>::WPS)) void attn_f32_kernel(
       wait_reads();
       load(tl, false);
       if (nk < 16) {
+        wait_loads<TL::NL>();  // V (the next K's loads came later)
+        TL::zero_from(nk, vt, lane);
 #pragma unroll
         for (int r = 0; r < 4; ++r)
           if (4 * g + r >= nk)

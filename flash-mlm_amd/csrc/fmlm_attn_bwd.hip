@@ -2282,18 +2282,20 @@ __global__ __launch_bounds__(256, F32BwdCfg<D>::WPS) void attn_bwd_dkv_f32_kerne
       for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
         for (int r = 0; r < 4; ++r) sa[kb][r] = fast_exp2(fmaf(sa[kb][r], c, -lse[r]));
-      const int kend = ku.causal_main ? min(s.n, si.mainlen) : s.n;  // keys this step's rows see
-      if (cur.p0 + wave * 16 + 16 > si.len || ku.j0 + C::KEYS > kend) {
-#pragma unroll
-        for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-            if (ku.j0 + kb * 16 + l16 >= kend || r0 + r >= si.len) sa[kb][r] = 0.f;
-      }
 #pragma unroll
       for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
         for (int r = 0; r < 4; ++r) dp[kb][r] = sa[kb][r] * (dp[kb][r] - dl[r]) * p.scale;
+      const int kend = ku.causal_main ? min(s.n, si.mainlen) : s.n;  // keys this step's rows see
+      if (cur.p0 + wave * 16 + 16 > si.len || ku.j0 + C::KEYS > kend) {
+        // (dO; a last row of Q that is not finite makes every weight of the row NaN anyway)
+        if (cur.p0 + wave * 16 + 16 > si.len) TL::zero_from(si.len - (cur.p0 + wave * 16), qt + TL::BYTES, lane);
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (ku.j0 + kb * 16 + l16 >= kend || r0 + r >= si.len) sa[kb][r] = dp[kb][r] = 0.f;
+      }
       mma_cols<D, KB>(qt + TL::BYTES, l16, g, sa, dv);
       if (C::NBUF == 1 && more) {
         wait_reads();

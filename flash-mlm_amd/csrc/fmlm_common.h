@@ -287,6 +287,12 @@ struct F32Tile {
 #pragma unroll
     for (int i = 0; i < NL; ++i) dma16_sbase(src, off[i], __builtin_amdgcn_readfirstlane(lds + i * 1024));
   }
+  // rows [n, 16) of a loaded tile to zero, n < 16: they repeat row n - 1, and where that row is not
+  // finite its product with their weight 0 would not be 0
+  static FMLM_DEV void zero_from(int n, uint32_t lds, int lane) {
+    for (int at = n * PITCH; at < BYTES; at += 1024)
+      if (at + 16 * lane < BYTES) *(FMLM_LDS f32x4*)(uintptr_t)(lds + at + 16 * lane) = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
   // the lane's address of row fragment 0 in the tile at LDS address lds (a multiple of 256)
   static FMLM_DEV uint32_t row_base(uint32_t lds, int l16, int g) { return lds + l16 * PITCH + 16 * (g ^ swz(l16)); }
   static FMLM_DEV f32x4 row(uint32_t base, int ds) {  // columns 16ds + 4g .. +4 of row l16

@@ -11,7 +11,8 @@ import numpy as np
 import pytest
 import torch
 
-from flash_mlm import InferenceCache, build_pack_metadata, flash_attn_mlm_compressed, unpack_from_kernel
+from flash_mlm import InferenceCache, build_pack_metadata, flash_attn_mlm, flash_attn_mlm_compressed, \
+    unpack_from_kernel
 from oracle import attention_ref as ar
 
 pytestmark = pytest.mark.gpu
@@ -84,3 +85,39 @@ def test_f32_backward_edges(D, H, lengths, ctx, causal, mla, device):
     for name, g, r in zip(["q", "k", "kc"] if mla else ["q", "k", "v", "kc", "vc"], got, ref):
         worst = np.abs(_np(g) - r).max() / np.abs(r).max()
         assert worst <= 2e-5, (name, worst)
+
+
+@pytest.mark.parametrize("D", [16, 64, 256])
+def test_f32_infinity_in_a_last_value_row(D, device):
+    """A value that is infinite in the last row of a key range reaches that column of every
+    row that attends to it and nothing else: key slots past a range's end hold no copy of
+    it (0 * inf would be NaN)."""
+    H, lengths, ctx = 2, [5, 33, 16], [17, 3, 70]
+    q, k, v, kc, vc, cu, cache, meta = _case(device, D, H, lengths, ctx, D)
+    v[0, 1, lengths[0] - 1, 3] = float("inf")  # sequence 0, head 1: main keys
+    vc[cu[2] - 1, 7] = float("-inf")           # sequence 1, head 0: context
+    out = unpack_from_kernel(flash_attn_mlm_compressed(q, k, v, H, meta, D ** -0.5, cache, 0, block_n=64), meta, H)
+    finite_v, finite_vc = v.clone(), vc.clone()
+    finite_v[0, 1, lengths[0] - 1, 3] = finite_vc[cu[2] - 1, 7] = 0.0
+    ref = ar.mlm_attention_packed(_np(q), _np(k), _np(finite_v), lengths, D ** -0.5, k_cache=_np(kc),
+                                  v_cache=_np(finite_vc), cu_seqlens_kv=cu, total_context_len=cu[-1],
+                                  context_batch_size=len(ctx))
+    ref[0, 1, :lengths[0], 3] = np.inf
+    ref[1, 0, :lengths[1], 7] = -np.inf
+    np.testing.assert_allclose(_np(out), ref, atol=TOL, rtol=TOL)
+
+
+@pytest.mark.parametrize("D", [16, 64, 256])
+def test_f32_infinity_in_a_last_gradient_row(D, device):
+    """The same for dO: one infinite entry in a sequence's last row makes that column of the
+    sequence's dv infinite, and no other entry of any dv."""
+    H, lengths = 2, [5, 33, 16]
+    q, k, v, _, _, _, _, meta = _case(device, D, H, lengths, [1, 1, 1], D, grad=True)
+    out = flash_attn_mlm_compressed(q, k, v, H, meta, D ** -0.5, block_n=64)
+    dout = torch.randn(out.shape, generator=torch.Generator().manual_seed(1)).to(device)
+    (want,) = torch.autograd.grad(out, [v], dout, retain_graph=True)
+    dout[lengths[0] - 1, 3] = float("inf")  # head 0, sequence 0, its last row
+    (got,) = torch.autograd.grad(out, [v], dout)
+    want = want.clone()
+    want[0, 0, :lengths[0], 3] = float("inf")
+    assert torch.equal(got, want)
