@@ -2234,7 +2234,8 @@ __global__ __launch_bounds__(256, (F32Cfg<D, QB>::WPS)) void attn_f32_kernel(
         ml[C::BQ + row] = L;
       }
     } else {
-      *(f32x4*)((float*)p.o + w.o_row0 + (int64_t)row * w.o_sn + col) = acc * (L > 0.f ? 1.f / L : 1.f);
+      // L is 0 only where every score is -inf (a row has keys, its own): NaN, as 0 * (1 / 0)
+      *(f32x4*)((float*)p.o + w.o_row0 + (int64_t)row * w.o_sn + col) = acc * (1.f / L);
       if (p.lse && col == 0) store_lse(p, w.h, w.q0, w.qpos0 + row, M, L);
     }
   }
@@ -2488,7 +2489,8 @@ __global__ __launch_bounds__(kMergeThreads) void merge_kernel(const fmlm_attn_pa
         l[sp] = M == -INFINITY ? 0.f : fast_exp2(m[sp] - M) * l[sp];
         L += l[sp];
       }
-      const float inv = L > 0.f ? 1.f / L : 0.f;
+      // L is 0 only where every score of the row is -inf (a row has keys, its own): NaN
+      const float inv = 1.f / L;
 #pragma unroll
       for (int sp = 0; sp < kMaxSplits; ++sp) s_w[r][sp] = l[sp] * inv;
       if (p.lse) store_lse(p, hq, si.q0, pos, M, L);

@@ -121,3 +121,34 @@ def test_f32_infinity_in_a_last_gradient_row(D, device):
     want = want.clone()
     want[0, 0, :lengths[0], 3] = float("inf")
     assert torch.equal(got, want)
+
+def _overflowing(device, D, n_keys, hidden, seed):
+    """One head of 9 queries over n_keys context keys.  Query 4's score with the first
+    `hidden` keys overflows to -inf (key entry 3e38 against -1e10), the others' do not."""
+    gen = torch.Generator().manual_seed(seed)
+    q, k, v = (torch.randn((1, 1, 9, D), generator=gen).to(device) for _ in range(3))
+    kc, vc = (torch.randn((n_keys, D), generator=gen).to(device) for _ in range(2))
+    q[..., 0] = 0.0
+    q[0, 0, 4, 0] = -1e10
+    k[..., 0] = 0.0
+    kc[:, 0] = 0.0
+    kc[:hidden, 0] = 3e38
+    return q, k, v, kc, vc
+
+
+@pytest.mark.parametrize("all_hidden", [False, True])
+@pytest.mark.parametrize("D,C", [(32, 40), (64, 100), (64, 5000), (256, 3000)])  # the last two are split
+def test_f32_scores_of_minus_infinity(D, C, all_hidden, device):
+    """Keys of score -inf have weight 0, also a whole tile or part of them; a row without any
+    other key has no softmax: NaN, and the other rows are not touched."""
+    q, k, v, kc, vc = _overflowing(device, D, C, C if all_hidden else C - C // 5, D)
+    if all_hidden:
+        k[..., 0] = 3e38
+    cache = InferenceCache()
+    cache.prefill_kv_cache(0, k_cache=kc, v_cache=vc, context_batch_size=1, is_mla=False, num_heads=1, head_dim=D)
+    out = flash_attn_mlm(q, k, v, D ** -0.5, inference_cache=cache, layer_id=0)
+    kk, vv = torch.cat([kc, k[0, 0]]).double(), torch.cat([vc, v[0, 0]]).double()
+    z = (q[0, 0].double() @ kk.T * D ** -0.5).float().double()  # -3e48 is -inf in float32
+    ref = torch.softmax(z, dim=-1) @ vv
+    assert bool(torch.isnan(ref[4]).all()) == all_hidden and not torch.isnan(ref[[0, 8]]).any()
+    torch.testing.assert_close(out[0, 0].double(), ref, atol=TOL, rtol=TOL, equal_nan=True)
