@@ -370,6 +370,18 @@ struct SplitArgs {
   int32_t dense_parts;  // 1: not split
 };
 
+// key tiles [tb, te) of a unit's part: the whole range costs no division (the two 64-bit ones
+// that this took before the first load were 0.5 us of a 50 us call of one round).
+// kMaxSplits * ntiles < 2^31
+FMLM_DEV void part_range(const WorkItem& w, int ntiles, int& tb, int& te) {
+  tb = 0;
+  te = ntiles;
+  if (w.split_n > 1) {
+    tb = (int)((uint32_t)(w.split_s * ntiles) / (uint32_t)w.split_n);
+    te = (int)((uint32_t)((w.split_s + 1) * ntiles) / (uint32_t)w.split_n);
+  }
+}
+
 // record i, or NULL when the launch has no room for records
 FMLM_DEV char* split_record(const int32_t* hdr, const SplitArgs& spa, int i) {
   char* base = spa.records;
@@ -1050,8 +1062,8 @@ __global__ __launch_bounds__(NW * 64, NW >= 8 ? 1 : 2) void attn_mfma3_kernel(
   const int nt1 = (w.seg[1].n + BK - 1) / BK;
   const int ntiles = nt0 + nt1;
   // key tiles [tb, te) of this unit: all of them, or part s of S of a split group
-  const int tb = (int)((int64_t)w.split_s * ntiles / w.split_n);
-  const int te = (int)((int64_t)(w.split_s + 1) * ntiles / w.split_n);
+  int tb, te;
+  part_range(w, ntiles, tb, te);
   // the partial last tile of each segment (-1: none) and the keys it holds; every other
   // tile holds BK keys
   const int pt0 = (w.seg[0].n % BK) ? nt0 - 1 : -1, pt1 = (w.seg[1].n % BK) ? ntiles - 1 : -1;
@@ -1711,8 +1723,8 @@ __global__ __launch_bounds__(MlaRowsCfg::NT, 1) void attn_mla_rows_kernel(
   const int nt1 = (w.seg[1].n + BK - 1) / BK;
   const int ntiles = nt0 + nt1;
   // this part's tiles (split-KV)
-  const int tb = SPLIT ? (int)((int64_t)w.split_s * ntiles / w.split_n) : 0;
-  const int te = SPLIT ? (int)((int64_t)(w.split_s + 1) * ntiles / w.split_n) : ntiles;
+  int tb = 0, te = ntiles;
+  if (SPLIT) part_range(w, ntiles, tb, te);
   PageWindow pwin;  // paged context: page ids of the tiles around the last one fetched
   page_window_reset(pwin);
 
@@ -2086,8 +2098,8 @@ __global__ __launch_bounds__(256, (F32Cfg<D, QB>::WPS)) void attn_f32_kernel(
   const int n0 = w.seg[0].n, n1 = w.seg[1].n;
   const int nt0 = (n0 + C::BK - 1) / C::BK;
   const int ntiles = nt0 + (n1 + C::BK - 1) / C::BK;
-  const int tb = (int)((int64_t)w.split_s * ntiles / w.split_n);
-  const int te = (int)((int64_t)(w.split_s + 1) * ntiles / w.split_n);
+  int tb, te;
+  part_range(w, ntiles, tb, te);
   const float* const kp0 = (const float*)w.seg[0].k + w.seg[0].kbase;
   const float* const kp1 = (const float*)w.seg[1].k + w.seg[1].kbase;
   const float* const vp0 = (const float*)w.seg[0].v + w.seg[0].vbase;
