@@ -2890,10 +2890,7 @@ static int check_params(const fmlm_attn_params& p) {
 static int launch_schedule(const fmlm_attn_params& p, const Launch& L, const SplitCfg& sc, char* sched,
                            bool own_records, hipStream_t s) {
   const SchedLayout l = sched_layout(p, L.bq, sc, L.hpack);
-  // the unit's 16-bit tile field: tiles of N rows, or of H*N (H*total_q) rows head-packed;
-  // queue entries are addressed with 32-bit indices
-  const int64_t rows = L.hpack ? (int64_t)p.H * (p.N > 0 ? p.N : p.total_q) : p.N;
-  if (kXcds * l.cap > 0x7fffffff || p.H > 0xffff || (rows + L.bq - 1) / L.bq > 0xffff) return FMLM_E_ARG;
+  if (!units_encodable(p, L.bq, l.cap, L.hpack)) return FMLM_E_ARG;
   int32_t* header = (int32_t*)sched;
   // 0: each launch brings its own records (split_record)
   const int64_t records_off = own_records ? 0 : l.records_off;

@@ -115,6 +115,14 @@ inline SchedLayout sched_layout(const fmlm_attn_params& p, int bq, const SplitCf
   return l;
 }
 
+// Whether the call's units fit their encoding: 16-bit heads, 16-bit tiles of a sequence's
+// rows (head-packed: of its H times as many), 32-bit indices of queue entries.
+inline bool units_encodable(const fmlm_attn_params& p, int bq, int64_t cap, bool hpack) {
+  const int64_t most = p.N > 0 && p.N < p.total_q ? p.N : p.total_q;  // tokens of a sequence
+  const int64_t rows = hpack ? (int64_t)p.H * most : p.N;
+  return kXcds * cap <= 0x7fffffff && p.H <= 0xffff && (rows + bq - 1) / bq <= 0xffff;
+}
+
 // Cuts the record count of a packed call so that the schedule and the records fit `cap`
 // bytes.  No split when fewer would fit than one per workgroup slot (head-packed: than the
 // units the unsplit call can have, each of which takes a record, see hpack_price).  Returns

@@ -89,6 +89,22 @@ int main() {
   latent("16 heads, 200 x 1 token, 2500 keys", 16, std::vector<int>(200, 1), std::vector<int>(200, 2500), scratch);
   latent("all empty", 16, {0, 0}, {0, 0}, scratch);
 
+  // a few tokens in a long padded sequence: the tiles are those of the tokens
+  for (int bq : {64, 128}) {
+    fmlm_attn_params p{};
+    p.B = 1;
+    p.H = 64;
+    p.N = 70000;
+    p.total_q = 40;
+    const bool ok = units_encodable(p, bq, queue_cap(p, bq, SplitCfg{}, true), true);
+    p.total_q = p.N = 200000;
+    const bool too_many = units_encodable(p, bq, queue_cap(p, bq, SplitCfg{}, true), true);
+    if (!ok || too_many) {
+      failures++;
+      std::printf("units_encodable, %d rows per tile: %d for 40 tokens, %d for 200000\n", bq, ok, too_many);
+    }
+  }
+
   std::mt19937 gen(1);
   auto uni = [&](int lo, int hi) { return std::uniform_int_distribution<int>(lo, hi)(gen); };
   auto size = [&](int lo, int hi) {  // spread over the logarithm
