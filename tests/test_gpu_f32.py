@@ -87,6 +87,31 @@ def test_f32_backward_edges(D, H, lengths, ctx, causal, mla, device):
         assert worst <= 2e-5, (name, worst)
 
 
+@pytest.mark.parametrize("D,mla", [(16, False), (64, False), (128, True), (256, False)])
+def test_f32_packed_split(D, mla, device):
+    """Few queries over long ragged contexts: the schedule splits key ranges, and the fp32
+    records are merged; outputs, row statistics (through the backward) and gradients."""
+    H, lengths, ctx = 2, [5, 0, 9], [6000, 300, 3001]
+    q, k, v, kc, vc, cu, cache, meta = _case(device, D, H, lengths, ctx, D, mla, grad=True)
+    scale = D ** -0.5
+    out = flash_attn_mlm_compressed(q, k, v, H, meta, scale, cache, 0, is_mla=mla, block_n=64)
+    (sched,) = meta.kernel_schedules.values()
+    assert int(sched[:8].view(torch.int32)[1]) > 0, "the shape is meant to split"
+    kw = dict(is_mla=mla, k_cache=_np(kc), v_cache=None if mla else _np(vc), cu_seqlens_kv=cu,
+              total_context_len=cu[-1], context_batch_size=len(ctx))
+    ref = ar.mlm_attention_packed(_np(q), _np(k), _np(k if mla else v), lengths, scale, **kw)
+    np.testing.assert_allclose(_np(unpack_from_kernel(out.detach(), meta, H)), ref, atol=TOL, rtol=TOL)
+    dout = torch.randn(out.shape, generator=torch.Generator().manual_seed(1)).to(device)
+    leaves = [q, k, kc] if mla else [q, k, v, kc, vc]
+    got = torch.autograd.grad(out, leaves, dout)
+    want = ar.mlm_attention_packed_backward(_np(q), _np(k), _np(k if mla else v),
+                                            _np(unpack_from_kernel(dout, meta, H)), lengths, scale, **kw)
+    want = [want[0], want[1], want[3]] if mla else want
+    for name, g, r in zip(["q", "k", "kc"] if mla else ["q", "k", "v", "kc", "vc"], got, want):
+        worst = np.abs(_np(g) - r).max() / np.abs(r).max()
+        assert worst <= 2e-5, (name, worst)
+
+
 @pytest.mark.parametrize("D", [16, 64, 256])
 def test_f32_infinity_in_a_last_value_row(D, device):
     """A value that is infinite in the last row of a key range reaches that column of every

@@ -3,7 +3,7 @@ real query row's log2-sum-exp, which the forward stores when a backward will fol
 which fmlm_attn_bwd then reads instead of recomputing).  Every forward kernel is covered:
 the pipelined MFMA kernel (dense and packed, unsplit and split key ranges, where
 merge_kernel writes the statistic), the 512-wide MLA kernel (head-packed tiles and dense
-rows), the fp32 SIMT kernel, and the paged-context instantiations (bit-equal to the same
+rows), the fp32 kernel, and the paged-context instantiations (bit-equal to the same
 context stored contiguously).  Reference: the float64 oracle's row_lse2
 (oracle/attention_ref.py), pinned by closed forms in test_oracle_attention.py.
 
@@ -24,7 +24,8 @@ import numpy as np
 import pytest
 import torch
 
-from flash_mlm import InferenceCache, _lib, build_pack_metadata, flash_attn_mlm, flash_attn_mlm_compressed
+from flash_mlm import InferenceCache, _lib, build_pack_metadata, flash_attn_mlm, flash_attn_mlm_compressed, \
+    unpack_from_kernel
 from flash_mlm.host import host as hh
 from oracle import attention_ref as ar
 
@@ -100,7 +101,7 @@ def test_row_stats_packed(dtype, D, mla, causal, ctx, device):
 @pytest.mark.parametrize("dtype,D,mla", [
     (torch.bfloat16, 64, False),   # pipelined kernel, dense rows
     (torch.bfloat16, 512, True),   # MLA kernel, dense rows
-    (torch.float32, 64, False),    # SIMT kernel
+    (torch.float32, 64, False),    # fp32 kernel
 ])
 def test_row_stats_dense(dtype, D, mla, device):
     gen = torch.Generator().manual_seed(7800 + D + mla)
@@ -208,3 +209,58 @@ def test_row_stats_paged_context_equal_contiguous(mla, D, device):
     got = _gpu_rows(plan, lengths, np.concatenate([[0], np.cumsum(lengths)]))
     for b, L in enumerate(lengths):
         _check(got[b], ref[b, :, :L], f"b={b}")
+
+
+@pytest.mark.parametrize("dtype,D,mla", [
+    (torch.bfloat16, 64, False), (torch.float16, 256, False), (torch.bfloat16, 512, True), (torch.float32, 64, False),
+])
+def test_row_stats_dense_split(dtype, D, mla, device):
+    """A dense call whose key ranges are split: merge_kernel writes the statistics."""
+    gen = torch.Generator().manual_seed(7900 + D + mla)
+    B, H, N, C = 2, 2, 37, 3000
+    scale = 1.0 / math.sqrt(D)
+    q, k, v = (_leaf((B, H, N, D), dtype, device, gen) for _ in range(3))
+    kc = _leaf((B * (1 if mla else H) * C, D), dtype, device, gen)
+    vc = None if mla else _leaf(kc.shape, dtype, device, gen)
+    cache = InferenceCache()
+    cache.prefill_kv_cache(0, k_cache=kc, v_cache=vc, context_batch_size=B, is_mla=mla, num_heads=H, head_dim=D)
+    plan = flash_attn_mlm(q, k, v, scale, cache, 0, is_mla=mla).grad_fn.plan
+    assert plan.records > 0, "the shape is meant to split"
+    ref = ar.mlm_row_lse2_dense(_np(q), _np(k), scale, is_mla=mla, k_cache=_np(kc), context_len=C,
+                                context_batch_size=B)
+    got = _gpu_rows(plan, [N] * B, [b * N for b in range(B)])
+    for b in range(B):
+        _check(got[b], ref[b], f"b={b}")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,lengths,ctx", [
+    (16, [3, 0, 2], [2500, 700, 1100]),  # tiles of 64 rows
+    (64, [33, 34], [1500, 900]),         # tiles of 128 rows
+])
+def test_row_stats_latent_split(H, lengths, ctx, dtype, device):
+    """A latent call whose key ranges are split: the statistics of the merged (head,
+    position) rows, and the gradients that the backward makes of them (2e-2 of the largest
+    entry, as for every 16-bit gradient)."""
+    gen = torch.Generator().manual_seed(8000 + H)
+    B, N, D = len(lengths), max(lengths), 512
+    scale = 1.0 / math.sqrt(D)
+    q, k = (_leaf((B, H, N, D), dtype, device, gen) for _ in range(2))
+    cache, kc, cu_kv, total = _packed_cache(ctx, H=H, D=D, mla=True, dtype=dtype, device=device, gen=gen)
+    meta = build_pack_metadata(torch.tensor(lengths, device=device, dtype=torch.int32), N, block_n=64)
+    out = flash_attn_mlm_compressed(q, k, k, H, meta, scale, cache, 0, is_mla=True, block_n=64)
+    (sched,) = meta.kernel_schedules.values()
+    assert int(sched[:8].view(torch.int32)[1]) > 0, "the shape is meant to split"
+    kw = dict(is_mla=True, k_cache=_np(kc), cu_seqlens_kv=cu_kv, total_context_len=total, context_batch_size=B)
+    ref = ar.mlm_row_lse2_packed(_np(q), _np(k), lengths, scale, **kw)
+    got = _gpu_rows(out.grad_fn.plan, lengths, np.concatenate([[0], np.cumsum(lengths)]))
+    for b, L in enumerate(lengths):
+        if L:
+            _check(got[b], ref[b, :, :L], f"b={b}")
+    dout = torch.randn(out.shape, generator=gen).to(dtype).to(device)
+    grads = torch.autograd.grad(out, [q, k, kc], dout)
+    want = ar.mlm_attention_packed_backward(_np(q), _np(k), _np(k), _np(unpack_from_kernel(dout, meta, H)), lengths,
+                                            scale, v_cache=None, **kw)
+    for name, g, r in zip(("q", "k", "kc"), grads, (want[0], want[1], want[3])):
+        worst = np.abs(_np(g) - r).max() / np.abs(r).max()
+        assert worst <= 2e-2, (name, worst)

@@ -9,6 +9,7 @@ output type of each other (2^-8 relative at bf16, 2^-11 at fp16), plus 1e-5 for 
 from __future__ import annotations
 
 import ctypes
+import random
 
 import numpy as np
 import pytest
@@ -69,6 +70,83 @@ def test_dense_split_matches_oracle_and_unsplit(B, H, N, D, C, cbs, dtype, devic
     torch.testing.assert_close(out.float(), whole.float(), atol=ulp * float(whole.float().abs().max()), rtol=ulp)
 
 
+def _split_groups(meta):
+    """Split groups of the one schedule of a metadata (header word 1)."""
+    (sched,) = meta.kernel_schedules.values()
+    return int(sched[:8].view(torch.int32)[1])
+
+
+@pytest.mark.parametrize("B,H,N,C,cbs", [(1, 4, 20, 3000, 1), (2, 3, 130, 2050, 2), (1, 1, 1, 1500, 1)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_dense_latent_split_matches_oracle_and_unsplit(dtype, B, H, N, C, cbs, device):
+    """The 512-wide latent in a dense call (per-head main keys, one latent context): tiles of
+    128 rows of one head, cut and merged."""
+    gen = torch.Generator().manual_seed(N)
+    D = 512
+    q, k = (_randn(gen, (B, H, N, D), dtype, device, 0.5) for _ in range(2))
+    kc = _randn(gen, (cbs * C, D), dtype, device, 0.5)
+    cache = InferenceCache()
+    cache.prefill_kv_cache(0, k_cache=kc, context_batch_size=cbs, is_mla=True, num_heads=H, head_dim=D)
+    scale = D ** -0.5
+    out, plan = hh._dense_impl(q, k, k, scale, cache, 0, True, None, False, run=False)
+    assert plan.records > 0, "the shape is meant to split"
+    plan()
+    ref = ar.mlm_attention_dense(_np(q), _np(k), _np(k), scale, is_mla=True, k_cache=_np(kc), context_len=C,
+                                 context_batch_size=cbs)
+    np.testing.assert_allclose(_np(out), ref, atol=1e-2, rtol=1e-2)
+    p = _lib.AttnParams.from_buffer_copy(plan.params)
+    whole = torch.full_like(out, float("nan"))
+    p.o, p.workspace, p.workspace_bytes = whole.data_ptr(), None, 0
+    _lib.check(plan.lib.fmlm_attn_fwd(ctypes.byref(p), plan.stream), "fmlm_attn_fwd")
+    # P is rounded to 16 bits against each part's own maximum: two roundings of weights and
+    # one of the output apart
+    ulp = {torch.bfloat16: 2.0**-8, torch.float16: 2.0**-11}[dtype]
+    torch.testing.assert_close(out.float(), whole.float(), atol=2 * ulp * float(whole.float().abs().max()), rtol=ulp)
+
+
+@pytest.mark.parametrize("H,lengths,ctx", [
+    # one tile of 64 rows, by work all 16 parts on one XCD
+    (16, [3], [4097]),
+    # by work the fullest XCD has 33 (38) parts, its 32 CUs take one each
+    (64, [8] * 16, random.Random(0).choices(range(2000, 6001), k=16)),
+    (64, [8] * 16, sorted(random.Random(2).choices(range(2000, 6001), k=16))),
+])
+def test_latent_parts_are_dealt_by_count(H, lengths, ctx, device):
+    """Where parts placed by work would crowd an XCD, the queues get equal counts instead;
+    every (tile, part) is one unit, and every part has a record of its own."""
+    gen = torch.Generator().manual_seed(H)
+    dtype, D, N, B = torch.bfloat16, 512, max(lengths), len(lengths)
+    q, k = (_randn(gen, (B, H, N, D), dtype, device, 0.5) for _ in range(2))
+    cu = [0, *np.cumsum(ctx).tolist()]
+    kc = _randn(gen, (cu[-1], D), dtype, device, 0.5)
+    cache = InferenceCache()
+    cache.prefill_kv_cache(0, k_cache=kc, total_context_len=cu[-1], context_batch_size=B, is_mla=True, num_heads=H,
+                           cu_seqlens_kv=torch.tensor(cu, dtype=torch.int32, device=device), head_dim=D)
+    meta = build_pack_metadata(torch.tensor(lengths, dtype=torch.int32, device=device), N, 64)
+    out = flash_attn_mlm_compressed(q, k, k, H, meta, D ** -0.5, cache, 0, is_mla=True, block_n=64)
+    (sched,) = meta.kernel_schedules.values()
+    words = sched.cpu().numpy().view(np.int32)
+    cap, queues = int(words[5]), words[8:16]
+    assert _split_groups(meta) > 0
+    assert queues.max() - queues.min() <= 1 and queues.sum() == words[0]
+    units = words[64:64 + 8 * cap * 4].reshape(8, cap, 4)
+    seen, records = set(), set()
+    for x in range(8):
+        for b, ht, rec0, w in units[x, :queues[x]]:
+            part, parts = ((int(w) >> 20) & 31, ((int(w) >> 25) & 31) + 1) if w >= 0 else (0, 1)
+            seen.add((int(b), int(ht) >> 16, part))
+            if parts > 1:
+                records.add(int(rec0) + part)
+    bq = 64 if H * sum(lengths) <= 4096 else 128
+    tiles = sum(-(-H * n // bq) for n in lengths)
+    assert len(seen) == words[0] and len({t[:2] for t in seen}) == tiles
+    assert len(records) == sum(1 for _ in seen) and max(records) < words[0]
+    ref = ar.mlm_attention_packed(_np(q), _np(k), _np(k), lengths, D ** -0.5, is_mla=True, k_cache=_np(kc),
+                                  cu_seqlens_kv=cu, total_context_len=cu[-1], context_batch_size=B)
+    np.testing.assert_allclose(_np(unpack_from_kernel(out, meta, H)), ref, atol=1e-2, rtol=1e-2)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("paged", [False, True])
 @pytest.mark.parametrize("H,lengths,ctx", [
     (64, [1, 0, 4, 2], [2000, 900, 0, 5]),       # tiles of 64, 128 and 256 rows, short and empty contexts
@@ -76,9 +154,9 @@ def test_dense_split_matches_oracle_and_unsplit(B, H, N, D, C, cbs, dtype, devic
     (5, [7, 1, 30], [333, 1024, 64 * 9]),        # odd heads: rows of a tile span heads
     (32, [4, 3] * 40, [640, 517] * 40),          # many groups: the merge takes larger chunks
 ])
-def test_latent_split_matches_oracle(H, lengths, ctx, paged, device):
+def test_latent_split_matches_oracle(H, lengths, ctx, paged, dtype, device):
     gen = torch.Generator().manual_seed(H)
-    dtype, D, N, B = torch.bfloat16, 512, max(lengths), len(lengths)
+    D, N, B = 512, max(lengths), len(lengths)
     q, k = (_randn(gen, (B, H, N, D), dtype, device, 0.5) for _ in range(2))
     cu = [0, *np.cumsum(ctx).tolist()]
     kc = _randn(gen, (cu[-1], D), dtype, device, 0.5)
@@ -101,6 +179,7 @@ def test_latent_split_matches_oracle(H, lengths, ctx, paged, device):
     meta = build_pack_metadata(torch.tensor(lengths, dtype=torch.int32, device=device), N, 64)
     scale = D ** -0.5
     out = flash_attn_mlm_compressed(q, k, k, H, meta, scale, cache, 0, is_mla=True, block_n=64)
+    assert _split_groups(meta) > 0, "the shape is meant to split"
     ref = ar.mlm_attention_packed(_np(q), _np(k), _np(k), lengths, scale, is_mla=True, k_cache=_np(kc),
                                   cu_seqlens_kv=cu, total_context_len=cu[-1], context_batch_size=B)
     np.testing.assert_allclose(_np(unpack_from_kernel(out, meta, H)), ref, atol=1e-2, rtol=1e-2)
