@@ -2387,6 +2387,8 @@ static BwdFns bwd_f32_fns() {
                 C::KEYS};
 }
 
+// (a paged context's table is set in two fp32 calls: through this entry alone, since the
+// forward refuses them, and with FMLM_FLAG_PREFILL over a layer that has one)
 static bool pick_bwd_f32(const fmlm_attn_params& p, BwdFns& f) {
   if (p.ctx_block_table) return false;
   switch (p.D) {

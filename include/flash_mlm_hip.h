@@ -251,7 +251,8 @@ typedef struct fmlm_attn_params {
    * workgroup, waves per workgroup): D = 16, 32: 1 = (128, 4); D = 64: 1 = (128, 4),
    * 2 = (256, 8), 3 = (64, 4), 4 = (256, 8) ping-pong; D = 128: 1 = (128, 4),
    * 2 = (256, 8), 3 = (64, 4), 4 = (128, 8), 5 = (256, 8) ping-pong; D = 256:
-   * 1 = (64, 4), 2 = (128, 8); MLA D = 512: 1 = (128, 8).  Ping-pong: the 8 waves run as
+   * 1 = (64, 4), 2 = (128, 8); MLA D = 512: 1 = (128, 8), in packed calls of at most 4096
+   * (head, position) rows (64, 8).  Ping-pong: the 8 waves run as
    * two groups half a key tile apart, so that one wave of each SIMD computes softmax
    * while the other issues MFMAs.  Replaces the reference's autotuned
    * BLOCK_M / BLOCK_N / num_warps (mlm_kernel.py:57-166).  Ignored by f32 inputs.       */
@@ -319,8 +320,10 @@ FMLM_API int fmlm_attn_fwd_noalloc(const fmlm_attn_params* p, void* stream);
  *           pool, zeroed by the caller, that the kernel adds into atomically: a page used
  *           by several context batches receives the sum of their gradients.
  * Rows not listed are not written.  dout is laid out like o (o_layout).
- * bf16 / f16 (MFMA) and f32 (SIMT), D in {16, 32, 64, 128, 256, 512}; with
- * FMLM_FLAG_CAUSAL_SEQ the main keys must be packed (kv_layout PACKED).
+ * bf16 / f16 / f32, D in {16, 32, 64, 128, 256, 512}: MFMA kernels, except 16-bit D = 16,
+ * D = 512 (16-bit without MLA, f32) and f32 with a paged context (which fmlm_attn_fwd does
+ * not run), which take SIMT kernels; with FMLM_FLAG_CAUSAL_SEQ the main keys must be packed
+ * (kv_layout PACKED).
  * workspace: fmlm_attn_bwd_workspace_bytes(p) bytes (per-row softmax statistics, the
  *           tile tables of the two kernels and a 64-byte record per tile).
  * ------------------------------------------------------------------------- */

@@ -82,7 +82,7 @@ def test_argument_rejection_without_launch():
     p.D = 64
     p.dtype = 7
     assert lib.fmlm_attn_bwd(p, g, None) == -2
-    p.dtype = _lib.DTYPE_F32  # SIMT kernels: accepted, then the missing workspace is reported
+    p.dtype = _lib.DTYPE_F32  # accepted, then the missing workspace is reported
     assert lib.fmlm_attn_bwd(p, g, None) == -5
     p.dtype = _lib.DTYPE_BF16
     assert lib.fmlm_attn_bwd(p, g, None) == -5  # no workspace

@@ -272,8 +272,9 @@ def test_backward_against_torch_fp32_autograd(device):
                              (torch.bfloat16, 16), (torch.float16, 16)] for m in ("ctx", "causal_mla_ctx")
 ] + [(torch.float32, 512, "causal_mla_ctx")])
 def test_backward_simt_kernels(dtype, D, mode, device):
-    """fp32 inputs and head dim 16 take the SIMT backward kernels; fp32 gradients are held
-    to 1e-4 of the largest reference entry, bf16/fp16 to the tolerance above."""
+    """16-bit head dim 16 and fp32 head dim 512 take the SIMT backward kernels, the other
+    fp32 cases the fp32 MFMA kernels; fp32 gradients are held to 1e-4 of the largest
+    reference entry, bf16/fp16 to the tolerance above."""
     gen = torch.Generator().manual_seed(8300 + D + (mode == "ctx"))
     mla, causal = "mla" in mode, "causal" in mode
     lengths = [70, 1, 0, 45]
@@ -305,7 +306,7 @@ def test_backward_simt_kernels(dtype, D, mode, device):
 
 def test_backward_dense_fp32_config1_shape(device):
     """The dense fp32 workload of the reference's CPU-runnable configuration, through the
-    SIMT backward."""
+    fp32 backward."""
     gen = torch.Generator().manual_seed(8400)
     B, H, N, D = 2, 8, 128, 64
     scale = 1.0 / math.sqrt(D)
