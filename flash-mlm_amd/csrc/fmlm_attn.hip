@@ -56,8 +56,9 @@ namespace fmlm {
 // kSplitRounds rounds, the key ranges of query tiles are cut into S parts each (a split
 // group).  Packed calls cut long ranges into parts of one length (seq_chunk; head-packed
 // calls by price, hpack_price; both in fmlm_split_plan.h), dense calls all tiles into equal
-// numbers of parts by arithmetic (split_cfg, no schedule).  Every part is a unit that writes a partial record (O / l as fp32, then m and l per
-// row) and a second kernel, merge_kernel, combines each group's records into the output.
+// numbers of parts by arithmetic (split_cfg, no schedule).  Every part is a unit that
+// writes a partial record (O / l as fp32, then m and l per row) and a second kernel,
+// merge_kernel, combines each group's records into the output.
 // (Merging inside the attention kernel would need device-scope release/acquire between
 // workgroups, which writes back and invalidates an XCD's whole L2 each time.)
 //

@@ -287,8 +287,8 @@ struct F32Tile {
 #pragma unroll
     for (int i = 0; i < NL; ++i) dma16_sbase(src, off[i], __builtin_amdgcn_readfirstlane(lds + i * 1024));
   }
-  // rows [n, 16) of a loaded tile to zero, n < 16: they repeat row n - 1, and where that row is not
-  // finite its product with their weight 0 would not be 0
+  // rows [n, 16) of a loaded tile to zero, n < 16: they repeat row n - 1, and where that row
+  // is not finite its product with their weight 0 would not be 0
   static FMLM_DEV void zero_from(int n, uint32_t lds, int lane) {
     for (int at = n * PITCH; at < BYTES; at += 1024)
       if (at + 16 * lane < BYTES) *(FMLM_LDS f32x4*)(uintptr_t)(lds + at + 16 * lane) = f32x4{0.f, 0.f, 0.f, 0.f};
